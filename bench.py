@@ -28,7 +28,7 @@ sys.path.insert(0, ROOT)
 METRIC = "chi(q,w) s per q-point: mixed/batched vs plain FP64 GPU at <=1e-5 rel err"
 ERR_BAR = 1e-5  # chi and eps^-1 relative Frobenius error of the mixed path against FP64
 PEAK = {"fp64": 78.6e12, "fp32": 157.3e12, "bf16x3": 2.5e15}  # dense MFMA, MI355X
-KERNEL = {"fp64": "k_chi_gemm<0>", "fp32": "k_chi_gemm<1>", "bf16x3": "k_chi_bf16x3"}
+KERNEL = {"fp64": "k_chi_f64", "fp32": "k_chi_gemm", "bf16x3": "k_chi_bf16x3"}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic.txt")
 
 

@@ -602,10 +602,7 @@ ChiLaunch chi_launch_heuristic(const rp_ctx* h, int prec) {
     c.nwg = bf16x3_workgroups(h->ncu);
     c.nsplit = bf16x3_nsplit(h->ng, h->nen, h->kpad, c.nwg);
   } else {
-    const int ntile = (h->ng + chi_tile() - 1) / chi_tile();
-    const size_t kchunks = h->kpad / chi_kchunk();
-    const long wgs = (long)ntile * ntile * h->nen;
-    c.nsplit = (int)std::min<long>((long)kchunks, std::max<long>(1, (2048 + wgs - 1) / wgs));
+    c.nsplit = chi_gemm_nsplit(prec, h->ng, h->nen, h->kpad, h->ncu);
   }
   return c;
 }
@@ -673,8 +670,8 @@ void issue_dyson(rp_ctx* h) {
 // ---------------------------------------------------------------- autotune
 // Candidates around the heuristic: for the split-BF16 kernel the K splits
 // whose work rounds per XCD slot (the heuristic's model) are within 15% of the
-// best, plus half and double the heuristic's; for the FP64/FP32 kernel the
-// splits that give 1024, 2048 and 4096 workgroups.  Each is timed on the
+// best, plus half and double the heuristic's; for the FP64/FP32 kernels half
+// and double the heuristic's split.  Each is timed on the
 // current q's data (one warm-up, then the best of two), and the fastest is
 // kept for every later q of the same shape.
 static std::vector<ChiLaunch> chi_candidates(const rp_ctx* h, int prec) {
@@ -700,11 +697,8 @@ static std::vector<ChiLaunch> chi_candidates(const rp_ctx* h, int prec) {
     if (base.nsplit > 1) add({base.nsplit / 2, base.nwg});
     if ((size_t)base.nsplit * 2 <= nchunks && base.nsplit * 2 <= 64) add({base.nsplit * 2, base.nwg});
   } else {
-    const int ntile = (h->ng + chi_tile() - 1) / chi_tile();
-    const size_t kchunks = h->kpad / chi_kchunk();
-    const long wgs = (long)ntile * ntile * h->nen;
-    for (long target : {1024L, 2048L, 4096L})
-      add({(int)std::min<long>((long)kchunks, std::max<long>(1, (target + wgs - 1) / wgs)), 0});
+    const int kchunks = (int)(h->kpad / chi_kchunk());
+    for (int sp : {base.nsplit / 2, base.nsplit * 2}) add({std::min(kchunks, std::max(1, sp)), 0});
   }
   return out;
 }

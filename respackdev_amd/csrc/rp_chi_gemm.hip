@@ -8,17 +8,17 @@
 // for the real part and (Im b | -Re b) for the imaginary part.
 //
 // Workgroup: 256 threads (2x2 waves), tile 64 G x 64 G' for one frequency;
-// each wave owns 2x2 MFMA blocks of 16x16.  A K-chunk of 32 complex rows of
-// both panels is staged in LDS (transposed to [G][K]) together with the 32
-// weights; the weights are applied to the right panel as it is read (scale on
-// load).  Precisions:
-//   FP64   v_mfma_f64_16x16x4f64, FP64 accumulators.
-//   FP32   v_mfma_f32_16x16x4f32; FP32 accumulators flushed into FP64 ones
-//          every kFlush chunks.
+// each wave owns 2x2 MFMA blocks of 16x16.  Precisions:
+//   FP64   k_chi_f64: v_mfma_f64_16x16x4f64, FP64 accumulators, the complex
+//          product as three real ones.
+//   FP32   k_chi_gemm: v_mfma_f32_16x16x4f32; FP32 accumulators flushed into
+//          FP64 ones every kFlush chunks.
 // (The split-BF16 precision has its own kernel, k_chi_bf16x3.)
 // The K range may be split over gridDim.z; partial tiles are summed in fixed
 // order by k_chi_reduce (deterministic), which also divides by the volume.
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 #include "rp_common.h"
 #include "rp_kernels.h"
@@ -48,9 +48,10 @@ __device__ inline void stage_chunk(const float2* __restrict__ A, size_t lda, siz
   if (t < kKC) sD[t] = dw[K0 + t];
 }
 
-// One output tile, precision selected by P.  out: partial[z][w][ng][ng] with
+// One output tile in FP32: a K-chunk of 32 complex rows of both panels is
+// staged in LDS (transposed to [G][K]) together with the 32 weights, which are
+// applied to the right panel as it is read.  out: partial[z][w][ng][ng] with
 // element (G, G') at out[... + G' * ng + G] (Fortran chiqw(ig,jg,ie) order).
-template <int P>
 __global__ void __launch_bounds__(256) k_chi_gemm(const float2* __restrict__ A, size_t lda,
                                                   const double2* __restrict__ dw, size_t ldd,
                                                   size_t kchunks_per_split, size_t kchunks,
@@ -85,106 +86,221 @@ __global__ void __launch_bounds__(256) k_chi_gemm(const float2* __restrict__ A, 
     for (int b = 0; b < 2; ++b)
       for (int v = 0; v < 4; ++v) accd_re[a][b][v] = accd_im[a][b][v] = 0.0;
 
-  if constexpr (P == RP_PREC_FP64) {
-    d4v acc_re[2][2], acc_im[2][2];
-    for (int a = 0; a < 2; ++a)
-      for (int b = 0; b < 2; ++b) acc_re[a][b] = acc_im[a][b] = d4v{0, 0, 0, 0};
-    const int h = q & 1;
-    for (size_t c = c_begin; c < c_end; ++c) {
-      stage_chunk(A, lda, c * kKC, g0, h0, dww, sL, sR, sD);
-      __syncthreads();
+  f4v acc_re[2][2], acc_im[2][2];
+  for (int a = 0; a < 2; ++a)
+    for (int b = 0; b < 2; ++b) acc_re[a][b] = acc_im[a][b] = f4v{0, 0, 0, 0};
+  const int h = q & 1;
+  int since = 0;
+  for (size_t c = c_begin; c < c_end; ++c) {
+    stage_chunk(A, lda, c * kKC, g0, h0, dww, sL, sR, sD);
+    __syncthreads();
 #pragma unroll 4
-      for (int s = 0; s < 16; ++s) {
-        const int kl = h * 16 + s;
-        double L[2], Rre[2], Rim[2];
-        const double2 dd = sD[kl];
+    for (int s = 0; s < 16; ++s) {
+      const int kl = h * 16 + s;
+      float L[2], Rre[2], Rim[2];
+      const float dx = (float)sD[kl].x, dy = (float)sD[kl].y;
+      for (int b = 0; b < 2; ++b) {
+        float2 la = sL[wm * 32 + b * 16 + li][kl];
+        L[b] = part ? la.y : la.x;
+        float2 ra = sR[wn * 32 + b * 16 + li][kl];
+        float bx = dx * ra.x - dy * ra.y;
+        float by = dx * ra.y + dy * ra.x;
+        Rre[b] = part ? by : bx;
+        Rim[b] = part ? -bx : by;
+      }
+      for (int a = 0; a < 2; ++a) {
+        if (!rowok[a]) continue;
         for (int b = 0; b < 2; ++b) {
-          float2 la = sL[wm * 32 + b * 16 + li][kl];
-          L[b] = part ? (double)la.y : (double)la.x;
-          float2 ra = sR[wn * 32 + b * 16 + li][kl];
-          double bx = dd.x * (double)ra.x - dd.y * (double)ra.y;
-          double by = dd.x * (double)ra.y + dd.y * (double)ra.x;
-          Rre[b] = part ? by : bx;
-          Rim[b] = part ? -bx : by;
-        }
-        for (int a = 0; a < 2; ++a) {
-          if (!rowok[a]) continue;
-          for (int b = 0; b < 2; ++b) {
-            if (!colok[b]) continue;
-            acc_re[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(L[a], Rre[b], acc_re[a][b], 0, 0, 0);
-            acc_im[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(L[a], Rim[b], acc_im[a][b], 0, 0, 0);
-          }
+          if (!colok[b]) continue;
+          acc_re[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(L[a], Rre[b], acc_re[a][b], 0, 0, 0);
+          acc_im[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(L[a], Rim[b], acc_im[a][b], 0, 0, 0);
         }
       }
-      __syncthreads();
     }
-    for (int a = 0; a < 2; ++a)
-      for (int b = 0; b < 2; ++b)
-        for (int v = 0; v < 4; ++v) {
-          accd_re[a][b][v] = acc_re[a][b][v];
-          accd_im[a][b][v] = acc_im[a][b][v];
-        }
-  } else {
-    static_assert(P == RP_PREC_FP32, "k_chi_gemm: FP64 or FP32");
-    f4v acc_re[2][2], acc_im[2][2];
-    for (int a = 0; a < 2; ++a)
-      for (int b = 0; b < 2; ++b) acc_re[a][b] = acc_im[a][b] = f4v{0, 0, 0, 0};
-    const int h = q & 1;
-    int since = 0;
-    for (size_t c = c_begin; c < c_end; ++c) {
-      stage_chunk(A, lda, c * kKC, g0, h0, dww, sL, sR, sD);
-      __syncthreads();
-#pragma unroll 4
-      for (int s = 0; s < 16; ++s) {
-        const int kl = h * 16 + s;
-        float L[2], Rre[2], Rim[2];
-        const float dx = (float)sD[kl].x, dy = (float)sD[kl].y;
+    __syncthreads();
+    if (++since == kFlush || c + 1 == c_end) {
+      since = 0;
+      for (int a = 0; a < 2; ++a)
         for (int b = 0; b < 2; ++b) {
-          float2 la = sL[wm * 32 + b * 16 + li][kl];
-          L[b] = part ? la.y : la.x;
-          float2 ra = sR[wn * 32 + b * 16 + li][kl];
-          float bx = dx * ra.x - dy * ra.y;
-          float by = dx * ra.y + dy * ra.x;
-          Rre[b] = part ? by : bx;
-          Rim[b] = part ? -bx : by;
-        }
-        for (int a = 0; a < 2; ++a) {
-          if (!rowok[a]) continue;
-          for (int b = 0; b < 2; ++b) {
-            if (!colok[b]) continue;
-            acc_re[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(L[a], Rre[b], acc_re[a][b], 0, 0, 0);
-            acc_im[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(L[a], Rim[b], acc_im[a][b], 0, 0, 0);
+          for (int v = 0; v < 4; ++v) {
+            accd_re[a][b][v] += (double)acc_re[a][b][v];
+            accd_im[a][b][v] += (double)acc_im[a][b][v];
           }
+          acc_re[a][b] = acc_im[a][b] = f4v{0, 0, 0, 0};
         }
-      }
-      __syncthreads();
-      if (++since == kFlush || c + 1 == c_end) {
-        since = 0;
-        for (int a = 0; a < 2; ++a)
-          for (int b = 0; b < 2; ++b) {
-            for (int v = 0; v < 4; ++v) {
-              accd_re[a][b][v] += (double)acc_re[a][b][v];
-              accd_im[a][b][v] += (double)acc_im[a][b][v];
-            }
-            acc_re[a][b] = acc_im[a][b] = f4v{0, 0, 0, 0};
-          }
-      }
     }
   }
 
-  // epilogue.  Result layout of a 16x16 block (checked on gfx950): the FP32
-  // and BF16 MFMAs leave C[4*(lane>>4)+v][lane&15] in element v of a lane, the
-  // FP64 MFMA leaves C[(lane>>4)+4*v][lane&15].
+  // epilogue: the FP32 MFMA leaves C[4*(lane>>4)+v][lane&15] of a 16x16 block
+  // in element v of a lane (checked on gfx950)
   double2* o = out + ((size_t)z * nen + w) * (size_t)ng * ng;
   for (int a = 0; a < 2; ++a)
     for (int b = 0; b < 2; ++b)
       for (int v = 0; v < 4; ++v) {
-        const int row = P == RP_PREC_FP64 ? q + 4 * v : 4 * q + v;
-        const int gi = g0 + wm * 32 + a * 16 + row;
+        const int gi = g0 + wm * 32 + a * 16 + 4 * q + v;
         const int hj = h0 + wn * 32 + b * 16 + li;
         if (gi < ng && hj < ng)
           o[(size_t)hj * ng + gi] = make_double2(accd_re[a][b][v], accd_im[a][b][v]);
       }
+}
+
+// One output tile in FP64.  With b = d a(G') the complex product conj(a) b is
+// three real ones (three real MFMAs per block and 4 K where the direct form
+// needs four):
+//   T1 = ar br,  T2 = ai bi,  T3 = (ar - ai)(br + bi),
+//   Re = T1 + T2,  Im = T3 - T1 + T2.
+// FP64 MFMAs and FP64 vector instructions share one unit per SIMD (run
+// together they reach 58 TFLOP/s, the MFMAs alone 79), so every vector
+// operation on the operands costs matrix time: the three left and three right
+// planes of a chunk are formed once per workgroup as it is staged (10 vector
+// operations per staged element pair against 192 MFMA flops per element of the
+// 64-wide tile) and the loop over the chunk is LDS reads and MFMAs only.
+// Planes are [k][64 + 16]: the four k of a read fall on both halves of the
+// banks.  The loads of the next chunk are in flight during the MFMAs.
+//
+// Bound by that unit.  NG 441, K 112500, 32 frequencies (5.6 TFLOP): 64.8 ms,
+// 67 TFLOP/s executed (the direct form with the weights applied on every read:
+// 108.5 ms).  Four workgroups per CU hide the staging, hence 8 K per chunk and
+// 128 registers: three (more registers, 8 K) 68.3 ms, two (16 K) 71 ms, two with
+// 128 x 64 tiles and fewer vector operations 75.6 ms, two double-buffered 78 ms.
+// Error against long double, relative norm: 7.8e-16 (direct form 6.6e-15; the
+// imaginary part alone, 50 times smaller than the real part here, 3e-14 against
+// 9e-15 of its own norm).
+//
+// The right block is the MFMA's first operand, so that D(row, col) =
+// (G', G) and the lanes of a result run along G, the fastest index of out.
+// The 16-blocks of [0, ng) are dealt evenly to the ntile tiles of an axis (four
+// at most: 10 blocks are 3 + 3 + 4, not 4 + 4 + 2), and a tile's blocks to its
+// waves so that the busiest has the fewest (4x4: 2x2 each; 3x3: three columns
+// of three).  Which wave takes which part rotates with the workgroup so that
+// the idler parts spread over the SIMDs.
+constexpr int kF64KC = 8;                // K rows per chunk
+constexpr int kF64Row = kTile + 16;      // doubles per plane row
+constexpr int kF64Plane = kF64KC * kF64Row;
+
+template <int NR, int NC>
+__device__ __forceinline__ void f64_chunk(const double* pl, const double* pr, int li, int lk,
+                                          d4v (&acc)[3][4]) {
+#pragma unroll
+  for (int k0 = 0; k0 < kF64KC; k0 += 4)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      double l[NR], r[NC];
+#pragma unroll
+      for (int b = 0; b < NC; ++b) r[b] = pr[p * kF64Plane + (k0 + lk) * kF64Row + li + 16 * b];
+#pragma unroll
+      for (int a = 0; a < NR; ++a) l[a] = pl[p * kF64Plane + (k0 + lk) * kF64Row + li + 16 * a];
+#pragma unroll
+      for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b)
+          acc[p][a * NC + b] =
+              __builtin_amdgcn_mfma_f64_16x16x4f64(r[b], l[a], acc[p][a * NC + b], 0, 0, 0);
+    }
+}
+
+__global__ void __launch_bounds__(256, 4) k_chi_f64(const float2* __restrict__ A, size_t lda,
+                                                    const double2* __restrict__ dw, size_t ldd,
+                                                    size_t chunks_per_split, size_t nchunks,
+                                                    int ng, int ntile, int nen,
+                                                    double2* __restrict__ out) {
+  __shared__ double sl[3 * kF64Plane], sr[3 * kF64Plane];
+  const int tm = (int)blockIdx.x % ntile, tn = (int)blockIdx.x / ntile;
+  const int nb = (ng + 15) / 16;
+  const int gb = tm * nb / ntile, hb = tn * nb / ntile;  // first block of the tile
+  const int g0 = 16 * gb, h0 = 16 * hb;
+  const int w = blockIdx.y, z = blockIdx.z;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int part = (wave + (int)(blockIdx.x + blockIdx.y + blockIdx.z)) & 3;
+  const int li = lane & 15, lk = lane >> 4;
+  const double2* dww = dw + (size_t)w * ldd;
+  const size_t c0 = (size_t)z * chunks_per_split;
+  const size_t c1 = c0 + chunks_per_split < nchunks ? c0 + chunks_per_split : nchunks;
+  const int nr = (tm + 1) * nb / ntile - gb, nc = (tn + 1) * nb / ntile - hb;  // 1..4 blocks
+
+  // thread (wave, lane) stages G = lane and G' = lane of the K rows wave and
+  // wave + 4 of a chunk; the weight of a row is uniform in the wave
+  constexpr int kE = kF64KC / 4;
+  float2 la[kE], ra[kE];
+  double2 dv[kE];
+  auto load = [&](size_t c) {
+#pragma unroll
+    for (int e = 0; e < kE; ++e) {
+      const size_t k = c * kF64KC + (size_t)(wave + 4 * e);
+      la[e] = A[k * lda + g0 + lane];
+      ra[e] = A[k * lda + h0 + lane];
+      dv[e] = dww[k];
+    }
+  };
+  auto stage = [&]() {
+#pragma unroll
+    for (int e = 0; e < kE; ++e) {
+      const int o = (wave + 4 * e) * kF64Row + lane;
+      const double ar = la[e].x, ai = la[e].y;
+      sl[o] = ar;
+      sl[kF64Plane + o] = ai;
+      sl[2 * kF64Plane + o] = ar - ai;
+      const double cr = ra[e].x, ci = ra[e].y;
+      const double br = dv[e].x * cr - dv[e].y * ci, bi = dv[e].x * ci + dv[e].y * cr;
+      sr[o] = br;
+      sr[kF64Plane + o] = bi;
+      sr[2 * kF64Plane + o] = br + bi;
+    }
+  };
+
+  d4v acc[3][4];
+#pragma unroll
+  for (int p = 0; p < 3; ++p)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[p][i] = d4v{0, 0, 0, 0};
+  double2* o = out + ((size_t)z * nen + w) * (size_t)ng * ng;
+  // the chunk loop of a wave that owns NR x NC blocks from block (rb, cb) of
+  // the tile on (none: it only stages)
+  auto tile = [&](auto rows, auto cols, int rb, int cb) {
+    constexpr int NR = decltype(rows)::value, NC = decltype(cols)::value;
+    for (size_t c = c0; c < c1; ++c) {
+      stage();
+      __syncthreads();
+      load(c + 1 < c1 ? c + 1 : c);
+      if constexpr (NR > 0) f64_chunk<NR, NC>(sl + 16 * rb, sr + 16 * cb, li, lk, acc);
+      __syncthreads();
+    }
+    // the FP64 MFMA leaves D[(lane>>4) + 4v][lane&15] in element v of a lane
+#pragma unroll
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+      for (int b = 0; b < NC; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int gi = g0 + (rb + a) * 16 + li;
+          const int hj = h0 + (cb + b) * 16 + lk + 4 * v;
+          const int i = a * NC + b;
+          const double t1 = acc[0][i][v], t2 = acc[1][i][v], t3 = acc[2][i][v];
+          if (gi < ng && hj < ng) o[(size_t)hj * ng + gi] = make_double2(t1 + t2, t3 - t1 + t2);
+        }
+  };
+  using std::integral_constant;
+  const integral_constant<int, 0> n0{};
+  const integral_constant<int, 1> n1{};
+  const integral_constant<int, 2> n2{};
+  const integral_constant<int, 3> n3{};
+  if (c0 < c1) load(c0);
+  if (nr == 4 && nc == 4) {
+    tile(n2, n2, 2 * (part & 1), 2 * (part >> 1));
+  } else if (nr == 2 && nc == 2) {
+    tile(n1, n1, part & 1, part >> 1);
+  } else if (nr <= nc) {  // a column of blocks per wave
+    if (part >= nc) tile(n0, n0, 0, 0);
+    else if (nr == 3) tile(n3, n1, 0, part);
+    else if (nr == 2) tile(n2, n1, 0, part);
+    else tile(n1, n1, 0, part);
+  } else {  // a row of blocks per wave
+    if (part >= nr) tile(n0, n0, 0, 0);
+    else if (nc == 3) tile(n1, n3, part, 0);
+    else if (nc == 2) tile(n1, n2, part, 0);
+    else tile(n1, n1, part, 0);
+  }
 }
 
 // chi[j] = sum_z partial[z][j] / volume, fixed order over z.
@@ -205,20 +321,38 @@ __global__ void k_chi_reduce(const double2* __restrict__ part, size_t n, int nsp
 int chi_tile() { return kTile; }
 int chi_kchunk() { return kKC; }
 
+// K splits.  FP32: enough for 2048 workgroups.  FP64: with W workgroups per
+// split, S = 4 resident per CU and C chunks of 32 K, a launch takes about
+//   (W sp / S + 1/2 round of tail) (C / sp + 2 chunks of start and end)
+// chunk times of a full CU (5.2 us: four workgroups' MFMAs), plus the traffic
+// of the partial tiles, written and read once per split (32 bytes per element
+// at about 4.5 TB/s); sp is where that is least, with at most 2 GiB of partials.
+int chi_gemm_nsplit(int prec, int ng, int nen, size_t kpad, int ncu) {
+  const int ntile = (ng + kTile - 1) / kTile;
+  const long kchunks = (long)(kpad / kKC), wgs = (long)ntile * ntile * nen;
+  if (prec != RP_PREC_FP64)
+    return (int)std::min<long>(kchunks, std::max<long>(1, (2048 + wgs - 1) / wgs));
+  const double per = 16.0 * ng * ng * nen;  // bytes of one partial set
+  const double cost = 2.0 * (double)wgs / (4.0 * ncu) + 2.0 * per / 4.5e6 / 5.2;
+  const double sp = std::min(std::sqrt(0.5 * (double)kchunks / cost), 2147483648.0 / per);
+  return (int)std::max(1.0, std::min((double)std::min<long>(kchunks, 64), std::round(sp)));
+}
+
 void launch_chi_gemm(int prec, const float2* A, size_t lda, const double2* dw, size_t ldd,
                      size_t kpad, int ng, int nen, int nsplit, double2* partial, hipStream_t s) {
   const int ntile = (ng + kTile - 1) / kTile;
   const size_t kchunks = kpad / kKC;
   const size_t per = (kchunks + nsplit - 1) / nsplit;
   dim3 grid(ntile * ntile, nen, nsplit);
+  constexpr size_t f = kKC / kF64KC;  // a split is a whole number of 32-row chunks in both
   switch (prec) {
     case RP_PREC_FP64:
-      hipLaunchKernelGGL(k_chi_gemm<RP_PREC_FP64>, grid, dim3(256), 0, s, A, lda, dw, ldd, per,
-                         kchunks, ng, ntile, nen, partial);
+      hipLaunchKernelGGL(k_chi_f64, grid, dim3(256), 0, s, A, lda, dw,
+                         ldd, per * f, kchunks * f, ng, ntile, nen, partial);
       break;
     case RP_PREC_FP32:
-      hipLaunchKernelGGL(k_chi_gemm<RP_PREC_FP32>, grid, dim3(256), 0, s, A, lda, dw, ldd, per,
-                         kchunks, ng, ntile, nen, partial);
+      hipLaunchKernelGGL(k_chi_gemm, grid, dim3(256), 0, s, A, lda, dw, ldd, per, kchunks, ng,
+                         ntile, nen, partial);
       break;
     default:
       throw Error("k_chi_gemm: FP64 or FP32 only (split-BF16 runs k_chi_bf16x3)");
