@@ -55,7 +55,7 @@ void swap_q(rp_ctx* h, QSlot& s) {
 
 void swap_scratch(rp_ctx* h, Scratch& s) {
   h->d_A.swap(s.d_A);
-  h->d_A3.swap(s.d_A3);
+  h->d_heads.swap(s.d_heads);
   h->d_wf.swap(s.d_wf);
   h->d_Ao.swap(s.d_Ao);
   h->d_sync.swap(s.d_sync);

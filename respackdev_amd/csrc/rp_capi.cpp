@@ -435,6 +435,7 @@ int rp_chiqw_prepare_q(rp_handle h, const double* qin, int32_t* ng, int32_t* lgo
       h->g0 = -1;
       for (int i = 0; i < h->ng; ++i)
         if (h->lg[3 * i] == 0 && h->lg[3 * i + 1] == 0 && h->lg[3 * i + 2] == 0) h->g0 = i;
+      RP_CHECK(!h->q0 || h->g0 >= 0, "G = 0 missing from the chi sphere at q = 0");
       const int ntk = h->ntk;
       h->ikq.assign(ntk, 0);
       h->shift.assign(3 * (size_t)ntk, 0);
@@ -572,14 +573,9 @@ void issue_pairdens(rp_ctx* h) {
                                h->nw[0], h->nw[1], h->nw[2], h->d_pdplan.p, h->pdplan[0], h->ng,
                                h->lda, (int)K, h->d_tw.p, h->d_A.p, s);
   if (h->q0) {
-    grow(h, h->d_A3, 3 * h->kpad * h->lda, "q = 0 pair-density buffer");
-    for (int ix = 0; ix < 3; ++ix)
-      if (h->kpad > K)
-        launch_zero(h->d_A3.p + (ix * h->kpad + K) * h->lda, (h->kpad - K) * h->lda * sizeof(float2), s);
-    // three copies laid out [ix][kpad][lda]
+    grow(h, h->d_heads, 3 * h->kpad, "q = 0 head buffer");
     launch_q0_heads(h->d_coef.p, h->d_kg0.p, h->d_ng0.p, h->ntk, h->ntg, h->d_pocc.p, h->d_pvir.p,
-                    h->d_eband.p, h->d_bvec.p, h->delt, h->g0, h->ng, h->lda, h->kpad, (int)K,
-                    h->d_A.p, h->d_A3.p, s);
+                    h->d_eband.p, h->d_bvec.p, h->delt, (int)K, h->kpad, h->d_heads.p, s);
   }
 }
 
@@ -615,7 +611,8 @@ void issue_operands(rp_ctx* h, int prec) {
   grow(h, h->d_Ao, h->kpad * h->lda * 8, "split operand buffer");
   grow(h, h->d_wf, (size_t)h->nen * h->kpad, "single-precision weight buffer");
   launch_weights_to_f32(h->d_w.p, (size_t)h->nen * h->kpad, h->d_wf.p, s);
-  launch_presplit(h->q0 ? h->d_A3.p : h->d_A.p, h->lda, h->kpad, h->d_Ao.p, s);
+  launch_presplit(h->d_A.p, h->lda, h->kpad, h->d_Ao.p, s);
+  if (h->q0) launch_presplit_column(h->d_heads.p, h->lda, h->kpad, h->g0, h->d_Ao.p, s);
 }
 
 void issue_accumulate(rp_ctx* h, int prec, const ChiLaunch& c, bool events, bool operands_ready) {
@@ -623,23 +620,47 @@ void issue_accumulate(rp_ctx* h, int prec, const ChiLaunch& c, bool events, bool
   const int ng = h->ng, nen = h->nen, nc = h->q0 ? 3 : 1;
   const size_t per = (size_t)ng * ng * nen;
   grow(h, h->d_chi, (size_t)nc * per, "chi buffer");
-  grow(h, h->d_part, (size_t)c.nsplit * per, "partial-sum buffer");
+  // (the head of a further direction at q = 0 needs at least 2 nen ng of it)
+  const size_t room = std::max((size_t)c.nsplit * per, 2 * (size_t)nen * ng);
+  grow(h, h->d_part, room, "partial-sum buffer");
   if (prec == RP_PREC_BF16X3) {
     grow(h, h->d_sync, bf16x3_sync_words(), "rendezvous counters");
     if (!operands_ready) issue_operands(h, prec);
   }
+  // At q = 0 the directions differ in the G = 0 column of A alone, so the second
+  // and third need only that row and column of chi: in FP64 one product for all
+  // frequencies (launch_chi_head), in the other precisions the tiles that hold
+  // them (2 ntile - 1 of ntile^2), whose elements keep their summation order.
+  // A metal at Gamma (NG 147, K 32000, 20 frequencies, FP64): three full
+  // contractions 6.2 ms, this 2.3 ms.
   for (int ix = 0; ix < nc; ++ix) {
-    const float2* A = h->q0 ? h->d_A3.p + (size_t)ix * h->kpad * h->lda : h->d_A.p;
-    if (prec == RP_PREC_BF16X3 && ix > 0) launch_presplit(A, h->lda, h->kpad, h->d_Ao.p, s);
+    const float2* head = h->d_heads.p + (size_t)ix * h->kpad;
+    const int cross = ix > 0 ? h->g0 : -1;
+    double2* chi = h->d_chi.p + (size_t)ix * per;
+    if (h->q0 && prec != RP_PREC_BF16X3)
+      launch_set_column(head, h->kpad, h->lda, h->g0, h->d_A.p, s);
+    if (ix > 0 && prec == RP_PREC_BF16X3)
+      launch_presplit_column(head, h->lda, h->kpad, h->g0, h->d_Ao.p, s);
     if (events) RP_HIP(hipEventRecord(h->gev[2 * ix], s));
+    if (ix > 0 && prec == RP_PREC_FP64) {
+      launch_chi_head(h->d_A.p, h->lda, h->d_w.p, h->kpad, h->kpad, ng, nen, head, 1.0 / h->volume,
+                      h->g0, h->d_chi.p, h->d_part.p, room, chi, s);
+      if (events) RP_HIP(hipEventRecord(h->gev[2 * ix + 1], s));
+      continue;
+    }
     if (prec == RP_PREC_BF16X3)
-      launch_chi_bf16x3(h->d_Ao.p, h->lda, h->d_wf.p, h->kpad, h->kpad, ng, nen, c.nsplit, c.nwg,
-                        c.span > 0 ? c.span : bf16x3_default_span(),
-                        h->d_part.p, h->d_sync.p, s);
+      launch_chi_bf16x3(h->d_Ao.p, h->lda, h->d_wf.p, h->kpad, h->kpad, ng, nen, c.nsplit, cross,
+                        c.nwg, c.span > 0 ? c.span : bf16x3_default_span(), h->d_part.p,
+                        h->d_sync.p, s);
     else
-      launch_chi_gemm(prec, A, h->lda, h->d_w.p, h->kpad, h->kpad, ng, nen, c.nsplit, h->d_part.p, s);
+      launch_chi_gemm(prec, h->d_A.p, h->lda, h->d_w.p, h->kpad, h->kpad, ng, nen, c.nsplit, cross,
+                      h->d_part.p, s);
     if (events) RP_HIP(hipEventRecord(h->gev[2 * ix + 1], s));
-    launch_chi_reduce(h->d_part.p, per, c.nsplit, 1.0 / h->volume, h->d_chi.p + (size_t)ix * per, s);
+    if (ix == 0)
+      launch_chi_reduce(h->d_part.p, per, c.nsplit, 1.0 / h->volume, chi, s);
+    else
+      launch_chi_reduce_cross(h->d_part.p, ng, nen, c.nsplit, 1.0 / h->volume, h->g0, h->d_chi.p,
+                              chi, s);
   }
 }
 
@@ -792,8 +813,9 @@ int rp_pairdens_batch(rp_handle h, float* m_out) {
     if (m_out) {
       const int nc = h->q0 ? 3 : 1;
       for (int ix = 0; ix < nc; ++ix) {
-        const float2* src = h->q0 ? h->d_A3.p + (size_t)ix * h->kpad * h->lda : h->d_A.p;
-        RP_HIP(hipMemcpy2DAsync(m_out + 2 * (size_t)ix * K * h->ng, sizeof(float2) * h->ng, src,
+        if (h->q0)
+          launch_set_column(h->d_heads.p + (size_t)ix * h->kpad, h->kpad, h->lda, h->g0, h->d_A.p, s);
+        RP_HIP(hipMemcpy2DAsync(m_out + 2 * (size_t)ix * K * h->ng, sizeof(float2) * h->ng, h->d_A.p,
                                 sizeof(float2) * h->lda, sizeof(float2) * h->ng, K, hipMemcpyDeviceToHost, s));
       }
     }

@@ -110,6 +110,18 @@ __global__ void __launch_bounds__(256) k_presplit(const float2* __restrict__ A, 
   for (int w = 0; w < 4; ++w) dst[w] = o[w];
 }
 
+// The octets of column g from H[K] (one direction's G = 0 entries at q = 0).
+__global__ void __launch_bounds__(256) k_presplit_column(const float2* __restrict__ H, size_t lda,
+                                                         size_t k8n, int g, u4v* __restrict__ Ao) {
+  const size_t k8 = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (k8 >= k8n) return;
+  u4v o[4];
+  make_octet(H + k8 * 8, o);
+  u4v* dst = Ao + (k8 * lda + g) * 4;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) dst[w] = o[w];
+}
+
 __device__ __forceinline__ bf8v as_bf8(u4v x) { return __builtin_bit_cast(bf8v, x); }
 
 // Element e (0..7) of one plane pair of an octet as hi + lo in FP32.
@@ -129,12 +141,13 @@ __global__ void k_weights_to_f32(const double2* __restrict__ dw, size_t n, float
 // per SIMD).  Item (split z, frequency w, tile) accumulates K chunks
 // [z*chunks_per_split, ...) into out, the FP64 partial [z][w][ng][ng] (element
 // (G,G') at G' * ng + G); every element of it is stored by exactly one item.
-// Columns of A beyond ng are zero; in edge tiles the waves whose rows or
+// cross >= 0: only the tiles of tile row and tile column `cross`.  Columns of A
+// beyond ng are zero; in edge tiles the waves whose rows or
 // columns all lie beyond ng skip their MFMAs.
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_chi_bf16x3(const u4v* __restrict__ Ao, size_t lda, const float2* __restrict__ df, size_t ldd,
              size_t chunks_per_split, size_t nchunks, int ng, int ntile, int nen, int nsplit,
-             int flush_chunks, double2* __restrict__ out, unsigned* __restrict__ sync) {
+             int flush_chunks, int cross, double2* __restrict__ out, unsigned* __restrict__ sync) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // two buffers of [left tile | right tile], each kTM (kTN) rows of kRowBytes
   constexpr int kBuf = (kTM + kTN) * kRowBytes;
@@ -147,7 +160,7 @@ k_chi_bf16x3(const u4v* __restrict__ Ao, size_t lda, const float2* __restrict__ 
   const int wm = (wave >> 2) & 1, wn = (wave + 2 * (wave >> 2)) & 3;
   const int li = lane & 15, q = lane >> 4;
   // this XCD's share of the (frequency, tile) pairs, walked split-major
-  const int ntiles = ntile * ntile, npairs = ntiles * nen;
+  const int ntiles = cross < 0 ? ntile * ntile : 2 * ntile - 1, npairs = ntiles * nen;
   const int xcd = (int)(blockIdx.x % kXcd), slot = (int)(blockIdx.x / kXcd);
   const int nslot = (int)(gridDim.x / kXcd);
   const int mypairs = (npairs - xcd + kXcd - 1) / kXcd;
@@ -165,7 +178,8 @@ k_chi_bf16x3(const u4v* __restrict__ Ao, size_t lda, const float2* __restrict__ 
   for (int item = slot; item < nitems; item += nslot) {
   const int z = item / mypairs, u = (item % mypairs) * kXcd + xcd;
   const int w = u / ntiles, tile = u % ntiles;
-  const int g0 = (tile % ntile) * kTM, h0 = (tile / ntile) * kTN;
+  const int2 tg = chi_tile_of(tile, ntile, cross);
+  const int g0 = tg.x * kTM, h0 = tg.y * kTN;
   const bool active = g0 + wm * 64 < ng && h0 + wn * 32 < ng;  // wave-uniform
   const float2* dww = df + (size_t)w * ldd;
   const size_t c0 = (size_t)z * chunks_per_split;
@@ -392,6 +406,13 @@ void launch_presplit(const float2* A, size_t lda, size_t kpad, void* Ao, hipStre
   RP_HIP(hipGetLastError());
 }
 
+void launch_presplit_column(const float2* H, size_t lda, size_t kpad, int g, void* Ao, hipStream_t s) {
+  const size_t k8n = kpad / 8;
+  hipLaunchKernelGGL(k_presplit_column, dim3((unsigned)((k8n + 255) / 256)), dim3(256), 0, s, H, lda,
+                     k8n, g, (u4v*)Ao);
+  RP_HIP(hipGetLastError());
+}
+
 void launch_weights_to_f32(const double2* dw, size_t n, float2* df, hipStream_t s) {
   unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 65536);
   hipLaunchKernelGGL(k_weights_to_f32, dim3(blocks), dim3(256), 0, s, dw, n, df);
@@ -436,8 +457,8 @@ int bf16x3_span_for_kappa(double kappa) {
 }
 
 void launch_chi_bf16x3(const void* Ao, size_t lda, const float2* df, size_t ldd, size_t kpad, int ng,
-                       int nen, int nsplit, int nwg, int span, double2* partial, unsigned* sync,
-                       hipStream_t s) {
+                       int nen, int nsplit, int cross, int nwg, int span, double2* partial,
+                       unsigned* sync, hipStream_t s) {
   RP_CHECK(span >= kKC && span % kKC == 0, "bf16x3 contraction: span must be a multiple of 32 K");
   RP_CHECK(lda % kTM == 0, "bf16x3 contraction needs lda a multiple of 128");
   RP_CHECK(kpad % kKC == 0, "bf16x3 contraction needs K padded to a multiple of 32");
@@ -451,7 +472,8 @@ void launch_chi_bf16x3(const void* Ao, size_t lda, const float2* df, size_t ldd,
   RP_HIP(hipFuncSetAttribute((const void*)k_chi_bf16x3, hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)lds));
   hipLaunchKernelGGL(k_chi_bf16x3, dim3(nwg), dim3(512), lds, s, (const u4v*)Ao, lda, df, ldd, per,
-                     nchunks, ng, ntile, nen, nsplit, span / kKC, partial, sync);
+                     nchunks, ng, ntile, nen, nsplit, span / kKC, cross < 0 ? -1 : cross / kTM, partial,
+                     sync);
   RP_HIP(hipGetLastError());
 }
 

@@ -55,13 +55,13 @@ __device__ inline void stage_chunk(const float2* __restrict__ A, size_t lda, siz
 __global__ void __launch_bounds__(256) k_chi_gemm(const float2* __restrict__ A, size_t lda,
                                                   const double2* __restrict__ dw, size_t ldd,
                                                   size_t kchunks_per_split, size_t kchunks,
-                                                  int ng, int ntile, int nen,
+                                                  int ng, int ntile, int nen, int cross,
                                                   double2* __restrict__ out) {
   __shared__ float2 sL[kTile][kLdsRow];
   __shared__ float2 sR[kTile][kLdsRow];
   __shared__ double2 sD[kKC];
-  const int tile = blockIdx.x;
-  const int tm = tile % ntile, tn = tile / ntile;
+  const int2 tg = chi_tile_of((int)blockIdx.x, ntile, cross);
+  const int tm = tg.x, tn = tg.y;
   const int g0 = tm * kTile, h0 = tn * kTile;
   const int w = blockIdx.y;
   const int z = blockIdx.z;
@@ -199,25 +199,37 @@ __device__ __forceinline__ void f64_chunk(const double* pl, const double* pr, in
     }
 }
 
+// HEAD: the row and the column of G = 0 of one direction at q = 0, whose column
+// of A is H.  The right columns are then c = (type, frequency), b = d_w H for
+// the column (type 0) and conj(d_w) H for the row (type 1, conjugated when
+// merged): every frequency in one product of NG x 2 nen x K instead of the
+// tiles of that row and column at each frequency.  out: partial[z][c][ng].
+template <bool HEAD>
 __global__ void __launch_bounds__(256, 4) k_chi_f64(const float2* __restrict__ A, size_t lda,
                                                     const double2* __restrict__ dw, size_t ldd,
                                                     size_t chunks_per_split, size_t nchunks,
                                                     int ng, int ntile, int nen,
+                                                    const float2* __restrict__ H,
                                                     double2* __restrict__ out) {
   __shared__ double sl[3 * kF64Plane], sr[3 * kF64Plane];
   const int tm = (int)blockIdx.x % ntile, tn = (int)blockIdx.x / ntile;
   const int nb = (ng + 15) / 16;
-  const int gb = tm * nb / ntile, hb = tn * nb / ntile;  // first block of the tile
+  const int ncol = HEAD ? 2 * nen : ng;
+  // first block of the tile in both axes and its blocks, 1..4
+  const int gb = tm * nb / ntile, hb = HEAD ? 4 * tn : tn * nb / ntile;
+  const int nr = (tm + 1) * nb / ntile - gb;
+  const int nc = HEAD ? min(4, (ncol + 15) / 16 - hb) : (tn + 1) * nb / ntile - hb;
   const int g0 = 16 * gb, h0 = 16 * hb;
   const int w = blockIdx.y, z = blockIdx.z;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int part = (wave + (int)(blockIdx.x + blockIdx.y + blockIdx.z)) & 3;
   const int li = lane & 15, lk = lane >> 4;
-  const double2* dww = dw + (size_t)w * ldd;
+  const int hc = h0 + lane < ncol ? h0 + lane : ncol - 1;  // HEAD: this lane's column
+  const double2* dww = dw + (size_t)(HEAD ? hc % nen : w) * ldd;
+  const double dsgn = HEAD && hc >= nen ? -1.0 : 1.0;
   const size_t c0 = (size_t)z * chunks_per_split;
   const size_t c1 = c0 + chunks_per_split < nchunks ? c0 + chunks_per_split : nchunks;
-  const int nr = (tm + 1) * nb / ntile - gb, nc = (tn + 1) * nb / ntile - hb;  // 1..4 blocks
 
   // thread (wave, lane) stages G = lane and G' = lane of the K rows wave and
   // wave + 4 of a chunk; the weight of a row is uniform in the wave
@@ -229,8 +241,9 @@ __global__ void __launch_bounds__(256, 4) k_chi_f64(const float2* __restrict__ A
     for (int e = 0; e < kE; ++e) {
       const size_t k = c * kF64KC + (size_t)(wave + 4 * e);
       la[e] = A[k * lda + g0 + lane];
-      ra[e] = A[k * lda + h0 + lane];
+      ra[e] = HEAD ? H[k] : A[k * lda + h0 + lane];
       dv[e] = dww[k];
+      if (HEAD) dv[e].y *= dsgn;
     }
   };
   auto stage = [&]() {
@@ -254,7 +267,7 @@ __global__ void __launch_bounds__(256, 4) k_chi_f64(const float2* __restrict__ A
   for (int p = 0; p < 3; ++p)
 #pragma unroll
     for (int i = 0; i < 4; ++i) acc[p][i] = d4v{0, 0, 0, 0};
-  double2* o = out + ((size_t)z * nen + w) * (size_t)ng * ng;
+  double2* o = out + ((size_t)z * (HEAD ? 1 : nen) + w) * (size_t)ng * ncol;
   // the chunk loop of a wave that owns NR x NC blocks from block (rb, cb) of
   // the tile on (none: it only stages)
   auto tile = [&](auto rows, auto cols, int rb, int cb) {
@@ -277,7 +290,7 @@ __global__ void __launch_bounds__(256, 4) k_chi_f64(const float2* __restrict__ A
           const int hj = h0 + (cb + b) * 16 + lk + 4 * v;
           const int i = a * NC + b;
           const double t1 = acc[0][i][v], t2 = acc[1][i][v], t3 = acc[2][i][v];
-          if (gi < ng && hj < ng) o[(size_t)hj * ng + gi] = make_double2(t1 + t2, t3 - t1 + t2);
+          if (gi < ng && hj < ncol) o[(size_t)hj * ng + gi] = make_double2(t1 + t2, t3 - t1 + t2);
         }
   };
   using std::integral_constant;
@@ -318,6 +331,34 @@ __global__ void k_chi_reduce(const double2* __restrict__ part, size_t n, int nsp
   }
 }
 
+// chi of a further direction at q = 0: row and column g from its own partials
+// (HEAD: k_chi_f64<true>'s [z][2][nen][ng], else tiles in chi's layout), every
+// other element the first direction's (the same operands).
+template <bool HEAD>
+__global__ void k_chi_reduce_cross(const double2* __restrict__ part, int ng, int nen, int nsplit,
+                                   double inv_vol, int g, const double2* __restrict__ chi0,
+                                   double2* __restrict__ chi) {
+  const size_t n = (size_t)ng * ng * nen, nh = 2 * (size_t)nen * ng;
+  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
+       i += (size_t)gridDim.x * blockDim.x) {
+    const int gi = (int)(i % ng), hj = (int)(i / ng % ng);
+    if (gi != g && hj != g) {
+      chi[i] = chi0[i];
+      continue;
+    }
+    const bool col = hj == g;
+    const size_t w = i / ((size_t)ng * ng);
+    const size_t at = HEAD ? (col ? w * ng + gi : (nen + w) * ng + hj) : i;
+    double x = 0.0, y = 0.0;
+    for (int z = 0; z < nsplit; ++z) {
+      const double2 v = part[(size_t)z * (HEAD ? nh : n) + at];
+      x += v.x;
+      y += HEAD && !col ? -v.y : v.y;
+    }
+    chi[i] = make_double2(x * inv_vol, y * inv_vol);
+  }
+}
+
 int chi_tile() { return kTile; }
 int chi_kchunk() { return kKC; }
 
@@ -339,20 +380,22 @@ int chi_gemm_nsplit(int prec, int ng, int nen, size_t kpad, int ncu) {
 }
 
 void launch_chi_gemm(int prec, const float2* A, size_t lda, const double2* dw, size_t ldd,
-                     size_t kpad, int ng, int nen, int nsplit, double2* partial, hipStream_t s) {
+                     size_t kpad, int ng, int nen, int nsplit, int cross, double2* partial,
+                     hipStream_t s) {
   const int ntile = (ng + kTile - 1) / kTile;
   const size_t kchunks = kpad / kKC;
   const size_t per = (kchunks + nsplit - 1) / nsplit;
-  dim3 grid(ntile * ntile, nen, nsplit);
+  dim3 grid(cross < 0 ? ntile * ntile : 2 * ntile - 1, nen, nsplit);
   constexpr size_t f = kKC / kF64KC;  // a split is a whole number of 32-row chunks in both
   switch (prec) {
     case RP_PREC_FP64:
-      hipLaunchKernelGGL(k_chi_f64, grid, dim3(256), 0, s, A, lda, dw,
-                         ldd, per * f, kchunks * f, ng, ntile, nen, partial);
+      RP_CHECK(cross < 0, "k_chi_f64: row and column of one G are launch_chi_head's");
+      hipLaunchKernelGGL(k_chi_f64<false>, grid, dim3(256), 0, s, A, lda, dw, ldd, per * f,
+                         kchunks * f, ng, ntile, nen, (const float2*)nullptr, partial);
       break;
     case RP_PREC_FP32:
       hipLaunchKernelGGL(k_chi_gemm, grid, dim3(256), 0, s, A, lda, dw, ldd, per, kchunks, ng,
-                         ntile, nen, partial);
+                         ntile, nen, cross < 0 ? -1 : cross / kTile, partial);
       break;
     default:
       throw Error("k_chi_gemm: FP64 or FP32 only (split-BF16 runs k_chi_bf16x3)");
@@ -378,6 +421,35 @@ void launch_zero(void* p, size_t bytes, hipStream_t s) {
   if (blocks < 1) blocks = 1;
   hipLaunchKernelGGL(k_zero, dim3(blocks), dim3(256), 0, s, (uint4*)p, n16,
                      (unsigned*)((char*)p + n16 * 16), ntail);
+  RP_HIP(hipGetLastError());
+}
+
+void launch_chi_reduce_cross(const double2* partial, int ng, int nen, int nsplit, double inv_vol,
+                             int g, const double2* chi0, double2* chi, hipStream_t s) {
+  const unsigned blocks = (unsigned)std::min<size_t>(((size_t)ng * ng * nen + 255) / 256, 65536);
+  hipLaunchKernelGGL(k_chi_reduce_cross<false>, dim3(blocks), dim3(256), 0, s, partial, ng, nen,
+                     nsplit, inv_vol, g, chi0, chi);
+  RP_HIP(hipGetLastError());
+}
+
+// One further direction at q = 0 in FP64 (its column g of A in place, H that
+// column): row and column g, then the merge with the first direction's chi.
+// room: double2 elements of partial.
+void launch_chi_head(const float2* A, size_t lda, const double2* dw, size_t ldd, size_t kpad, int ng,
+                     int nen, const float2* H, double inv_vol, int g, const double2* chi0,
+                     double2* partial, size_t room, double2* chi, hipStream_t s) {
+  const int ntile = (ng + kTile - 1) / kTile, ctile = (2 * nen + kTile - 1) / kTile;
+  const size_t kchunks = kpad / kF64KC;
+  // a split of at least 16 chunks each, at most 64, within the partials' room
+  size_t nsplit = std::min<size_t>(std::max<size_t>(1, kchunks / 16), 64);
+  nsplit = std::min(nsplit, room / ((size_t)2 * nen * ng));
+  RP_CHECK(nsplit >= 1, "chi head: no room for its partials");
+  const size_t per = (kchunks + nsplit - 1) / nsplit;
+  hipLaunchKernelGGL(k_chi_f64<true>, dim3(ntile * ctile, 1, (unsigned)nsplit), dim3(256), 0, s, A,
+                     lda, dw, ldd, per, kchunks, ng, ntile, nen, H, partial);
+  const unsigned blocks = (unsigned)std::min<size_t>(((size_t)ng * ng * nen + 255) / 256, 65536);
+  hipLaunchKernelGGL(k_chi_reduce_cross<true>, dim3(blocks), dim3(256), 0, s, partial, ng, nen,
+                     (int)nsplit, inv_vol, g, chi0, chi);
   RP_HIP(hipGetLastError());
 }
 

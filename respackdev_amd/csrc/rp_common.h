@@ -103,6 +103,14 @@ __host__ __device__ inline zd operator/(zd a, zd b) {
 }
 __host__ __device__ inline zd operator/(double s, zd b) { return zd{s, 0.0} / b; }
 __host__ __device__ inline double absz(zd a) { return hypot(a.x, a.y); }
+// Tile (row, column) number `tile` of a contraction launch: all ntile x ntile,
+// rows fastest, or with cross >= 0 the 2 ntile - 1 of row and column `cross`.
+__device__ __forceinline__ int2 chi_tile_of(int tile, int ntile, int cross) {
+  if (cross < 0) return make_int2(tile % ntile, tile / ntile);
+  if (tile < ntile) return make_int2(tile, cross);
+  const int c = tile - ntile;
+  return make_int2(cross, c < cross ? c : c + 1);
+}
 __device__ __forceinline__ zd logz(zd a) { return {log(hypot(a.x, a.y)), atan2(a.y, a.x)}; }
 
 }  // namespace rp

@@ -92,7 +92,7 @@ struct QSlot {
 
 // Work buffers of the stages (shared by all q of one launch sequence).
 struct Scratch {
-  DevBuf<float2> d_A, d_A3, d_wf;
+  DevBuf<float2> d_A, d_heads, d_wf;
   DevBuf<unsigned char> d_Ao;
   DevBuf<unsigned> d_sync;
   DevBuf<double2> d_w, d_part, d_chi, d_drude;
@@ -167,7 +167,8 @@ struct rp_ctx {
   double prep_seconds = 0;
   DevBuf<int> d_lg, d_ikq, d_shift, d_pocc, d_pvir, d_intra, d_pdplan, d_status, d_ipiv, d_gjwork;
   DevBuf<double2> d_drude;  // per intraband band and direction: sum_k Im x(k) p(k)^2
-  DevBuf<float2> d_A, d_A3;
+  DevBuf<float2> d_A;
+  DevBuf<float2> d_heads;      // q = 0: the G = 0 column of A per direction, [3][kpad]
   DevBuf<unsigned char> d_Ao;  // split-bf16 octets of the left operand
   DevBuf<float2> d_wf;         // single-precision copy of the weights
   DevBuf<unsigned> d_sync;     // per-XCD rendezvous counters of the split-BF16 contraction

@@ -72,8 +72,8 @@ void launch_rho_from_grid_hbm(double2* P, int npair, int nx, int ny, int nz, con
                               int ntk, const double2* twtab, double2* rho, hipStream_t s);
 void launch_q0_heads(const double2* coef, const int* kg, const int* ng0, int ntk, int ntg,
                      const int* pocc, const int* pvir, const double* eband, const double* bvec,
-                     double delt, int g0, int ng, size_t lda, size_t rows, int nK, const float2* A,
-                     float2* A3, hipStream_t s);
+                     double delt, int nK, size_t rows, float2* H, hipStream_t s);
+void launch_set_column(const float2* H, size_t n, size_t lda, int g, float2* A, hipStream_t s);
 
 // rp_tetra.hip
 size_t tetra_lds_bytes(int nk3, int nf);
@@ -95,7 +95,13 @@ int chi_tile();
 int chi_kchunk();
 int chi_gemm_nsplit(int prec, int ng, int nen, size_t kpad, int ncu);
 void launch_chi_gemm(int prec, const float2* A, size_t lda, const double2* dw, size_t ldd,
-                     size_t kpad, int ng, int nen, int nsplit, double2* partial, hipStream_t s);
+                     size_t kpad, int ng, int nen, int nsplit, int cross, double2* partial,
+                     hipStream_t s);
+void launch_chi_head(const float2* A, size_t lda, const double2* dw, size_t ldd, size_t kpad, int ng,
+                     int nen, const float2* H, double inv_vol, int g, const double2* chi0,
+                     double2* partial, size_t room, double2* chi, hipStream_t s);
+void launch_chi_reduce_cross(const double2* partial, int ng, int nen, int nsplit, double inv_vol,
+                             int g, const double2* chi0, double2* chi, hipStream_t s);
 void launch_chi_reduce(const double2* partial, size_t n, int nsplit, double inv_vol, double2* chi,
                        hipStream_t s);
 // zero `bytes` (a multiple of 4) at p (16-byte aligned) with a fill kernel
@@ -103,6 +109,7 @@ void launch_zero(void* p, size_t bytes, hipStream_t s);
 
 // rp_chi_bf16.hip
 size_t bf16x3_lda_multiple();
+void launch_presplit_column(const float2* H, size_t lda, size_t kpad, int g, void* Ao, hipStream_t s);
 void launch_presplit(const float2* A, size_t lda, size_t kpad, void* Ao, hipStream_t s);
 void launch_weights_to_f32(const double2* dw, size_t n, float2* df, hipStream_t s);
 int bf16x3_nsplit(int ng, int nen, size_t kpad, int nwg);
@@ -114,7 +121,7 @@ int bf16x3_default_span();
 // has 1-norm kappa (the amplification of chi's error)
 int bf16x3_span_for_kappa(double kappa);
 void launch_chi_bf16x3(const void* Ao, size_t lda, const float2* df, size_t ldd, size_t kpad, int ng,
-                       int nen, int nsplit, int nwg, int span, double2* partial, unsigned* sync,
+                       int nen, int nsplit, int cross, int nwg, int span, double2* partial, unsigned* sync,
                        hipStream_t s);
 
 // rp_dyson.hip

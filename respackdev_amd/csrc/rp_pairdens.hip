@@ -777,15 +777,21 @@ __global__ void __launch_bounds__(256) k_rho_from_grid(
 #undef RP_PD_SWITCH
 
 // q = 0: the G = 0 entry per direction ix is -i<vir|p|occ>/de (calc_VMab,
-// chiqw_sub.F:207-232, and chiqw.F:1787-1805), zero when |de| <= delt.
-// Writes three copies A3[ix][K][lda] from A[K][lda] with that entry replaced.
-// grid: K blocks, 64 threads.  coef as in k_band_grids.
+// chiqw_sub.F:207-232, and chiqw.F:1787-1805), zero when |de| <= delt, to
+// H[ix][K] (ld rows, which pads with zeros).  The three directions' pair
+// densities differ in that column alone: A holds the rest once, and each
+// direction puts its column in place (k_set_column, or the split octets'
+// k_presplit_column).  grid: rows blocks, 64 threads.  coef as in k_band_grids.
 __global__ void __launch_bounds__(64) k_q0_heads(
     const double2* __restrict__ coef, const int* __restrict__ kg, const int* __restrict__ ng0,
     int ntk, int ntg, const int* __restrict__ pocc, const int* __restrict__ pvir,
-    const double* __restrict__ eband, const double* bvec, double delt, int g0, int ng,
-    size_t lda, size_t rows, const float2* __restrict__ A, float2* __restrict__ A3) {
+    const double* __restrict__ eband, const double* bvec, double delt, int nK,
+    size_t rows, float2* __restrict__ H) {
   const int K = blockIdx.x;
+  if (K >= nK) {  // padding row (uniform)
+    if (threadIdx.x < 3) H[threadIdx.x * rows + K] = make_float2(0.f, 0.f);
+    return;
+  }
   const int p = K / ntk, k = K % ntk;
   const int jo = pocc[p], iv = pvir[p];
   const double2* ck = coef + ((size_t)jo * ntk + k) * ntg;
@@ -814,18 +820,20 @@ __global__ void __launch_bounds__(64) k_q0_heads(
   }
   double de = eband[(size_t)iv * ntk + k] - eband[(size_t)jo * ntk + k];
   if (fabs(de) < delt) de = delt;
-  const float2* src = A + (size_t)K * lda;
-  for (int ix = 0; ix < 3; ++ix) {
-    float2* dst = A3 + ((size_t)ix * rows + K) * lda;
-    for (int i = threadIdx.x; i < (int)lda; i += blockDim.x) dst[i] = src[i];
-    __syncthreads();
-    if (threadIdx.x == 0 && g0 >= 0 && g0 < ng) {
-      // vm = i*S ; vm = -i*(vm - 0)/de = S/de
-      double vr = red[2 * ix][0] / de, vi = red[2 * ix + 1][0] / de;
-      // m_tmp is complex(8) in the reference (no single rounding of this entry)
-      dst[g0] = fabs(de) <= delt ? make_float2(0.f, 0.f) : make_float2((float)vr, (float)vi);
-    }
+  if (threadIdx.x < 3) {
+    const int ix = threadIdx.x;
+    // vm = i*S ; vm = -i*(vm - 0)/de = S/de
+    const double vr = red[2 * ix][0] / de, vi = red[2 * ix + 1][0] / de;
+    // m_tmp is complex(8) in the reference (no single rounding of this entry)
+    H[ix * rows + K] = fabs(de) <= delt ? make_float2(0.f, 0.f) : make_float2((float)vr, (float)vi);
   }
+}
+
+// A[K][g] = H[K] for the n rows K.
+__global__ void __launch_bounds__(256) k_set_column(const float2* __restrict__ H, size_t n,
+                                                    size_t lda, int g, float2* __restrict__ A) {
+  const size_t K = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  if (K < n) A[K * lda + g] = H[K];
 }
 
 size_t twiddle_entries() { return 2 * (size_t)kTwHalf; }
@@ -1069,10 +1077,15 @@ size_t pruned_transform_lds_bytes(int nx, int ny, int nz, int nzz) {
 
 void launch_q0_heads(const double2* coef, const int* kg, const int* ng0, int ntk, int ntg,
                      const int* pocc, const int* pvir, const double* eband, const double* bvec,
-                     double delt, int g0, int ng, size_t lda, size_t rows, int nK, const float2* A,
-                     float2* A3, hipStream_t s) {
-  hipLaunchKernelGGL(k_q0_heads, dim3(nK), dim3(64), 0, s, coef, kg, ng0, ntk, ntg, pocc, pvir,
-                     eband, bvec, delt, g0, ng, lda, rows, A, A3);
+                     double delt, int nK, size_t rows, float2* H, hipStream_t s) {
+  hipLaunchKernelGGL(k_q0_heads, dim3((unsigned)rows), dim3(64), 0, s, coef, kg, ng0, ntk, ntg, pocc,
+                     pvir, eband, bvec, delt, nK, rows, H);
+  RP_HIP(hipGetLastError());
+}
+
+void launch_set_column(const float2* H, size_t n, size_t lda, int g, float2* A, hipStream_t s) {
+  hipLaunchKernelGGL(k_set_column, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, H, n, lda, g,
+                     A);
   RP_HIP(hipGetLastError());
 }
 
