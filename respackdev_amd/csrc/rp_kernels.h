@@ -173,6 +173,7 @@ void launch_w_fourier(const double2* func, const double2* funcw, const double* s
 // band-tail closure network (rp_mlp.hip)
 int mlp_max_width();
 int mlp_chunk();
+int mlp_row_slack();  // rows readable past the batch in the inputs of launch_linear_fwd
 void launch_to_bf16(const float* src, size_t n, unsigned short* dst, hipStream_t s);
 void launch_linear_fwd(const float* A, int n, int nin, const unsigned short* W, const float* b, int nout,
                        int act, float* Z, float* Aout, hipStream_t s);

@@ -38,7 +38,7 @@ void reserve_batch(Mlp& m, int n) {
   }
   for (int d : m.dims) wmax = std::max(wmax, d);
   m.d_z.reserve(tot);
-  m.d_a.reserve(tot);
+  m.d_a.reserve(tot + (size_t)mlp_row_slack() * wmax);
   m.d_dz0.reserve((size_t)n * wmax);
   m.d_dz1.reserve((size_t)n * wmax);
   const size_t nchunks = ((size_t)n + mlp_chunk() - 1) / mlp_chunk();
@@ -46,17 +46,21 @@ void reserve_batch(Mlp& m, int n) {
   m.nmax = n;
 }
 
-// Forward pass over n samples at x (device, [n][nin]); returns the output (device).
-const float* forward(Mlp& m, const float* x, int n, hipStream_t s) {
+// BF16 copy of the parameters, for the forward passes until they change.
+void to_bf16(Mlp& m, hipStream_t s) { launch_to_bf16(m.d_p.p, m.nparams, m.d_pb.p, s); }
+
+// Forward pass over n samples at x (device, [n][nin]) with the current BF16
+// copy; returns the output (device).  keep: the hidden pre-activations are
+// kept for backward().
+const float* forward(Mlp& m, const float* x, int n, bool keep, hipStream_t s) {
   const int L = nlayers(m);
-  launch_to_bf16(m.d_p.p, m.nparams, m.d_pb.p, s);
   const float* a = x;
   for (int l = 1; l <= L; ++l) {
     float* z = m.d_z.p + m.aoff[l];
     float* an = m.d_a.p + m.aoff[l];
     const int act = l < L ? 1 : 0;
     launch_linear_fwd(a, n, m.dims[l - 1], m.d_pb.p + m.woff[l - 1], m.d_p.p + m.boff[l - 1], m.dims[l], act,
-                      z, an, s);
+                      act && !keep ? nullptr : z, an, s);
     a = an;
   }
   return m.d_z.p + m.aoff[L];
@@ -172,11 +176,12 @@ int rp_mlp_forward(rp_handle h, int64_t n, const float* x, float* y) {
     const int nin = m.dims.front(), nout = m.dims.back();
     const int64_t blk = 65536;
     reserve_batch(m, (int)std::min<int64_t>(n, blk));
-    m.d_xb.reserve((size_t)std::min<int64_t>(n, blk) * nin);
+    m.d_xb.reserve(((size_t)std::min<int64_t>(n, blk) + mlp_row_slack()) * nin);
+    to_bf16(m, s);
     for (int64_t r0 = 0; r0 < n; r0 += blk) {
       const int nb = (int)std::min<int64_t>(blk, n - r0);
       RP_HIP(hipMemcpyAsync(m.d_xb.p, x + (size_t)r0 * nin, sizeof(float) * nb * nin, hipMemcpyHostToDevice, s));
-      const float* dy = forward(m, m.d_xb.p, nb, s);
+      const float* dy = forward(m, m.d_xb.p, nb, false, s);
       RP_HIP(hipMemcpyAsync(y + (size_t)r0 * nout, dy, sizeof(float) * nb * nout, hipMemcpyDeviceToHost, s));
       RP_HIP(hipStreamSynchronize(s));
     }
@@ -191,11 +196,12 @@ int rp_mlp_gradient(rp_handle h, int64_t n, const float* x, const float* t, floa
     hipStream_t s = h->stream;
     const int nin = m.dims.front(), nout = m.dims.back();
     reserve_batch(m, (int)n);
-    m.d_xb.reserve((size_t)n * nin);
+    m.d_xb.reserve(((size_t)n + mlp_row_slack()) * nin);
     m.d_tb.reserve((size_t)n * nout);
     RP_HIP(hipMemcpyAsync(m.d_xb.p, x, sizeof(float) * n * nin, hipMemcpyHostToDevice, s));
     RP_HIP(hipMemcpyAsync(m.d_tb.p, t, sizeof(float) * n * nout, hipMemcpyHostToDevice, s));
-    forward(m, m.d_xb.p, (int)n, s);
+    to_bf16(m, s);
+    forward(m, m.d_xb.p, (int)n, true, s);
     const double l = backward(m, m.d_xb.p, m.d_tb.p, (int)n, s);
     RP_HIP(hipMemcpy(grad, m.d_g.p, sizeof(float) * m.nparams, hipMemcpyDeviceToHost));
     if (loss) *loss = l;
@@ -214,7 +220,7 @@ int rp_mlp_train(rp_handle h, int64_t n, const float* x, const float* t, int32_t
     m.d_x.upload(x, (size_t)n * nin, s);
     m.d_t.upload(t, (size_t)n * nout, s);
     reserve_batch(m, batch);
-    m.d_xb.reserve((size_t)batch * nin);
+    m.d_xb.reserve(((size_t)batch + mlp_row_slack()) * nin);
     m.d_tb.reserve((size_t)batch * nout);
     m.d_idx.reserve(batch);
     std::mt19937_64 g(seed);
@@ -224,7 +230,8 @@ int rp_mlp_train(rp_handle h, int64_t n, const float* x, const float* t, int32_t
       for (int j = 0; j < batch; ++j) idx[j] = (int)(g() % (uint64_t)n);
       RP_HIP(hipMemcpyAsync(m.d_idx.p, idx.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
       launch_gather_rows(m.d_x.p, m.d_t.p, m.d_idx.p, batch, nin, nout, m.d_xb.p, m.d_tb.p, s);
-      forward(m, m.d_xb.p, batch, s);
+      to_bf16(m, s);
+      forward(m, m.d_xb.p, batch, true, s);
       const double l = backward(m, m.d_xb.p, m.d_tb.p, batch, s);  // synchronizes: idx may be refilled
       ++m.step;
       const double c1 = 1.0 - std::pow((double)b1, (double)m.step);
