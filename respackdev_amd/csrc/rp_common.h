@@ -75,6 +75,29 @@ struct DevBuf {
   }
 };
 
+// Owning pinned host buffer.
+template <class T>
+struct HostBuf {
+  T* p = nullptr;
+  size_t n = 0;
+  HostBuf() = default;
+  HostBuf(const HostBuf&) = delete;
+  HostBuf& operator=(const HostBuf&) = delete;
+  ~HostBuf() { release(); }
+  void release() {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    n = 0;
+  }
+  void reserve(size_t m) {
+    if (m <= n && p) return;
+    release();
+    if (m == 0) return;
+    RP_HIP(hipHostMalloc((void**)&p, m * sizeof(T), hipHostMallocDefault));
+    n = m;
+  }
+};
+
 // ------------------------------------------------------------ device complex
 struct zd {
   double x, y;

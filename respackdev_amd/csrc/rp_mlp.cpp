@@ -39,59 +39,90 @@ void reserve_batch(Mlp& m, int n) {
   for (int d : m.dims) wmax = std::max(wmax, d);
   m.d_z.reserve(tot);
   m.d_a.reserve(tot + (size_t)mlp_row_slack() * wmax);
-  m.d_dz0.reserve((size_t)n * wmax);
-  m.d_dz1.reserve((size_t)n * wmax);
-  const size_t nchunks = ((size_t)n + mlp_chunk() - 1) / mlp_chunk();
-  m.d_part.reserve(nchunks * (size_t)wmax * (wmax + 1));
+  m.d_dz0.reserve(((size_t)n + mlp_row_slack()) * wmax);
+  m.d_dz1.reserve(((size_t)n + mlp_row_slack()) * wmax);
   m.nmax = n;
 }
 
 // BF16 copy of the parameters, for the forward passes until they change.
 void to_bf16(Mlp& m, hipStream_t s) { launch_to_bf16(m.d_p.p, m.nparams, m.d_pb.p, s); }
 
-// Forward pass over n samples at x (device, [n][nin]) with the current BF16
-// copy; returns the output (device).  keep: the hidden pre-activations are
-// kept for backward().
-const float* forward(Mlp& m, const float* x, int n, bool keep, hipStream_t s) {
-  const int L = nlayers(m);
+// The hidden layers over n samples at x (device, [n][nin]) with the current BF16
+// copy; returns the output layer's input.  keep: the pre-activations are kept
+// for backward().
+const float* hidden(Mlp& m, const float* x, int n, bool keep, hipStream_t s) {
   const float* a = x;
-  for (int l = 1; l <= L; ++l) {
-    float* z = m.d_z.p + m.aoff[l];
+  for (int l = 1; l < nlayers(m); ++l) {
     float* an = m.d_a.p + m.aoff[l];
-    const int act = l < L ? 1 : 0;
-    launch_linear_fwd(a, n, m.dims[l - 1], m.d_pb.p + m.woff[l - 1], m.d_p.p + m.boff[l - 1], m.dims[l], act,
-                      act && !keep ? nullptr : z, an, s);
+    launch_linear_fwd(a, n, m.dims[l - 1], m.d_pb.p + m.woff[l - 1], m.d_p.p + m.boff[l - 1], m.dims[l], 1,
+                      keep ? m.d_z.p + m.aoff[l] : nullptr, an, s);
     a = an;
   }
-  return m.d_z.p + m.aoff[L];
+  return a;
 }
 
-// Mean-squared-error gradient into d_g after forward(); returns the loss.
-double backward(Mlp& m, const float* x, const float* t, int n, hipStream_t s) {
+// Forward pass; returns the output (device).
+const float* forward(Mlp& m, const float* x, int n, hipStream_t s) {
   const int L = nlayers(m);
-  const float* y = m.d_z.p + m.aoff[L];
-  const size_t mo = (size_t)n * m.dims[L];
-  const int nb = (int)std::min<size_t>((mo + 255) / 256, 1024);
-  m.d_loss.reserve(nb);
+  const float* a = hidden(m, x, n, false, s);
+  float* y = m.d_z.p + m.aoff[L];
+  launch_linear_fwd(a, n, m.dims[L - 1], m.d_pb.p + m.woff[L - 1], m.d_p.p + m.boff[L - 1], m.dims[L], 0, y,
+                    nullptr, s);
+  return y;
+}
+
+// An Adam step's constants.
+struct Adam {
+  float lr_t, b1, b2, c2, eps;
+};
+
+// Forward pass over n samples and the mean-squared-error gradient into d_g, the
+// loss partials into lossp (launch_output_loss_blocks of them); with adam, the
+// step and the new BF16 copy.  The gradient partials of all layers are reduced
+// by one launch, or layer by layer above kMergedChunks chunks (the partials of
+// one layer are then held at a time).  Enqueues only.
+constexpr int kMergedChunks = 512;
+void step_all(Mlp& m, const float* x, const float* t, int n, double* lossp, const Adam* adam,
+              hipStream_t s) {
+  const int L = nlayers(m), nchunks = (n + mlp_chunk() - 1) / mlp_chunk();
+  const bool merged = nchunks <= kMergedChunks;
+  std::vector<size_t> poff(L, 0);
+  size_t tot = 0, most = 0;
+  for (int l = 0; l < L; ++l) {
+    const size_t per = (size_t)nchunks * m.dims[l + 1] * (m.dims[l] + 1);
+    if (merged) poff[l] = tot;
+    tot += per;
+    most = std::max(most, per);
+  }
+  m.d_part.reserve(merged ? tot : most);
+  const float* a = hidden(m, x, n, true, s);
   float* dz = m.d_dz0.p;
   float* dzn = m.d_dz1.p;
-  launch_mse(y, t, mo, 1.0f / (float)mo, dz, m.d_loss.p, nb, s);
+  launch_output_loss(a, n, m.dims[L - 1], m.d_pb.p + m.woff[L - 1], m.d_p.p + m.boff[L - 1], m.dims[L], t,
+                     1.0f / (float)((size_t)n * m.dims[L]), m.d_z.p + m.aoff[L], dz, lossp, s);
+  auto finish = [&](int l0, int l1, const float* part, bool step) {
+    const Adam c = step ? *adam : Adam{0, 0, 0, 0, 0};
+    launch_finish(l0, l1, m.dims.data(), m.woff.data(), poff.data() + l0, part, nchunks, m.d_g.p, m.d_p.p,
+                  m.d_pb.p, step ? m.d_m1.p : nullptr, step ? m.d_m2.p : nullptr, c.lr_t, c.b1, c.b2, c.c2,
+                  c.eps, s);
+  };
   for (int l = L; l >= 1; --l) {
     const float* ain = l == 1 ? x : m.d_a.p + m.aoff[l - 1];
-    launch_linear_bwd_w(dz, ain, n, m.dims[l - 1], m.dims[l], m.d_part.p, m.d_g.p + m.woff[l - 1],
-                        m.d_g.p + m.boff[l - 1], s);
-    if (l > 1) {
-      launch_linear_bwd_data(dz, n, m.dims[l], m.d_pb.p + m.woff[l - 1], m.dims[l - 1],
-                             m.d_z.p + m.aoff[l - 1], 1, dzn, s);
-      std::swap(dz, dzn);
-    }
+    launch_bwd_layer(dz, ain, n, m.dims[l - 1], m.dims[l], m.d_pb.p + m.woff[l - 1],
+                     l > 1 ? m.d_z.p + m.aoff[l - 1] : nullptr, l > 1 ? dzn : nullptr,
+                     m.d_part.p + poff[l - 1], s);
+    std::swap(dz, dzn);
+    if (!merged) finish(l - 1, l, m.d_part.p, false);
   }
-  std::vector<double> lp(nb);
-  RP_HIP(hipMemcpyAsync(lp.data(), m.d_loss.p, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
-  RP_HIP(hipStreamSynchronize(s));
+  if (merged) finish(0, L, m.d_part.p, adam != nullptr);
+  else if (adam) finish(0, L, nullptr, true);
+}
+
+// Sum of the loss partials of one step over the values they average.
+double loss_of(const double* lp, int nb, size_t values) {
   double sum = 0.0;
-  for (double v : lp) sum += v;
-  return sum / (double)mo;
+  for (int i = 0; i < nb; ++i) sum += lp[i];
+  return sum / (double)values;
 }
 
 // Uniform in [-1, 1) from the raw 64-bit stream (independent of the library's
@@ -181,7 +212,7 @@ int rp_mlp_forward(rp_handle h, int64_t n, const float* x, float* y) {
     for (int64_t r0 = 0; r0 < n; r0 += blk) {
       const int nb = (int)std::min<int64_t>(blk, n - r0);
       RP_HIP(hipMemcpyAsync(m.d_xb.p, x + (size_t)r0 * nin, sizeof(float) * nb * nin, hipMemcpyHostToDevice, s));
-      const float* dy = forward(m, m.d_xb.p, nb, false, s);
+      const float* dy = forward(m, m.d_xb.p, nb, s);
       RP_HIP(hipMemcpyAsync(y + (size_t)r0 * nout, dy, sizeof(float) * nb * nout, hipMemcpyDeviceToHost, s));
       RP_HIP(hipStreamSynchronize(s));
     }
@@ -200,11 +231,15 @@ int rp_mlp_gradient(rp_handle h, int64_t n, const float* x, const float* t, floa
     m.d_tb.reserve((size_t)n * nout);
     RP_HIP(hipMemcpyAsync(m.d_xb.p, x, sizeof(float) * n * nin, hipMemcpyHostToDevice, s));
     RP_HIP(hipMemcpyAsync(m.d_tb.p, t, sizeof(float) * n * nout, hipMemcpyHostToDevice, s));
+    const int nb = launch_output_loss_blocks((int)n, nout);
+    m.d_loss.reserve(nb);
     to_bf16(m, s);
-    forward(m, m.d_xb.p, (int)n, true, s);
-    const double l = backward(m, m.d_xb.p, m.d_tb.p, (int)n, s);
-    RP_HIP(hipMemcpy(grad, m.d_g.p, sizeof(float) * m.nparams, hipMemcpyDeviceToHost));
-    if (loss) *loss = l;
+    step_all(m, m.d_xb.p, m.d_tb.p, (int)n, m.d_loss.p, nullptr, s);
+    std::vector<double> lp(nb);
+    RP_HIP(hipMemcpyAsync(lp.data(), m.d_loss.p, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
+    RP_HIP(hipMemcpyAsync(grad, m.d_g.p, sizeof(float) * m.nparams, hipMemcpyDeviceToHost, s));
+    RP_HIP(hipStreamSynchronize(s));
+    if (loss) *loss = loss_of(lp.data(), nb, (size_t)n * nout);
   });
 }
 
@@ -222,22 +257,38 @@ int rp_mlp_train(rp_handle h, int64_t n, const float* x, const float* t, int32_t
     reserve_batch(m, batch);
     m.d_xb.reserve(((size_t)batch + mlp_row_slack()) * nin);
     m.d_tb.reserve((size_t)batch * nout);
-    m.d_idx.reserve(batch);
+    for (int i = 0; i < 2; ++i) {
+      m.h_idx[i].reserve(batch);
+      if (!m.ev[i]) RP_HIP(hipEventCreateWithFlags(&m.ev[i], hipEventDisableTiming));
+    }
+    // The steps are enqueued without waiting for each other; the rows of a step
+    // are drawn while the one before runs.  The losses are read back every
+    // kLossSteps steps.
+    constexpr int kLossSteps = 256;
+    const int nb = launch_output_loss_blocks(batch, nout);
+    std::vector<double> lp((size_t)std::min(steps, kLossSteps) * nb);
+    m.d_loss.reserve(lp.size());
     std::mt19937_64 g(seed);
-    std::vector<int> idx(batch);
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+    to_bf16(m, s);
     for (int st = 0; st < steps; ++st) {
+      int* idx = m.h_idx[st & 1].p;
+      if (st >= 2) RP_HIP(hipEventSynchronize(m.ev[st & 1]));  // the gather of step st - 2 is done
       for (int j = 0; j < batch; ++j) idx[j] = (int)(g() % (uint64_t)n);
-      RP_HIP(hipMemcpyAsync(m.d_idx.p, idx.data(), sizeof(int) * batch, hipMemcpyHostToDevice, s));
-      launch_gather_rows(m.d_x.p, m.d_t.p, m.d_idx.p, batch, nin, nout, m.d_xb.p, m.d_tb.p, s);
-      to_bf16(m, s);
-      forward(m, m.d_xb.p, batch, true, s);
-      const double l = backward(m, m.d_xb.p, m.d_tb.p, batch, s);  // synchronizes: idx may be refilled
+      launch_gather_rows(m.d_x.p, m.d_t.p, idx, batch, nin, nout, m.d_xb.p, m.d_tb.p, s);
+      RP_HIP(hipEventRecord(m.ev[st & 1], s));
       ++m.step;
       const double c1 = 1.0 - std::pow((double)b1, (double)m.step);
       const double c2 = 1.0 / (1.0 - std::pow((double)b2, (double)m.step));
-      launch_adam(m.d_p.p, m.d_g.p, m.d_m1.p, m.d_m2.p, m.nparams, (float)(lr / c1), b1, b2, (float)c2, eps, s);
-      if (losses) losses[st] = l;
+      const Adam adam{(float)(lr / c1), b1, b2, (float)c2, eps};
+      const int k = st % kLossSteps;
+      step_all(m, m.d_xb.p, m.d_tb.p, batch, m.d_loss.p + (size_t)k * nb, &adam, s);
+      if (losses && (k + 1 == kLossSteps || st + 1 == steps)) {
+        RP_HIP(hipMemcpyAsync(lp.data(), m.d_loss.p, sizeof(double) * nb * (k + 1), hipMemcpyDeviceToHost, s));
+        RP_HIP(hipStreamSynchronize(s));
+        for (int i = 0; i <= k; ++i)
+          losses[st - k + i] = loss_of(lp.data() + (size_t)i * nb, nb, (size_t)batch * nout);
+      }
     }
     RP_HIP(hipStreamSynchronize(s));
   });

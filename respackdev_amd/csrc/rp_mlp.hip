@@ -57,6 +57,24 @@ __global__ void k_to_bf16(const float* __restrict__ src, size_t n, unsigned shor
 // allocated for them), their results are not stored.
 constexpr int kRowsS = 8;  // samples per wave
 template <int K>
+__device__ __forceinline__ void rows_loop(const float* __restrict__ row,
+                                          const unsigned (*sw)[kMaxIn + 1], int cl,
+                                          float (&acc)[kRowsS]) {
+#pragma unroll 1
+  for (int j = 0; j < K; j += K < 8 ? K : 8) {
+#pragma unroll
+    for (int e = 0; e < (K < 8 ? K : 8); e += 2) {
+      const unsigned u = sw[(j + e) / 2][cl];
+      const float w0 = __builtin_bit_cast(float, u << 16);
+      const float w1 = __builtin_bit_cast(float, u & 0xffff0000u);
+#pragma unroll
+      for (int s = 0; s < kRowsS; ++s)
+        acc[s] = fmaf(row[s * K + j + e + 1], w1, fmaf(row[s * K + j + e], w0, acc[s]));
+    }
+  }
+}
+
+template <int K>
 __global__ void __launch_bounds__(256) k_rows_fwd(const float* __restrict__ in, int n,
                                                   const unsigned short* __restrict__ W,
                                                   const float* __restrict__ b, int cols,
@@ -81,19 +99,7 @@ __global__ void __launch_bounds__(256) k_rows_fwd(const float* __restrict__ in, 
     float acc[kRowsS];
 #pragma unroll
     for (int s = 0; s < kRowsS; ++s) acc[s] = bias;
-    const float* row = in + (size_t)r0 * K;
-#pragma unroll 1
-    for (int j = 0; j < K; j += 8) {
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        const unsigned u = sw[(j + e) / 2][cl];
-        const float w0 = __builtin_bit_cast(float, u << 16);
-        const float w1 = __builtin_bit_cast(float, u & 0xffff0000u);
-#pragma unroll
-        for (int s = 0; s < kRowsS; ++s)
-          acc[s] = fmaf(row[s * K + j + e + 1], w1, fmaf(row[s * K + j + e], w0, acc[s]));
-      }
-    }
+    rows_loop<K>(in + (size_t)r0 * K, sw, cl, acc);
     if (c < cols) {
 #pragma unroll
       for (int s = 0; s < kRowsS; ++s) {
@@ -107,15 +113,19 @@ __global__ void __launch_bounds__(256) k_rows_fwd(const float* __restrict__ in, 
 }
 
 // Narrow outputs (fewer than 16: the last layer): a thread per sample, W uniform
-// over the wave; nin a multiple of 4.  The same sums as k_linear_fwd.
+// over the wave; nin a multiple of 4.  The same sums as k_linear_fwd.  With
+// targets T also the mean-squared error, as k_mse: dY = 2 (Y - T) scale and the
+// block's loss sum.
 __global__ void __launch_bounds__(64) k_narrow_fwd(const float* __restrict__ in, int n, int nin,
                                                    const unsigned short* __restrict__ W,
                                                    const float* __restrict__ b, int nout, int act,
-                                                   float* __restrict__ Z, float* __restrict__ Aout) {
+                                                   float* __restrict__ Z, float* __restrict__ Aout,
+                                                   const float* __restrict__ T, float scale,
+                                                   float* __restrict__ dY, double* __restrict__ lossp) {
   const int r = blockIdx.x * 64 + threadIdx.x;
-  if (r >= n) return;
-  const float4* row = (const float4*)(in + (size_t)r * nin);
-  for (int o = 0; o < nout; ++o) {
+  const float4* row = (const float4*)(in + (size_t)(r < n ? r : 0) * nin);
+  double loss = 0.0;
+  for (int o = 0; o < nout && r < n; ++o) {
     const unsigned short* w = W + (size_t)o * nin;
     float acc = b[o];
 #pragma unroll 8
@@ -129,6 +139,15 @@ __global__ void __launch_bounds__(64) k_narrow_fwd(const float* __restrict__ in,
     const size_t idx = (size_t)r * nout + o;
     if (Z) Z[idx] = acc;
     if (act) Aout[idx] = gelu(acc);
+    if (T) {
+      const float d = acc - T[idx];
+      dY[idx] = 2.0f * d * scale;
+      loss += (double)d * d;
+    }
+  }
+  if (T) {  // uniform
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+    if (threadIdx.x == 0) lossp[blockIdx.x] = loss;
   }
 }
 
@@ -179,32 +198,167 @@ __global__ void __launch_bounds__(256) k_linear_bwd_data(const float* __restrict
   }
 }
 
-// Partial weight and bias gradients over one chunk of kChunk samples:
-// part[c][o][i] = sum_{n in chunk} dZ[n][o] A[n][i], part[c][o][nin] = sum dZ[n][o].
-// grid (nchunks, nout); block 256 (threads i <= nin work).
-__global__ void __launch_bounds__(256) k_linear_bwd_w(const float* __restrict__ dZ, const float* __restrict__ A,
-                                                     int n, int nin, int nout, float* __restrict__ part) {
-  const int c = blockIdx.x, o = blockIdx.y, i = threadIdx.x;
-  if (i > nin) return;
-  const int s0 = c * kChunk, s1 = min(n, s0 + kChunk);
-  float acc = 0.0f;
-  for (int s = s0; s < s1; ++s) {
-    const float d = dZ[(size_t)s * nout + o];
-    acc = fmaf(d, i < nin ? A[(size_t)s * nin + i] : 1.0f, acc);
-  }
-  part[((size_t)c * nout + o) * (nin + 1) + i] = acc;
+// Partial weight and bias gradients over chunks of kChunk samples:
+//   part[c][o][i] = sum_{n in chunk} dZ[n][o] A[n][i], part[c][o][nin] = sum dZ[n][o].
+// A wave is one job of a chunk: the wider side of the layer along its lanes, kWg
+// of the other side as uniform (scalar) loads, so that a sample costs one
+// coalesced vector load, one scalar load and kWg FMAs; 16 samples' loads are in
+// flight at a time.  Sums run over the samples in order (the bits of a loop over
+// one output).  Jobs per chunk: lane groups x uniform groups, then the biases.
+constexpr int kWg = 4;
+__host__ __device__ inline bool bwd_w_lanes_in(int nin, int nout) { return nin >= nout; }
+__host__ __device__ inline int bwd_w_jobs(int nin, int nout) {
+  const int l = bwd_w_lanes_in(nin, nout) ? nin : nout, u = bwd_w_lanes_in(nin, nout) ? nout : nin;
+  return ((l + 63) / 64) * ((u + kWg - 1) / kWg) + (nout + 63) / 64;
 }
 
-// grad W[o][i] (and b[o] at i == nin) = sum over chunks, in chunk order.
-__global__ void k_reduce_w(const float* __restrict__ part, int nchunks, int nin, int nout,
-                           float* __restrict__ gW, float* __restrict__ gb) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= nout * (nin + 1)) return;
-  float acc = 0.0f;
-  for (int c = 0; c < nchunks; ++c) acc += part[(size_t)c * nout * (nin + 1) + idx];
-  const int o = idx / (nin + 1), i = idx % (nin + 1);
-  if (i < nin) gW[(size_t)o * nin + i] = acc;
-  else gb[o] = acc;
+__device__ __forceinline__ void bwd_w_job(const float* __restrict__ dZ, const float* __restrict__ A,
+                                          int n, int nin, int nout, int job, int lane,
+                                          float* __restrict__ part) {
+  const int per = bwd_w_jobs(nin, nout);
+  const int c = job / per, k = job % per;
+  const int s0 = c * kChunk, s1 = min(n, s0 + kChunk);
+  float* out = part + (size_t)c * nout * (nin + 1);
+  const bool li = bwd_w_lanes_in(nin, nout);
+  const int L = li ? nin : nout, U = li ? nout : nin;
+  const int lw = (L + 63) / 64, nug = (U + kWg - 1) / kWg;
+  if (k >= lw * nug) {  // biases
+    const int o = (k - lw * nug) * 64 + lane, ol = o < nout ? o : nout - 1;
+    float acc = 0.0f;
+#pragma unroll 16
+    for (int s = s0; s < s1; ++s) acc += dZ[(size_t)s * nout + ol];
+    if (o < nout) out[(size_t)o * (nin + 1) + nin] = acc;
+    return;
+  }
+  const int l = (k % lw) * 64 + lane, ll = l < L ? l : L - 1, u0 = k / lw * kWg;
+  const float* ls = (li ? A : dZ) + ll;
+  const float* us = (li ? dZ : A) + u0;
+  float acc[kWg];
+#pragma unroll
+  for (int g = 0; g < kWg; ++g) acc[g] = 0.0f;
+  int s = s0;
+  if (u0 + kWg <= U) {
+#pragma unroll 1
+    for (; s + 16 <= s1; s += 16) {
+      float lv[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) lv[e] = ls[(size_t)(s + e) * L];
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int g = 0; g < kWg; ++g) acc[g] = fmaf(us[(size_t)(s + e) * U + g], lv[e], acc[g]);
+    }
+  }
+#pragma unroll 4
+  for (; s < s1; ++s) {
+    const float lv = ls[(size_t)s * L];
+#pragma unroll
+    for (int g = 0; g < kWg; ++g)
+      acc[g] = fmaf(us[(size_t)s * U + (u0 + g < U ? g : 0)], lv, acc[g]);
+  }
+  if (l >= L) return;
+#pragma unroll
+  for (int g = 0; g < kWg; ++g) {
+    const int u = u0 + g;
+    if (u < U) out[li ? (size_t)u * (nin + 1) + l : (size_t)l * (nin + 1) + u] = acc[g];
+  }
+}
+
+// Jobs [0, njobs), four waves per block.
+__global__ void __launch_bounds__(256) k_bwd_w(const float* __restrict__ dZ, const float* __restrict__ A,
+                                               int n, int nin, int nout, int njobs,
+                                               float* __restrict__ part) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int job = (int)blockIdx.x * 4 + wave;
+  if (job < njobs) bwd_w_job(dZ, A, n, nin, nout, job, threadIdx.x & 63, part);
+}
+
+// The backward step of one layer in one launch: blocks [0, ndata) form
+// dA = dZ W (times gelu'(Zprev)) as k_rows_fwd does (lane = input i, W[o][i] as
+// pairs over o, K = nout), the others the weight gradient's jobs; both need dZ
+// alone.  dZ is readable up to a multiple of kRowsS past n.
+template <int K>
+__global__ void __launch_bounds__(256) k_bwd(const float* __restrict__ dZ, const float* __restrict__ A,
+                                             const unsigned short* __restrict__ W,
+                                             const float* __restrict__ Zprev, int n, int nin, int ndata,
+                                             int njobs, float* __restrict__ dA, float* __restrict__ part) {
+  __shared__ unsigned sw[K / 2][kMaxIn + 1];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  if ((int)blockIdx.x >= ndata) {
+    const int job = ((int)blockIdx.x - ndata) * 4 + wave;
+    if (job < njobs) bwd_w_job(dZ, A, n, nin, K, job, lane, part);
+    return;
+  }
+  for (int e = threadIdx.x; e < (K / 2) * nin; e += 256) {
+    const int o2 = e / nin, i = e % nin;
+    sw[o2][i] = (unsigned)W[(size_t)2 * o2 * nin + i] | ((unsigned)W[(size_t)(2 * o2 + 1) * nin + i] << 16);
+  }
+  __syncthreads();
+  const int cw = (nin + 63) / 64;
+  const int c = (wave % cw) * 64 + lane, cl = c < nin ? c : nin - 1;
+  const int step = ndata * (4 / cw) * kRowsS;
+  for (int r0 = ((int)blockIdx.x * (4 / cw) + wave / cw) * kRowsS; r0 < n; r0 += step) {
+    float acc[kRowsS];
+#pragma unroll
+    for (int s = 0; s < kRowsS; ++s) acc[s] = 0.0f;
+    rows_loop<K>(dZ + (size_t)r0 * K, sw, cl, acc);
+    if (c < nin) {
+#pragma unroll
+      for (int s = 0; s < kRowsS; ++s) {
+        if (r0 + s >= n) break;
+        const size_t idx = (size_t)(r0 + s) * nin + c;
+        dA[idx] = acc[s] * gelu_grad(Zprev[idx]);
+      }
+    }
+  }
+}
+
+// Per parameter of the layers in t: the gradient from the partials (in chunk
+// order) when part is set, an Adam step (bias-corrected: lr_t = lr / (1 - b1^t),
+// c2 = 1 / (1 - b2^t)) with the new BF16 copy when m1 is set.
+struct MlpLayers {
+  int n;
+  int nin[8], nout[8];
+  size_t off[8], part[8];  // W_l in the parameters (b_l follows it), its partials
+};
+__global__ void __launch_bounds__(256) k_finish(MlpLayers t, const float* __restrict__ part, int nchunks,
+                                                float* __restrict__ g, float* __restrict__ p,
+                                                unsigned short* __restrict__ pb, float* __restrict__ m1,
+                                                float* __restrict__ m2, float lr_t, float b1, float b2,
+                                                float c2, float eps) {
+  size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+  int l = 0;
+  for (; l < t.n; ++l) {
+    const size_t m = (size_t)t.nout[l] * (t.nin[l] + 1);
+    if (e < m) break;
+    e -= m;
+  }
+  if (l == t.n) return;
+  const int nin = t.nin[l], nout = t.nout[l];
+  const size_t per = (size_t)nout * (nin + 1), nw = (size_t)nout * nin;
+  const size_t idx = t.off[l] + e;
+  float gi;
+  if (part) {
+    // partial of W[o][i] at o (nin + 1) + i, of b[o] at o (nin + 1) + nin
+    const size_t at = e < nw ? e / nin * (nin + 1) + e % nin : (e - nw) * (nin + 1) + nin;
+    const float* src = part + t.part[l] + at;
+    float acc = 0.0f;
+#pragma unroll 16
+    for (int c = 0; c < nchunks; ++c) acc += src[(size_t)c * per];
+    g[idx] = gi = acc;
+  } else {
+    gi = g[idx];
+  }
+  if (m1) {
+    const float a = b1 * m1[idx] + (1.0f - b1) * gi;
+    const float v = b2 * m2[idx] + (1.0f - b2) * gi * gi;
+    m1[idx] = a;
+    m2[idx] = v;
+    const float pn = p[idx] - lr_t * a / (sqrtf(v * c2) + eps);
+    p[idx] = pn;
+    pb[idx] = __builtin_bit_cast(unsigned short, (__bf16)pn);
+  }
 }
 
 // Mean-squared error: dY = 2 (Y - T) / (n * nout); loss partial sums per block.
@@ -226,27 +380,20 @@ __global__ void __launch_bounds__(256) k_mse(const float* __restrict__ Y, const 
   if (threadIdx.x == 0) lossp[blockIdx.x] = red[0];
 }
 
-// Adam on FP32 masters (bias-corrected step sizes a1 = lr / (1 - b1^t), a2 = 1 / (1 - b2^t)).
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m1,
-                       float* __restrict__ m2, size_t n, float lr_t, float b1, float b2, float c2, float eps) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-    const float gi = g[i];
-    const float a = b1 * m1[i] + (1.0f - b1) * gi;
-    const float v = b2 * m2[i] + (1.0f - b2) * gi * gi;
-    m1[i] = a;
-    m2[i] = v;
-    p[i] -= lr_t * a / (sqrtf(v * c2) + eps);
-  }
-}
-
-// Gathers a minibatch: xb[j] = x[idx[j]], tb[j] = t[idx[j]].
-__global__ void k_gather_rows(const float* __restrict__ x, const float* __restrict__ t, const int* __restrict__ idx,
-                              int nb, int nin, int nout, float* __restrict__ xb, float* __restrict__ tb) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
+// Gathers a minibatch: xb[j] = x[idx[j]], tb[j] = t[idx[j]], a thread per value.
+// idx may be pinned host memory (each entry is then read over the bus).
+__global__ void __launch_bounds__(256) k_gather_rows(const float* __restrict__ x,
+                                                     const float* __restrict__ t,
+                                                     const int* __restrict__ idx, int nb, int nin,
+                                                     int nout, float* __restrict__ xb,
+                                                     float* __restrict__ tb) {
+  const int w = nin + nout;
+  const long long e = blockIdx.x * 256LL + threadIdx.x;
+  const int j = (int)(e / w), i = (int)(e % w);
   if (j >= nb) return;
   const size_t r = (size_t)idx[j];
-  for (int i = 0; i < nin; ++i) xb[(size_t)j * nin + i] = x[r * nin + i];
-  for (int o = 0; o < nout; ++o) tb[(size_t)j * nout + o] = t[r * nout + o];
+  if (i < nin) xb[(size_t)j * nin + i] = x[r * nin + i];
+  else tb[(size_t)j * nout + i - nin] = t[r * nout + i - nin];
 }
 
 int mlp_max_width() { return kMaxIn; }
@@ -278,7 +425,7 @@ void launch_linear_fwd(const float* A, int n, int nin, const unsigned short* W, 
   else if (wide && nin == 8) RP_ROWS(8);
   else if (nout < 16 && nin % 4 == 0 && al)
     hipLaunchKernelGGL(k_narrow_fwd, dim3((n + 63) / 64), dim3(64), 0, s, A, n, nin, W, b, nout, act, Z,
-                       Aout);
+                       Aout, (const float*)nullptr, 0.0f, (float*)nullptr, (double*)nullptr);
   else
     hipLaunchKernelGGL(k_linear_fwd, dim3((n + kRows - 1) / kRows), dim3(256), 0, s, A, n, nin, W, b, nout,
                        act, Z, Aout);
@@ -286,41 +433,80 @@ void launch_linear_fwd(const float* A, int n, int nin, const unsigned short* W, 
   RP_HIP(hipGetLastError());
 }
 
-void launch_linear_bwd_data(const float* dZ, int n, int nout, const unsigned short* W, int nin,
-                            const float* Zprev, int act, float* dA, hipStream_t s) {
+// The output layer with the mean-squared error: Y, dY and the loss partials
+// (nlossp of them at most: launch_output_loss_blocks).
+int launch_output_loss_blocks(int n, int nout) {
+  return nout < 16 ? (n + 63) / 64 : (int)std::min<size_t>(((size_t)n * nout + 255) / 256, 1024);
+}
+void launch_output_loss(const float* A, int n, int nin, const unsigned short* W, const float* b, int nout,
+                        const float* T, float scale, float* Y, float* dY, double* lossp, hipStream_t s) {
+  const int nlossp = launch_output_loss_blocks(n, nout);
+  const bool al = ((uintptr_t)W % 16) == 0 && ((uintptr_t)A % 16) == 0;
+  if (nout < 16 && nin % 4 == 0 && al) {
+    hipLaunchKernelGGL(k_narrow_fwd, dim3(nlossp), dim3(64), 0, s, A, n, nin, W, b, nout, 0, Y,
+                       (float*)nullptr, T, scale, dY, lossp);
+  } else {
+    launch_linear_fwd(A, n, nin, W, b, nout, 0, Y, nullptr, s);
+    hipLaunchKernelGGL(k_mse, dim3(nlossp), dim3(256), 0, s, Y, T, (size_t)n * nout, scale, dY, lossp);
+  }
+  RP_HIP(hipGetLastError());
+}
+
+// Backward step of one layer: the weight-gradient partials, and with dA also
+// dA = dZ W gelu'(Zprev).
+void launch_bwd_layer(const float* dZ, const float* A, int n, int nin, int nout, const unsigned short* W,
+                      const float* Zprev, float* dA, float* part, hipStream_t s) {
   RP_CHECK(nin <= kMaxIn && nout <= kMaxIn && n > 0, "MLP layer wider than 128 or empty batch");
-  hipLaunchKernelGGL(k_linear_bwd_data, dim3((n + kRows - 1) / kRows), dim3(256), 0, s, dZ, n, nout, W, nin,
-                     Zprev, act, dA);
+  const int nchunks = (n + kChunk - 1) / kChunk, njobs = nchunks * bwd_w_jobs(nin, nout);
+  const int nw = (njobs + 3) / 4;
+  const int per = kRowsS * (nin > 64 ? 2 : 4);
+  const int nd = std::min((n + per - 1) / per, 2048);
+#define RP_BWD(KK)                                                                                   \
+  case KK:                                                                                           \
+    hipLaunchKernelGGL(k_bwd<KK>, dim3(nd + nw), dim3(256), 0, s, dZ, A, W, Zprev, n, nin, nd, njobs, \
+                       dA, part);                                                                    \
+    break;
+  if (!dA) {
+    hipLaunchKernelGGL(k_bwd_w, dim3(nw), dim3(256), 0, s, dZ, A, n, nin, nout, njobs, part);
+  } else {
+    switch (nout) {
+      RP_BWD(2) RP_BWD(8) RP_BWD(16) RP_BWD(32) RP_BWD(64) RP_BWD(128)
+      default:
+        hipLaunchKernelGGL(k_bwd_w, dim3(nw), dim3(256), 0, s, dZ, A, n, nin, nout, njobs, part);
+        hipLaunchKernelGGL(k_linear_bwd_data, dim3((n + kRows - 1) / kRows), dim3(256), 0, s, dZ, n, nout,
+                           W, nin, Zprev, 1, dA);
+    }
+  }
+#undef RP_BWD
   RP_HIP(hipGetLastError());
 }
 
-void launch_linear_bwd_w(const float* dZ, const float* A, int n, int nin, int nout, float* part, float* gW,
-                         float* gb, hipStream_t s) {
-  RP_CHECK(nin <= kMaxIn && nout <= kMaxIn && n > 0, "MLP layer wider than 128 or empty batch");
-  const int nchunks = (n + kChunk - 1) / kChunk;
-  hipLaunchKernelGGL(k_linear_bwd_w, dim3(nchunks, nout), dim3(256), 0, s, dZ, A, n, nin, nout, part);
-  RP_HIP(hipGetLastError());
-  const int m = nout * (nin + 1);
-  hipLaunchKernelGGL(k_reduce_w, dim3((m + 255) / 256), dim3(256), 0, s, part, nchunks, nin, nout, gW, gb);
-  RP_HIP(hipGetLastError());
-}
-
-void launch_mse(const float* Y, const float* T, size_t m, float scale, float* dY, double* lossp, int nblocks,
-                hipStream_t s) {
-  hipLaunchKernelGGL(k_mse, dim3(nblocks), dim3(256), 0, s, Y, T, m, scale, dY, lossp);
-  RP_HIP(hipGetLastError());
-}
-
-void launch_adam(float* p, const float* g, float* m1, float* m2, size_t n, float lr_t, float b1, float b2,
-                 float c2, float eps, hipStream_t s) {
-  const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 4096);
-  hipLaunchKernelGGL(k_adam, dim3(blocks), dim3(256), 0, s, p, g, m1, m2, n, lr_t, b1, b2, c2, eps);
+// Layers [l0, l1) (dims[l0 ..], W_l at woff[l]): gradients from part (unless
+// null; layer l's partials at poff[l - l0]) and, with m1, an Adam step.
+void launch_finish(int l0, int l1, const int* dims, const size_t* woff, const size_t* poff,
+                   const float* part, int nchunks, float* g, float* p, unsigned short* pb, float* m1,
+                   float* m2, float lr_t, float b1, float b2, float c2, float eps, hipStream_t s) {
+  for (int a = l0; a < l1; a += 8) {
+    MlpLayers t;
+    t.n = std::min(8, l1 - a);
+    size_t tot = 0;
+    for (int i = 0; i < t.n; ++i) {
+      t.nin[i] = dims[a + i];
+      t.nout[i] = dims[a + i + 1];
+      t.off[i] = woff[a + i];
+      t.part[i] = part ? poff[a + i - l0] : 0;
+      tot += (size_t)t.nout[i] * (t.nin[i] + 1);
+    }
+    hipLaunchKernelGGL(k_finish, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, t, part, nchunks, g,
+                       p, pb, m1, m2, lr_t, b1, b2, c2, eps);
+  }
   RP_HIP(hipGetLastError());
 }
 
 void launch_gather_rows(const float* x, const float* t, const int* idx, int nb, int nin, int nout, float* xb,
                         float* tb, hipStream_t s) {
-  hipLaunchKernelGGL(k_gather_rows, dim3((nb + 255) / 256), dim3(256), 0, s, x, t, idx, nb, nin, nout, xb, tb);
+  const long long m = (long long)nb * (nin + nout);
+  hipLaunchKernelGGL(k_gather_rows, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, x, t, idx, nb, nin, nout, xb, tb);
   RP_HIP(hipGetLastError());
 }
 

@@ -19,9 +19,14 @@ struct Mlp {
   DevBuf<float> d_z, d_a;              // pre-activations / activations, per layer [n][width]
   DevBuf<float> d_dz0, d_dz1, d_part;  // gradient work buffers
   DevBuf<float> d_x, d_t, d_xb, d_tb;  // data (resident for training) and minibatch
-  DevBuf<int> d_idx;
-  DevBuf<double> d_loss;
+  HostBuf<int> h_idx[2];               // minibatch rows of two steps (pinned, read by the gather)
+  hipEvent_t ev[2] = {};               // the gathers that read them
+  DevBuf<double> d_loss;               // loss partials of every step
   std::vector<size_t> aoff;            // offsets of layer l's [n][width] in d_z / d_a
+  ~Mlp() {
+    for (auto& e : ev)
+      if (e) (void)hipEventDestroy(e);
+  }
 };
 
 }  // namespace rp
