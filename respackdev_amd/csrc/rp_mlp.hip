@@ -50,36 +50,55 @@ __global__ void k_to_bf16(const float* __restrict__ src, size_t n, unsigned shor
 // over the inputs stays rolled: unrolled, the compiler issues every scalar load
 // at its start and spills.  Each output sums b + a_0 w_0 + a_1 w_1 + ... in that
 // order, as k_linear_fwd does: the same bits.  Bound by the FP32 FMAs and the
-// scalar loads' latency: 60000 samples of 128 -> 128 take 57 us (35 TFLOP/s), and
-// a forward pass of 300011 samples 1.31 ms with its copies, against 3.03 ms when
+// scalar loads' latency: 60000 samples of 128 -> 128 take 47 us (42 TFLOP/s), and
+// a forward pass of 300011 samples 1.23 ms with its copies, against 3.03 ms when
 // every layer ran k_linear_fwd (W read uncoalesced, once per sample).  Z, A:
 // pre-activation and gelu(Z), each optional.  Rows up to a multiple of kRowsS past n are read (in is
 // allocated for them), their results are not stored.
-constexpr int kRowsS = 8;  // samples per wave
-template <int K>
+constexpr int kRowsS = 8;     // samples per wave at most
+// Batches from here on take 8 samples per wave; smaller ones 4, which gives the
+// scalar loads' latency two waves per SIMD at 4096 samples (a 128 -> 128 layer
+// 13.1 us with 8, 9.4 us with 4 and rows_touch).
+constexpr int kRowsBig = 16384;
+template <int K, int S>
 __device__ __forceinline__ void rows_loop(const float* __restrict__ row,
                                           const unsigned (*sw)[kMaxIn + 1], int cl,
-                                          float (&acc)[kRowsS]) {
+                                          float (&acc)[S]) {
+  constexpr int CH = K < 64 / S ? K : 64 / S;  // inputs per pass: 64 scalar registers
 #pragma unroll 1
-  for (int j = 0; j < K; j += K < 8 ? K : 8) {
+  for (int j = 0; j < K; j += CH) {
 #pragma unroll
-    for (int e = 0; e < (K < 8 ? K : 8); e += 2) {
+    for (int e = 0; e < CH; e += 2) {
       const unsigned u = sw[(j + e) / 2][cl];
       const float w0 = __builtin_bit_cast(float, u << 16);
       const float w1 = __builtin_bit_cast(float, u & 0xffff0000u);
 #pragma unroll
-      for (int s = 0; s < kRowsS; ++s)
+      for (int s = 0; s < S; ++s)
         acc[s] = fmaf(row[s * K + j + e + 1], w1, fmaf(row[s * K + j + e], w0, acc[s]));
     }
   }
 }
 
-template <int K>
+// One load of every 64-byte line of S rows of K floats, so that the scalar loads
+// that follow find them in this XCD's L2 (the rows come from other XCDs).
+template <int K, int S>
+__device__ __forceinline__ void rows_touch(const float* __restrict__ row, int lane) {
+  constexpr int lines = (S * K + 15) / 16;
+  const float v = row[16 * (lane < lines ? lane : 0)];
+  asm volatile("" ::"v"(v));
+}
+
+template <int K, int S>
 __global__ void __launch_bounds__(256) k_rows_fwd(const float* __restrict__ in, int n,
                                                   const unsigned short* __restrict__ W,
                                                   const float* __restrict__ b, int cols,
                                                   float* __restrict__ Z, float* __restrict__ Aout) {
   __shared__ unsigned sw[K / 2][kMaxIn + 1];  // + 1: the staging writes fall on different banks
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int cw = (cols + 63) / 64;  // 1 or 2
+  int r0 = ((int)blockIdx.x * (4 / cw) + wave / cw) * S;
+  if (r0 < n) rows_touch<K, S>(in + (size_t)r0 * K, lane);
   for (int e = threadIdx.x; e < cols * (K / 8); e += 256) {
     const int c = e / (K / 8), j = e % (K / 8);
     const uint4 v = ((const uint4*)W)[e];
@@ -89,20 +108,18 @@ __global__ void __launch_bounds__(256) k_rows_fwd(const float* __restrict__ in, 
     sw[4 * j + 3][c] = v.w;
   }
   __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int cw = (cols + 63) / 64;  // 1 or 2
   const int c = (wave % cw) * 64 + lane, cl = c < cols ? c : cols - 1;
   const float bias = b[cl];
-  const int step = (int)gridDim.x * (4 / cw) * kRowsS;
-  for (int r0 = ((int)blockIdx.x * (4 / cw) + wave / cw) * kRowsS; r0 < n; r0 += step) {
-    float acc[kRowsS];
+  const int step = (int)gridDim.x * (4 / cw) * S;
+  for (; r0 < n; r0 += step) {
+    if (r0 + step < n) rows_touch<K, S>(in + (size_t)(r0 + step) * K, lane);
+    float acc[S];
 #pragma unroll
-    for (int s = 0; s < kRowsS; ++s) acc[s] = bias;
-    rows_loop<K>(in + (size_t)r0 * K, sw, cl, acc);
+    for (int s = 0; s < S; ++s) acc[s] = bias;
+    rows_loop<K, S>(in + (size_t)r0 * K, sw, cl, acc);
     if (c < cols) {
 #pragma unroll
-      for (int s = 0; s < kRowsS; ++s) {
+      for (int s = 0; s < S; ++s) {
         if (r0 + s >= n) break;
         const size_t idx = (size_t)(r0 + s) * cols + c;
         if (Z) Z[idx] = acc[s];
@@ -200,115 +217,189 @@ __global__ void __launch_bounds__(256) k_linear_bwd_data(const float* __restrict
 
 // Partial weight and bias gradients over chunks of kChunk samples:
 //   part[c][o][i] = sum_{n in chunk} dZ[n][o] A[n][i], part[c][o][nin] = sum dZ[n][o].
-// A wave is one job of a chunk: the wider side of the layer along its lanes, kWg
-// of the other side as uniform (scalar) loads, so that a sample costs one
-// coalesced vector load, one scalar load and kWg FMAs; 16 samples' loads are in
-// flight at a time.  Sums run over the samples in order (the bits of a loop over
-// one output).  Jobs per chunk: lane groups x uniform groups, then the biases.
-constexpr int kWg = 4;
-__host__ __device__ inline bool bwd_w_lanes_in(int nin, int nout) { return nin >= nout; }
-__host__ __device__ inline int bwd_w_jobs(int nin, int nout) {
-  const int l = bwd_w_lanes_in(nin, nout) ? nin : nout, u = bwd_w_lanes_in(nin, nout) ? nout : nin;
-  return ((l + 63) / 64) * ((u + kWg - 1) / kWg) + (nout + 63) / 64;
+// A workgroup is one job of a chunk: 64 of the wider side of the layer along its
+// lanes by 16 of the other.  Half a chunk of both sides sits in LDS (40 KB, so
+// that three workgroups share a CU) with the other half's loads in flight: the
+// operands come from other XCDs, about a microsecond away, and a loop that loads
+// 16 samples at a time spent 16 such latencies on the chunk (a backward launch of a 128 -> 128 layer at 4096
+// samples: 24.8 us then, 20.1 us now; the last layer's 26.7 and 11.2 us; 26.8 us
+// with whole chunks in 80 KB).  Each wave takes four of the 16; per sample one LDS read along the lanes, one broadcast and four
+// FMAs.  Sums run over the samples in order (the bits of a loop over one output).
+constexpr int kWu = 16;
+struct BwdW {
+  int L, U, lw, nu;  // wider and other side, lane groups, groups of kWu
+  bool in;           // the lanes run along the inputs
+};
+__host__ __device__ inline BwdW bwd_w_shape(int nin, int nout) {
+  BwdW b;
+  b.in = nin >= nout;
+  b.L = b.in ? nin : nout;
+  b.U = b.in ? nout : nin;
+  b.lw = (b.L + 63) / 64;
+  b.nu = (b.U + kWu - 1) / kWu;
+  return b;
 }
+constexpr int kWs = 128;  // samples of a chunk in LDS at a time
+constexpr size_t kBwdWLds = sizeof(float) * kWs * (64 + kWu);
 
-__device__ __forceinline__ void bwd_w_job(const float* __restrict__ dZ, const float* __restrict__ A,
-                                          int n, int nin, int nout, int job, int lane,
-                                          float* __restrict__ part) {
-  const int per = bwd_w_jobs(nin, nout);
-  const int c = job / per, k = job % per;
-  const int s0 = c * kChunk, s1 = min(n, s0 + kChunk);
-  float* out = part + (size_t)c * nout * (nin + 1);
-  const bool li = bwd_w_lanes_in(nin, nout);
-  const int L = li ? nin : nout, U = li ? nout : nin;
-  const int lw = (L + 63) / 64, nug = (U + kWg - 1) / kWg;
-  if (k >= lw * nug) {  // biases
-    const int o = (k - lw * nug) * 64 + lane, ol = o < nout ? o : nout - 1;
-    float acc = 0.0f;
-#pragma unroll 16
-    for (int s = s0; s < s1; ++s) acc += dZ[(size_t)s * nout + ol];
-    if (o < nout) out[(size_t)o * (nin + 1) + nin] = acc;
-    return;
-  }
-  const int l = (k % lw) * 64 + lane, ll = l < L ? l : L - 1, u0 = k / lw * kWg;
-  const float* ls = (li ? A : dZ) + ll;
-  const float* us = (li ? dZ : A) + u0;
-  float acc[kWg];
+// kWs rows of src[.][ld] from row s0 on (zero from ns on), columns c0 .. c0 + W
+// (zero past ld): into registers, then to dst[kWs][W].  al: 16-byte loads.
+template <int W>
+struct StageCols {
+  float4 v[kWs * W / 1024];
+  __device__ __forceinline__ void load(const float* __restrict__ src, int ld, int c0, int s0, int ns,
+                                       bool al) {
 #pragma unroll
-  for (int g = 0; g < kWg; ++g) acc[g] = 0.0f;
-  int s = s0;
-  if (u0 + kWg <= U) {
-#pragma unroll 1
-    for (; s + 16 <= s1; s += 16) {
-      float lv[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) lv[e] = ls[(size_t)(s + e) * L];
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-#pragma unroll
-        for (int g = 0; g < kWg; ++g) acc[g] = fmaf(us[(size_t)(s + e) * U + g], lv[e], acc[g]);
+    for (int k = 0; k < kWs * W / 1024; ++k) {
+      const int e = (int)threadIdx.x + 256 * k, s = e / (W / 4), c = c0 + 4 * (e % (W / 4));
+      const float* p = src + (size_t)(s0 + s) * ld + c;
+      v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (s < ns && c < ld) {
+        if (al) {
+          v[k] = *(const float4*)p;
+        } else {
+          v[k].x = p[0];
+          if (c + 1 < ld) v[k].y = p[1];
+          if (c + 2 < ld) v[k].z = p[2];
+          if (c + 3 < ld) v[k].w = p[3];
+        }
+      }
     }
   }
-#pragma unroll 4
-  for (; s < s1; ++s) {
-    const float lv = ls[(size_t)s * L];
+  __device__ __forceinline__ void store(float* dst) const {
 #pragma unroll
-    for (int g = 0; g < kWg; ++g)
-      acc[g] = fmaf(us[(size_t)s * U + (u0 + g < U ? g : 0)], lv, acc[g]);
+    for (int k = 0; k < kWs * W / 1024; ++k) ((float4*)dst)[threadIdx.x + 256 * k] = v[k];
   }
-  if (l >= L) return;
+};
+
+__device__ __forceinline__ void bwd_w_job(const float* __restrict__ dZ, const float* __restrict__ A,
+                                          int n, int nin, int nout, int job, float* lds,
+                                          float* __restrict__ part) {
+  const BwdW b = bwd_w_shape(nin, nout);
+  const int per = b.lw * b.nu, c = job / per, k = job % per;
+  const int l0 = (k % b.lw) * 64, u0 = (k / b.lw) * kWu;
+  const int s0 = c * kChunk, ns = min(n - s0, kChunk);
+  float* sl = lds;              // [kWs][64]
+  float* su = lds + kWs * 64;   // [kWs][kWu]
+  const float* L = b.in ? A : dZ;
+  const float* U = b.in ? dZ : A;
+  const bool all = b.L % 4 == 0 && ((uintptr_t)L % 16) == 0;
+  const bool alu = b.U % 4 == 0 && ((uintptr_t)U % 16) == 0;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l = l0 + lane, uw = u0 + 4 * wave;
+  // the biases beside the first lane group (lanes along the inputs), or by the
+  // last wave along the lanes
+  const bool bu = b.in && l0 == 0, bl = !b.in && u0 == 0 && wave == 3;
+  float acc[4] = {0.f, 0.f, 0.f, 0.f}, bias[4] = {0.f, 0.f, 0.f, 0.f};
+  StageCols<64> vl;
+  StageCols<kWu> vu;
+  vl.load(L, b.L, l0, s0, ns, all);
+  vu.load(U, b.U, u0, s0, ns, alu);
+  for (int h = 0; h < ns; h += kWs) {
+    const int m = min(kWs, ns - h);
+    __syncthreads();
+    vl.store(sl);
+    vu.store(su);
+    __syncthreads();
+    if (h + kWs < ns) {  // the rest of the chunk in flight meanwhile
+      vl.load(L, b.L, l0, s0 + h + kWs, ns - h - kWs, all);
+      vu.load(U, b.U, u0, s0 + h + kWs, ns - h - kWs, alu);
+    }
+    if (uw < b.U) {
+      if (bu) {
+#pragma unroll 8
+        for (int s = 0; s < m; ++s) {
+          const float lv = sl[s * 64 + lane];
+          const float4 uv = *(const float4*)(su + s * kWu + 4 * wave);
+          acc[0] = fmaf(uv.x, lv, acc[0]);
+          acc[1] = fmaf(uv.y, lv, acc[1]);
+          acc[2] = fmaf(uv.z, lv, acc[2]);
+          acc[3] = fmaf(uv.w, lv, acc[3]);
+          bias[0] += uv.x;
+          bias[1] += uv.y;
+          bias[2] += uv.z;
+          bias[3] += uv.w;
+        }
+      } else {
+#pragma unroll 8
+        for (int s = 0; s < m; ++s) {
+          const float lv = sl[s * 64 + lane];
+          const float4 uv = *(const float4*)(su + s * kWu + 4 * wave);
+          acc[0] = fmaf(uv.x, lv, acc[0]);
+          acc[1] = fmaf(uv.y, lv, acc[1]);
+          acc[2] = fmaf(uv.z, lv, acc[2]);
+          acc[3] = fmaf(uv.w, lv, acc[3]);
+        }
+      }
+    }
+    if (bl) {
+#pragma unroll 8
+      for (int s = 0; s < m; ++s) bias[0] += sl[s * 64 + lane];
+    }
+  }
+  float* out = part + (size_t)c * nout * (nin + 1);
 #pragma unroll
-  for (int g = 0; g < kWg; ++g) {
-    const int u = u0 + g;
-    if (u < U) out[li ? (size_t)u * (nin + 1) + l : (size_t)l * (nin + 1) + u] = acc[g];
+  for (int g = 0; g < 4; ++g) {
+    const int u = uw + g;
+    if (u >= b.U) break;
+    if (l < b.L) out[b.in ? (size_t)u * (nin + 1) + l : (size_t)l * (nin + 1) + u] = acc[g];
+    if (bu && lane == g) out[(size_t)u * (nin + 1) + nin] = bias[g];
   }
+  if (bl && l < nout) out[(size_t)l * (nin + 1) + nin] = bias[0];
 }
 
-// Jobs [0, njobs), four waves per block.
+// grid: njobs.
 __global__ void __launch_bounds__(256) k_bwd_w(const float* __restrict__ dZ, const float* __restrict__ A,
-                                               int n, int nin, int nout, int njobs,
-                                               float* __restrict__ part) {
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int job = (int)blockIdx.x * 4 + wave;
-  if (job < njobs) bwd_w_job(dZ, A, n, nin, nout, job, threadIdx.x & 63, part);
+                                               int n, int nin, int nout, float* __restrict__ part) {
+  extern __shared__ float4 mlp_lds[];
+  bwd_w_job(dZ, A, n, nin, nout, blockIdx.x, (float*)mlp_lds, part);
 }
 
-// The backward step of one layer in one launch: blocks [0, ndata) form
-// dA = dZ W (times gelu'(Zprev)) as k_rows_fwd does (lane = input i, W[o][i] as
-// pairs over o, K = nout), the others the weight gradient's jobs; both need dZ
-// alone.  dZ is readable up to a multiple of kRowsS past n.
-template <int K>
+// The backward step of one layer in one launch: blocks [0, nw) are the weight
+// gradient's jobs (the longer ones), the others form dA = dZ W (times
+// gelu'(Zprev)) as k_rows_fwd does (lane = input i, W[o][i] as pairs over o,
+// K = nout); both need dZ alone.  dZ is readable up to a multiple of kRowsS past n.
+template <int K, int S>
 __global__ void __launch_bounds__(256) k_bwd(const float* __restrict__ dZ, const float* __restrict__ A,
                                              const unsigned short* __restrict__ W,
-                                             const float* __restrict__ Zprev, int n, int nin, int ndata,
-                                             int njobs, float* __restrict__ dA, float* __restrict__ part) {
-  __shared__ unsigned sw[K / 2][kMaxIn + 1];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  if ((int)blockIdx.x >= ndata) {
-    const int job = ((int)blockIdx.x - ndata) * 4 + wave;
-    if (job < njobs) bwd_w_job(dZ, A, n, nin, K, job, lane, part);
+                                             const float* __restrict__ Zprev, int n, int nin, int nw,
+                                             float* __restrict__ dA, float* __restrict__ part) {
+  extern __shared__ float4 mlp_lds[];
+  if ((int)blockIdx.x < nw) {
+    bwd_w_job(dZ, A, n, nin, K, (int)blockIdx.x, (float*)mlp_lds, part);
     return;
   }
-  for (int e = threadIdx.x; e < (K / 2) * nin; e += 256) {
-    const int o2 = e / nin, i = e % nin;
-    sw[o2][i] = (unsigned)W[(size_t)2 * o2 * nin + i] | ((unsigned)W[(size_t)(2 * o2 + 1) * nin + i] << 16);
-  }
-  __syncthreads();
+  const int block = (int)blockIdx.x - nw, ndata = (int)gridDim.x - nw;
+  unsigned(*sw)[kMaxIn + 1] = (unsigned(*)[kMaxIn + 1]) mlp_lds;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int cw = (nin + 63) / 64;
-  const int c = (wave % cw) * 64 + lane, cl = c < nin ? c : nin - 1;
-  const int step = ndata * (4 / cw) * kRowsS;
-  for (int r0 = ((int)blockIdx.x * (4 / cw) + wave / cw) * kRowsS; r0 < n; r0 += step) {
-    float acc[kRowsS];
+  int r0 = (block * (4 / cw) + wave / cw) * S;
+  if (r0 < n) rows_touch<K, S>(dZ + (size_t)r0 * K, lane);
+  for (int i = lane; i < nin; i += 64)
 #pragma unroll
-    for (int s = 0; s < kRowsS; ++s) acc[s] = 0.0f;
-    rows_loop<K>(dZ + (size_t)r0 * K, sw, cl, acc);
+    for (int k = 0; k < (K + 7) / 8; ++k) {
+      const int o2 = wave + 4 * k;
+      if (o2 < K / 2)
+        sw[o2][i] = (unsigned)W[(size_t)2 * o2 * nin + i] | ((unsigned)W[(size_t)(2 * o2 + 1) * nin + i] << 16);
+    }
+  __syncthreads();
+  const int c = (wave % cw) * 64 + lane, cl = c < nin ? c : nin - 1;
+  const int step = ndata * (4 / cw) * S;
+  for (; r0 < n; r0 += step) {
+    if (r0 + step < n) rows_touch<K, S>(dZ + (size_t)(r0 + step) * K, lane);
+    float z[S], acc[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      z[s] = Zprev[(size_t)(r0 + s < n ? r0 + s : r0) * nin + cl];
+      acc[s] = 0.0f;
+    }
+    rows_loop<K, S>(dZ + (size_t)r0 * K, sw, cl, acc);
     if (c < nin) {
 #pragma unroll
-      for (int s = 0; s < kRowsS; ++s) {
+      for (int s = 0; s < S; ++s) {
         if (r0 + s >= n) break;
-        const size_t idx = (size_t)(r0 + s) * nin + c;
-        dA[idx] = acc[s] * gelu_grad(Zprev[idx]);
+        dA[(size_t)(r0 + s) * nin + c] = acc[s] * gelu_grad(z[s]);
       }
     }
   }
@@ -414,10 +505,12 @@ void launch_linear_fwd(const float* A, int n, int nin, const unsigned short* W, 
   // kernel runs
   const bool al = ((uintptr_t)W % 16) == 0 && ((uintptr_t)A % 16) == 0;
   const bool wide = nout >= 16 && al;
-  const int per = kRowsS * (nout > 64 ? 2 : 4);  // samples of a workgroup and pass
+  const bool big = n >= kRowsBig;
+  const int per = (big ? kRowsS : kRowsS / 2) * (nout > 64 ? 2 : 4);  // samples of a workgroup and pass
   const dim3 grid(std::min((n + per - 1) / per, 2048));
-#define RP_ROWS(KK) \
-  hipLaunchKernelGGL(k_rows_fwd<KK>, grid, dim3(256), 0, s, A, n, W, b, nout, Z, act ? Aout : nullptr)
+#define RP_ROWS(KK)                                                                              \
+  hipLaunchKernelGGL((big ? k_rows_fwd<KK, kRowsS> : k_rows_fwd<KK, kRowsS / 2>), grid, dim3(256), 0, s, A, \
+                     n, W, b, nout, Z, act ? Aout : nullptr)
   if (wide && nin == 128) RP_ROWS(128);
   else if (wide && nin == 64) RP_ROWS(64);
   else if (wide && nin == 32) RP_ROWS(32);
@@ -457,22 +550,30 @@ void launch_output_loss(const float* A, int n, int nin, const unsigned short* W,
 void launch_bwd_layer(const float* dZ, const float* A, int n, int nin, int nout, const unsigned short* W,
                       const float* Zprev, float* dA, float* part, hipStream_t s) {
   RP_CHECK(nin <= kMaxIn && nout <= kMaxIn && n > 0, "MLP layer wider than 128 or empty batch");
-  const int nchunks = (n + kChunk - 1) / kChunk, njobs = nchunks * bwd_w_jobs(nin, nout);
-  const int nw = (njobs + 3) / 4;
-  const int per = kRowsS * (nin > 64 ? 2 : 4);
+  const BwdW b = bwd_w_shape(nin, nout);
+  const int nw = (n + kChunk - 1) / kChunk * b.lw * b.nu;  // weight-gradient jobs
+  const bool big = n >= kRowsBig;
+  const int per = (big ? kRowsS : kRowsS / 2) * (nin > 64 ? 2 : 4);
   const int nd = std::min((n + per - 1) / per, 2048);
-#define RP_BWD(KK)                                                                                   \
-  case KK:                                                                                           \
-    hipLaunchKernelGGL(k_bwd<KK>, dim3(nd + nw), dim3(256), 0, s, dZ, A, W, Zprev, n, nin, nd, njobs, \
-                       dA, part);                                                                    \
-    break;
+  auto weights = [&] {
+    RP_HIP(hipFuncSetAttribute((const void*)k_bwd_w, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)kBwdWLds));
+    hipLaunchKernelGGL(k_bwd_w, dim3(nw), dim3(256), kBwdWLds, s, dZ, A, n, nin, nout, part);
+  };
+  auto both = [&](auto kernel) {
+    RP_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)kBwdWLds));
+    hipLaunchKernelGGL(kernel, dim3(nd + nw), dim3(256), kBwdWLds, s, dZ, A, W, Zprev, n, nin, nw, dA, part);
+  };
+#define RP_BWD(KK) \
+  case KK: both(big ? k_bwd<KK, kRowsS> : k_bwd<KK, kRowsS / 2>); break;
   if (!dA) {
-    hipLaunchKernelGGL(k_bwd_w, dim3(nw), dim3(256), 0, s, dZ, A, n, nin, nout, njobs, part);
+    weights();
   } else {
     switch (nout) {
       RP_BWD(2) RP_BWD(8) RP_BWD(16) RP_BWD(32) RP_BWD(64) RP_BWD(128)
       default:
-        hipLaunchKernelGGL(k_bwd_w, dim3(nw), dim3(256), 0, s, dZ, A, n, nin, nout, njobs, part);
+        weights();
         hipLaunchKernelGGL(k_linear_bwd_data, dim3((n + kRows - 1) / kRows), dim3(256), 0, s, dZ, n, nout,
                            W, nin, Zprev, 1, dA);
     }
