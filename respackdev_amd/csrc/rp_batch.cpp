@@ -265,8 +265,7 @@ int rp_chiqw_batch_result(rp_handle h, int32_t iq, int32_t* ng, int32_t* ndir, i
     if (epsinv_out) {
       RP_HIP(hipSetDevice(h->device));
       const size_t n = (size_t)(s.q0 ? 3 : 1) * h->nen * s.ng * s.ng;
-      RP_HIP(hipMemcpyAsync(epsinv_out, s.d_eps.p, sizeof(double2) * n, hipMemcpyDeviceToHost, h->stream));
-      RP_HIP(hipStreamSynchronize(h->stream));
+      copy_to_host(h, epsinv_out, s.d_eps.p, sizeof(double2) * n);
     }
   });
 }

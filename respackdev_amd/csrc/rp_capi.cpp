@@ -724,6 +724,11 @@ static std::vector<ChiLaunch> chi_candidates(const rp_ctx* h, int prec) {
   return out;
 }
 
+// bytes of chi or eps^-1 of the prepared q, every frequency and direction
+static size_t chi_bytes(const rp_ctx* h) {
+  return sizeof(double2) * (size_t)h->nbatch() * h->ng * h->ng;
+}
+
 // seconds between two recorded (and completed) events
 static double event_seconds(hipEvent_t a, hipEvent_t b) {
   float ms = 0.0f;
@@ -849,10 +854,8 @@ int rp_chi_accumulate(rp_handle h, int32_t precision, double* chi_out) {
     const int nc = h->q0 ? 3 : 1;
     const ChiLaunch c = chi_launch(h, precision);
     issue_accumulate(h, precision, c, true);
-    if (chi_out)
-      RP_HIP(hipMemcpyAsync(chi_out, h->d_chi.p, sizeof(double2) * nc * (size_t)h->ng * h->ng * h->nen,
-                            hipMemcpyDeviceToHost, s));
     RP_HIP(hipStreamSynchronize(s));
+    if (chi_out) copy_to_host(h, chi_out, h->d_chi.p, chi_bytes(h));
     h->gemm_seconds = 0;
     h->gemm_launches = nc;
     for (int ix = 0; ix < nc; ++ix) {
@@ -871,7 +874,7 @@ int rp_chi_set(rp_handle h, const double* chi_in) {
     RP_HIP(hipSetDevice(h->device));
     const size_t n = (size_t)h->ng * h->ng * h->nen * (h->q0 ? 3 : 1);
     h->d_chi.reserve(n);
-    RP_HIP(hipMemcpy(h->d_chi.p, chi_in, sizeof(double2) * n, hipMemcpyHostToDevice));
+    copy_to_device(h, h->d_chi.p, chi_in, sizeof(double2) * n);
     h->have_chi = true;
   });
 }
@@ -883,10 +886,7 @@ int rp_dyson(rp_handle h, double* epsinv_out) {
     hipStream_t s = h->stream;
     issue_dyson(h);
     check_status(h, "Dyson step");
-    if (epsinv_out)
-      RP_HIP(hipMemcpyAsync(epsinv_out, h->d_eps.p, sizeof(double2) * h->nbatch() * (size_t)h->ng * h->ng,
-                            hipMemcpyDeviceToHost, s));
-    RP_HIP(hipStreamSynchronize(s));
+    if (epsinv_out) copy_to_host(h, epsinv_out, h->d_eps.p, chi_bytes(h));
   });
 }
 
@@ -901,9 +901,9 @@ int rp_chiqw_q(rp_handle h, const double* q, int32_t precision, double* epsinv_o
     RP_HIP(hipEventRecord(h->ev[1], s));
     if (rp_tetra_weights_batch(h, nullptr)) throw Error(g_err);
     RP_HIP(hipEventRecord(h->ev[2], s));
-    if (rp_chi_accumulate(h, precision, chi_out)) throw Error(g_err);
+    if (rp_chi_accumulate(h, precision, nullptr)) throw Error(g_err);
     RP_HIP(hipEventRecord(h->ev[3], s));
-    if (rp_dyson(h, epsinv_out)) throw Error(g_err);
+    if (rp_dyson(h, nullptr)) throw Error(g_err);
     RP_HIP(hipEventRecord(h->ev[4], s));
     // an ill-conditioned eps amplifies the FP32 accumulation error of the
     // split-BF16 contraction: run it again with the span its eps^-1 calls for
@@ -916,9 +916,9 @@ int rp_chiqw_q(rp_handle h, const double* q, int32_t precision, double* epsinv_o
     if (sp) {
       h->q_span = sp;
       RP_HIP(hipEventRecord(h->ev[1], s));
-      if (rp_chi_accumulate(h, precision, chi_out)) throw Error(g_err);
+      if (rp_chi_accumulate(h, precision, nullptr)) throw Error(g_err);
       RP_HIP(hipEventRecord(h->ev[2], s));
-      if (rp_dyson(h, epsinv_out)) throw Error(g_err);
+      if (rp_dyson(h, nullptr)) throw Error(g_err);
       RP_HIP(hipEventRecord(h->ev[3], s));
       RP_HIP(hipEventSynchronize(h->ev[3]));
       const double ta = event_seconds(h->ev[1], h->ev[2]), td = event_seconds(h->ev[2], h->ev[3]);
@@ -926,6 +926,9 @@ int rp_chiqw_q(rp_handle h, const double* q, int32_t precision, double* epsinv_o
       st[3] += td;
       st[4] += ta + td;
     }
+    // the results leave once, after any second run
+    if (chi_out) copy_to_host(h, chi_out, h->d_chi.p, chi_bytes(h));
+    if (epsinv_out) copy_to_host(h, epsinv_out, h->d_eps.p, chi_bytes(h));
     if (timings) {
       for (int i = 0; i < 5; ++i) timings[i] = st[i];
       timings[5] = h->prep_seconds;

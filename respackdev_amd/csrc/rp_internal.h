@@ -182,6 +182,7 @@ struct rp_ctx {
   int q_span = 0;                // the span chosen for the current q (0: the default)
   double last_kappa = 0;         // |eps^-1|_1 of the last q checked by adapt_span
   DevBuf<double> d_kappa;
+  rp::HostBuf<char> h_copy;      // pinned chunks of the large host copies (16 MiB)
   std::vector<rp::TuneEntry> tune;
   std::unique_ptr<rp::Batch> batch;
 
@@ -201,6 +202,10 @@ struct rp_ctx {
 };
 
 namespace rp {
+// Copies between device memory and a caller's host array, after the work on
+// h->stream; done when they return (rp_copy.cpp).
+void copy_to_host(rp_ctx* h, void* dst, const void* dev, size_t bytes);
+void copy_to_device(rp_ctx* h, void* dev, const void* src, size_t bytes);
 // Stage bodies (rp_capi.cpp): enqueue only, on h->stream.
 void check_status(rp_ctx* h, const char* what);
 // Throws the error a non-zero status word of the kernels stands for.
