@@ -155,16 +155,21 @@ void launch_w_contract(const float2* eps, const long long* eps_off, const double
                        int nwf, int nen, int max_nge, double2* xw, double2* funcw,
                        hipStream_t s);
 // xg: scratch of j_contract_scratch(sum over q of NG_eps, npair) complex values
+size_t j_x_elems(int nge, int ncol);
+size_t j_z_elems(int nge, int ncol);
+int j_row_shares(int ngroups, int nen, int max_ncol, int max_nge, int ncu);
+size_t j_group_bytes();
+void pack_j_group(void* at, int nge, int iqir, int mbeg, int ncol, long long xoff, long long zoff);
 void launch_j_contract(const float2* eps, const long long* eps_off, const double2* rho,
-                       const long long* rho_off, const int4* qinfo, const int* minv,
-                       const double2* pf1, const double2* pf2, const long long* map_off,
-                       double2* xg, const double2* shell, int ntq, int npair, int nen,
-                       double2* funcw, hipStream_t s);
-size_t j_contract_scratch(size_t sum_nge, int npair);
-void launch_j_func(const double2* rho, const long long* rho_off, const int4* qinfo, int ntq,
-                   int npair, double2* func, double2* shell, hipStream_t s);
-void launch_j_sum(const double2* func, const double2* funcw, int ntq, int nwf, int nen, int r0,
-                  double volume, double chead, const double2* cheadw, double2* xmat,
+                       const long long* rho_off, long long rho_r, const int4* qinfo,
+                       const int* minv, const double2* pf1, const double2* pf2,
+                       const long long* map_off, const void* groups, const int* gmem, int ngroups,
+                       int max_nge, int max_ncol, int npair, int nr, int nrs, int ntq, int nen,
+                       double2* xs, double2* zs, double2* funcw, hipStream_t s);
+void launch_j_func(const double2* rho, const long long* rho_off, long long rho_r, const int4* qinfo,
+                   int ntq, int npair, int nr, double2* func, hipStream_t s);
+void launch_j_sum(const double2* func, const double2* funcw, int ntq, int nwf, int nen, int nr, int nrs,
+                  const int* isr0, double volume, double chead, const double2* cheadw, double2* xmat,
                   double2* jmat, size_t wstride, hipStream_t s);
 void launch_w_fourier(const double2* func, const double2* funcw, const double* sq, int ntq, int nwf,
                       int nen, const int na[3], double volume, double chead, const double2* cheadw,

@@ -70,6 +70,11 @@ struct W3d {
   DevBuf<long long> d_geo_qg_off, d_geo_plan_off;
   // summed pair-density grids P[q][p][r] of a chunk of q (launch_pair_rsum)
   DevBuf<double2> d_P;
+  // exchange (rp_j3d_run): work buffers kept between calls, sized to a batch of R
+  DevBuf<double2> d_pfk, d_jrho, d_jfunc, d_jfuncw, d_jx, d_jj, d_jz, d_jxs;
+  DevBuf<long long> d_joff;
+  DevBuf<char> d_jgrp;
+  DevBuf<int> d_jmem, d_jr0;
   DevBuf<double2> d_rho, d_pf1, d_pf2, d_func, d_shell, d_funcw, d_cheadw, d_vmat, d_wmat;
   // device seconds of the last rp_w3d_funcs (rho, func, W contraction, total)
   // and rp_j3d_run (rho of every R, func and sums, J contraction, total),
@@ -257,6 +262,8 @@ void ensure_geometry(W3d& w, hipStream_t s) {
   w.geo_ready = true;
 }
 
+// Work buffers of a batch of R of the exchange.
+constexpr size_t kJBudgetBytes = size_t(2) << 30;
 // Bound on the summed pair-density grids held at once (q chunks of launch_pair_rsum).
 constexpr size_t kPBudgetBytes = size_t(1) << 30;
 
@@ -711,58 +718,102 @@ int rp_j3d_run(rp_handle h, int32_t nr, const int32_t* rvec, double* xmat, doubl
     // e^{-i 2pi k.R} per R and k (calc_intJ.F:646-650)
     const double tpi = 2.0 * std::acos(-1.0);
     std::vector<double2> pfk((size_t)nr * ntk);
-    for (int r = 0; r < nr; ++r)
+    std::vector<int> r0(nr);
+    for (int r = 0; r < nr; ++r) {
+      r0[r] = rvec[3 * r] == 0 && rvec[3 * r + 1] == 0 && rvec[3 * r + 2] == 0;
       for (int k = 0; k < ntk; ++k) {
         const double ph = tpi * (w.sk0[3 * k] * rvec[3 * r] + w.sk0[3 * k + 1] * rvec[3 * r + 1] +
                                  w.sk0[3 * k + 2] * rvec[3 * r + 2]);
         pfk[(size_t)r * ntk + k] = make_double2(std::cos(ph), -std::sin(ph));
       }
-    DevBuf<double2> d_pfk;
-    d_pfk.upload(pfk, s);
+    }
+    w.d_pfk.upload(pfk, s);
+    w.d_jr0.upload(r0, s);
     // rho per (R, q): [r][q][p][G]
     std::vector<long long> joff(w.ntq);
     long long tot = 0;
     for (int iq = 0; iq < w.ntq; ++iq) { joff[iq] = tot; tot += (long long)npair * w.ngpsi[iq]; }
-    DevBuf<long long> d_joff;
-    d_joff.upload(joff, s);
-    DevBuf<double2> d_jrho, d_jfunc, d_jshell, d_jfuncw, d_x, d_j, d_cw, d_xg;
-    d_jrho.reserve((size_t)tot * nr);
-    ensure_geometry(w, s);
-    w.events(2 + 2 * (size_t)nr);
-    RP_HIP(hipEventRecord(w.ev[0], s));
-    for (int r = 0; r < nr; ++r)
-      rho_all_q(w, true, d_pfk.p + (size_t)r * ntk, d_joff.p, d_jrho.p + (size_t)r * tot, s);
-    RP_HIP(hipEventRecord(w.ev[1], s));
-    d_jfunc.reserve((size_t)w.ntq * npair);
-    d_jshell.reserve((size_t)w.ntq * npair);
-    d_jfuncw.reserve((size_t)w.ntq * nen * npair);
-    d_x.reserve((size_t)nr * npair);
-    d_j.reserve((size_t)nr * nen * npair);
-    d_cw.upload(w.cheadw, s);
-    d_xg.reserve(j_contract_scratch(w.minv.size(), npair));
-    for (int r = 0; r < nr; ++r) {
-      const double2* rho = d_jrho.p + (size_t)r * tot;
-      launch_j_func(rho, d_joff.p, w.d_qinfo.p, w.ntq, npair, d_jfunc.p, d_jshell.p, s);
-      RP_HIP(hipEventRecord(w.ev[2 + 2 * r], s));
-      launch_j_contract(w.d_eps.p, w.d_eps_off.p, rho, d_joff.p, w.d_qinfo.p, w.d_minv.p, w.d_pf1.p,
-                        w.d_pf2.p, w.d_map_off.p, d_xg.p, d_jshell.p, w.ntq, npair, nen, d_jfuncw.p,
-                        s);
-      RP_HIP(hipEventRecord(w.ev[3 + 2 * r], s));
-      const int r0 = rvec[3 * r] == 0 && rvec[3 * r + 1] == 0 && rvec[3 * r + 2] == 0;
-      launch_j_sum(d_jfunc.p, d_jfuncw.p, w.ntq, nwf, nen, r0, w.volume, w.chead, d_cw.p,
-                   d_x.p + (size_t)r * npair, d_j.p + (size_t)r * npair, (size_t)nr * npair, s);
+    w.d_joff.upload(joff, s);
+    // the full-mesh q of each irreducible one: the groups of the contraction
+    std::vector<std::vector<int>> by(w.nq_irr);
+    for (int q = 0; q < w.ntq; ++q) by[w.qinfo[q].z].push_back(q);
+    std::vector<int> mem, mbeg;
+    size_t sum_nge = 0;
+    for (const auto& v : by) {
+      mbeg.push_back((int)mem.size());
+      mem.insert(mem.end(), v.begin(), v.end());
+      for (int q : v) sum_nge += (size_t)w.nge[q];
     }
+    w.d_jmem.upload(mem, s);
+    // R in batches whose rho, X, Z (32 bytes a row and column) and row sums stay
+    // near kJBudgetBytes; one R at least
+    const int max_nge = *std::max_element(w.nge.begin(), w.nge.end());
+    int most = 0;
+    for (const auto& v : by) most = std::max(most, (int)v.size());
+    const size_t per_r = 16 * (size_t)tot + 32 * sum_nge * npair + 64 * (size_t)w.ntq * nen * npair;
+    const int nrb = (int)std::max<size_t>(1, std::min<size_t>(nr, kJBudgetBytes / per_r));
+    w.d_jx.reserve((size_t)nr * npair);
+    w.d_jj.reserve((size_t)nr * nen * npair);
+    w.d_cheadw.upload(w.cheadw, s);
+    w.d_jrho.reserve((size_t)tot * nrb);
+    w.d_jfunc.reserve((size_t)nrb * w.ntq * npair);
+    ensure_geometry(w, s);
+    const int nbatch = (nr + nrb - 1) / nrb;
+    w.events(2 + 4 * (size_t)nbatch);
+    std::vector<char> grp(by.size() * j_group_bytes());
+    int grp_nr = 0;
+    for (int bt = 0; bt < nbatch; ++bt) {
+      const int ra = bt * nrb, nb = std::min(nrb, nr - ra);
+      if (grp_nr != nb) {  // columns and offsets of the groups for this many R
+        size_t xt = 0, zt = 0;
+        RP_HIP(hipStreamSynchronize(s));  // the previous upload has left grp
+        for (size_t g = 0; g < by.size(); ++g) {
+          const int nge = w.nge[by[g][0]], ncol = (int)by[g].size() * nb * npair;
+          pack_j_group(grp.data() + g * j_group_bytes(), nge, (int)g, mbeg[g], ncol, (long long)xt,
+                       (long long)zt);
+          xt += j_x_elems(nge, ncol);
+          zt += j_z_elems(nge, ncol);
+        }
+        w.d_jgrp.upload(grp.data(), grp.size(), s);
+        w.d_jxs.reserve(xt);
+        w.d_jz.reserve(zt);
+        grp_nr = nb;
+      }
+      const int max_ncol = most * nb * npair;
+      const int nrs = j_row_shares((int)by.size(), nen, max_ncol, max_nge, h->ncu);
+      w.d_jfuncw.reserve((size_t)nrs * nb * w.ntq * nen * npair);
+      hipEvent_t* ev = &w.ev[2 + 4 * bt];
+      RP_HIP(hipEventRecord(ev[0], s));
+      for (int r = 0; r < nb; ++r)
+        rho_all_q(w, true, w.d_pfk.p + (size_t)(ra + r) * ntk, w.d_joff.p, w.d_jrho.p + (size_t)r * tot,
+                  s);
+      RP_HIP(hipEventRecord(ev[1], s));
+      launch_j_func(w.d_jrho.p, w.d_joff.p, tot, w.d_qinfo.p, w.ntq, npair, nb, w.d_jfunc.p, s);
+      RP_HIP(hipEventRecord(ev[2], s));
+      launch_j_contract(w.d_eps.p, w.d_eps_off.p, w.d_jrho.p, w.d_joff.p, tot, w.d_qinfo.p, w.d_minv.p,
+                        w.d_pf1.p, w.d_pf2.p, w.d_map_off.p, w.d_jgrp.p, w.d_jmem.p, (int)by.size(),
+                        max_nge, max_ncol, npair, nb, nrs, w.ntq, nen, w.d_jxs.p, w.d_jz.p,
+                        w.d_jfuncw.p, s);
+      RP_HIP(hipEventRecord(ev[3], s));
+      launch_j_sum(w.d_jfunc.p, w.d_jfuncw.p, w.ntq, nwf, nen, nb, nrs, w.d_jr0.p + ra, w.volume,
+                   w.chead, w.d_cheadw.p, w.d_jx.p + (size_t)ra * npair,
+                   w.d_jj.p + (size_t)ra * npair, (size_t)nr * npair, s);
+    }
+    RP_HIP(hipEventRecord(w.ev[1], s));
     if (xmat)
-      RP_HIP(hipMemcpyAsync(xmat, d_x.p, sizeof(double2) * nr * npair, hipMemcpyDeviceToHost, s));
+      RP_HIP(hipMemcpyAsync(xmat, w.d_jx.p, sizeof(double2) * nr * npair, hipMemcpyDeviceToHost, s));
     if (jmat)
-      RP_HIP(hipMemcpyAsync(jmat, d_j.p, sizeof(double2) * nr * nen * npair, hipMemcpyDeviceToHost, s));
+      RP_HIP(hipMemcpyAsync(jmat, w.d_jj.p, sizeof(double2) * nr * nen * npair, hipMemcpyDeviceToHost, s));
     RP_HIP(hipStreamSynchronize(s));
-    double tj = 0.0;
-    for (int r = 0; r < nr; ++r) tj += event_s(w.ev[2 + 2 * r], w.ev[3 + 2 * r]);
-    w.stage_s[4] = event_s(w.ev[0], w.ev[1]);
+    double tr = 0.0, tj = 0.0;
+    for (int bt = 0; bt < nbatch; ++bt) {
+      tr += event_s(w.ev[2 + 4 * bt], w.ev[3 + 4 * bt]);
+      tj += event_s(w.ev[4 + 4 * bt], w.ev[5 + 4 * bt]);
+    }
+    w.stage_s[4] = tr;
     w.stage_s[6] = tj;
-    w.stage_s[7] = event_s(w.ev[0], w.ev[3 + 2 * (nr - 1)]);
-    w.stage_s[5] = w.stage_s[7] - w.stage_s[4] - tj;
+    w.stage_s[7] = event_s(w.ev[2], w.ev[1]);
+    w.stage_s[5] = w.stage_s[7] - tr - tj;
     if (heads) {
       heads[0] = w.chead;
       heads[1] = 0.0;

@@ -13,6 +13,9 @@
 // map and a phase per G, folded into the rho vectors so that eps^-1 is read
 // once, coalesced, straight from its irreducible copy.  Finally the lattice
 // Fourier sums with the Hybertsen-Louie heads (k_w_fourier).
+#include <algorithm>
+#include <type_traits>
+
 #include "rp_common.h"
 #include "rp_kernels.h"
 
@@ -260,244 +263,292 @@ __global__ void __launch_bounds__(512) k_w_contract(
 }
 
 // calc_j3d's contraction on the FP64 matrix cores: funcw_pp of the diagonal
-// pairs, by k_w_contract's formula, with Y = E X as real products v_mfma_f64_16x16x4 (Re Y =
-// Er Xr - Ei Xi, Im Y = Er Xi + Ei Xr) over 16-row blocks of E and 16-column
-// blocks of up to 32 pair vectors (blockIdx.z picks the 32).  X comes from
-// k_j_xvec, [b][32 groups] in HBM (zero past the last pair).  A wave takes up
-// to kJA row blocks per pass (wave + 8 j) and the passes cover every row, so
-// a workgroup reads E once: E is read once per (q, w) for up to 32 pair vectors
-// and once per (q, w, group of 32) beyond (NWF >= 6).  Lane
-// l supplies A(l % 16, l / 16) and B(l / 16, l % 16) and holds
-// D(l / 16 + 4 v, l % 16), v < 4 (checked on the GPU with row- and column-numbered
-// operands).  grid: (nen, ntq, groups), 512 threads.
-constexpr int kJA = 1;
-__global__ void __launch_bounds__(256) k_j_xvec(const double2* __restrict__ rho,
+// pairs of every R of a batch, by k_w_contract's formula.  A group is an
+// irreducible q: its columns are the pair vectors of every full-mesh q that
+// shares its eps^-1 and of every R, c = (member * nr + R) * npair + p, so that
+// eps^-1 is read once per 64 columns instead of once per (q, R) and the columns
+// fill the 16-wide blocks (25 pairs of one q and R fill 25 of 32; the 350 of two
+// q and seven R all but two of 352).
+//
+// k_j_vecs forms once per batch, for every group, X [nbp][cpad] (nbp: NG_eps
+// rounded up to 8 rows, cpad: the columns to 16, zero beyond) and Z [NG_eps][cpad].  k_j_contract then takes 64 columns of one
+// (group, w): Y = E X as three real products, Re Y = T1 - T2, Im Y = T3 - T1 - T2
+// with T1 = er xr, T2 = ei xi, T3 = (er + ei)(xr + xi), over tiles of up to 64
+// rows and 8 columns of E at a time staged in LDS, and folds each tile into the
+// sums over rows Z_c(a) Y(a, c).  A wave takes one column block of 16 and every
+// row block of the tile (with fewer column blocks the rows are dealt out).
+// Bound by the FP64 MFMAs (shared with the FP64 vector unit, hence planes formed
+// once per workgroup): 64 q, 16 frequencies, 25 pairs, NG_eps ~310: seven
+// R 2.01 ms (52 TFLOP/s executed; 4.20 ms with every (q, R) on its own and four
+// real products), one R 0.37 ms (0.59).  Three workgroups per CU; two take 2.18
+// ms, four spill.
+constexpr int kJT = 64, kJKC = 8;                 // rows / columns of a tile, K per chunk
+constexpr int kJRow = kJT + 16, kJPlane = kJKC * kJRow;
+
+struct JGroup {
+  int nge, iqir, mbeg, ncol;   // first member in gmem, columns
+  long long xoff, zoff;        // first element of X and of Z
+};
+
+__global__ void __launch_bounds__(256) k_j_vecs(const double2* __restrict__ rho,
                                                 const long long* __restrict__ rho_off,
-                                                const int4* __restrict__ qinfo,
+                                                long long rho_r, const int4* __restrict__ qinfo,
                                                 const int* __restrict__ minv,
                                                 const double2* __restrict__ pf1,
                                                 const double2* __restrict__ pf2,
-                                                const long long* __restrict__ map_off, int nv,
-                                                int g32, double2* __restrict__ xg) {
-  const int q = blockIdx.x;
-  const int4 qi = qinfo[q];
-  const int nge = qi.x, ngpsi = qi.y, trs = qi.w;
-  const double2* r = rho + rho_off[q];
-  const int* mi = minv + map_off[q];
-  const double2* p1 = pf1 + map_off[q];
-  const double2* p2 = pf2 + map_off[q];
-  double2* out = xg + map_off[q] * g32;
-  for (int e = threadIdx.x; e < nge * g32; e += blockDim.x) {
-    const int b = e / g32, c = e % g32;
-    double2 v = make_double2(0.0, 0.0);
-    if (c < nv) {
-      const int g = mi[b];
-      const double2 rv = r[(size_t)c * ngpsi + g];
-      const double2 p = trs == 1 ? p2[g] : p1[g];
-      // trs = +1: conj(rho) pf2; trs = -1: rho pf1
-      const double xr = rv.x, xi = trs == 1 ? -rv.y : rv.y;
-      v = make_double2(xr * p.x - xi * p.y, xr * p.y + xi * p.x);
+                                                const long long* __restrict__ map_off,
+                                                const JGroup* __restrict__ grp,
+                                                const int* __restrict__ gmem, int np, int nr,
+                                                double2* __restrict__ xs, double2* __restrict__ zs) {
+  const JGroup g = grp[blockIdx.z];
+  const int nbp = (g.nge + kJKC - 1) / kJKC * kJKC, cpad = (g.ncol + 15) / 16 * 16;
+  const int c0 = blockIdx.x * 32, b0 = blockIdx.y * 32;
+  if (c0 >= cpad || b0 >= nbp) return;
+  __shared__ double2 sx[32][33], sz[32][33];  // [c][b]
+  const int lane = threadIdx.x & 31, row = threadIdx.x >> 5;
+  for (int i = row; i < 32; i += 8) {  // rows G along the lanes, one column each
+    const int c = c0 + i, b = b0 + lane;
+    double2 x = make_double2(0.0, 0.0), z = x;
+    if (c < g.ncol && b < g.nge) {
+      const int m = c / (nr * np), r = c / np % nr, p = c % np;
+      const int q = gmem[g.mbeg + m];
+      const int4 qi = qinfo[q];
+      const long long mo = map_off[q];
+      const int gg = minv[mo + b];
+      const double2 v = rho[(long long)r * rho_r + rho_off[q] + (long long)p * qi.y + gg];
+      const double2 p1 = pf1[mo + gg], p2 = pf2[mo + gg];
+      // trs = +1: X = conj(rho) pf2, Z = rho pf1; trs = -1: X = rho pf1, Z = conj(rho) pf2
+      const double2 a = make_double2(v.x * p1.x - v.y * p1.y, v.x * p1.y + v.y * p1.x);
+      const double2 d = make_double2(v.x * p2.x + v.y * p2.y, v.x * p2.y - v.y * p2.x);
+      x = qi.w == 1 ? d : a;
+      z = qi.w == 1 ? a : d;
     }
-    out[e] = v;
-  }
-}
-
-__global__ void __launch_bounds__(512) k_j_contract(
-    const float2* __restrict__ eps, const long long* __restrict__ eps_off,
-    const double2* __restrict__ rho, const long long* __restrict__ rho_off,
-    const int4* __restrict__ qinfo, const int* __restrict__ minv,
-    const double2* __restrict__ pf1, const double2* __restrict__ pf2,
-    const long long* __restrict__ map_off, const double2* __restrict__ xg, int g32,
-    const double2* __restrict__ shell, int nv, int nen, double2* __restrict__ funcw) {
-  const int w = blockIdx.x, q = blockIdx.y, grp = blockIdx.z;
-  const int4 qi = qinfo[q];
-  const int nge = qi.x, ngpsi = qi.y, iqir = qi.z, trs = qi.w;
-  const int ld = w3d_eps_ld(nge);
-  const float2* E = eps + eps_off[iqir] + (size_t)w * ld * nge;
-  const int c0 = grp * 32, nvb = min(32, nv - c0);
-  const double2* Xq = xg + map_off[q] * g32 + c0;  // (b, c) at Xq[b * g32 + c]
-  const double2* r = rho + rho_off[q] + (size_t)c0 * ngpsi;
-  const int* mi = minv + map_off[q];
-  const double2* p1 = pf1 + map_off[q];
-  const double2* p2 = pf2 + map_off[q];
-  __shared__ double red[32][8][2];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const int nab = (nge + 15) / 16;
-  double sre[2] = {0.0, 0.0}, sim[2] = {0.0, 0.0};  // this lane's sums for c = 16 cb + li
-  for (int a0 = 0; a0 < nab; a0 += 8 * kJA) {
-    jd4 accr[kJA][2], acci[kJA][2];
-    int arow[kJA];
-#pragma unroll
-    for (int j = 0; j < kJA; ++j) {
-      // rows nge .. ld-1 are the zero padding, rows past ld (row blocks past
-      // the last) read row 0; their sums are never used
-      const int a = (a0 + wave + 8 * j) * 16 + li;
-      arow[j] = a < ld ? a : 0;
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) accr[j][cb] = acci[j][cb] = jd4{0.0, 0.0, 0.0, 0.0};
-    }
-    // the next step's X and E are loaded during this step's MFMAs (the last
-    // step loads itself again); columns past nge contribute zero
-    int bn = lk < nge ? lk : nge - 1;
-    double2 xn[2];
-    float2 en[kJA];
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) xn[cb] = Xq[(size_t)bn * g32 + cb * 16 + li];
-#pragma unroll
-    for (int j = 0; j < kJA; ++j) en[j] = E[(size_t)bn * ld + arow[j]];
-    for (int b0 = 0; b0 < nge; b0 += 4) {
-      const bool bv = b0 + lk < nge;
-      double xr[2], xi[2], nxi[2];
-      float2 ec[kJA];
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        xr[cb] = bv ? xn[cb].x : 0.0;
-        xi[cb] = bv ? xn[cb].y : 0.0;
-        nxi[cb] = -xi[cb];
-      }
-#pragma unroll
-      for (int j = 0; j < kJA; ++j) ec[j] = en[j];
-      const int b1 = (b0 + 4 < nge ? b0 + 4 : b0) + lk;
-      bn = b1 < nge ? b1 : nge - 1;
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) xn[cb] = Xq[(size_t)bn * g32 + cb * 16 + li];
-#pragma unroll
-      for (int j = 0; j < kJA; ++j) en[j] = E[(size_t)bn * ld + arow[j]];
-#pragma unroll
-      for (int j = 0; j < kJA; ++j) {
-        const double er = ec[j].x, ei = ec[j].y;
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-          accr[j][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(er, xr[cb], accr[j][cb], 0, 0, 0);
-          accr[j][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei, nxi[cb], accr[j][cb], 0, 0, 0);
-          acci[j][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(er, xi[cb], acci[j][cb], 0, 0, 0);
-          acci[j][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei, xr[cb], acci[j][cb], 0, 0, 0);
-        }
-      }
-    }
-    // Z_c(a) Y(a, c) for this lane's rows a = 16 (row block) + lk + 4 v and columns c
-#pragma unroll
-    for (int j = 0; j < kJA; ++j) {
-      const int ab = a0 + wave + 8 * j;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int a = ab * 16 + lk + 4 * v;
-        if (ab >= nab || a >= nge) continue;
-        const int g = mi[a];
-        const double2 pp = trs == 1 ? p1[g] : p2[g];
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb) {
-          const int c = cb * 16 + li;
-          if (c >= nvb) continue;
-          const double2 rv = r[(size_t)c * ngpsi + g];
-          double zr, zi;
-          if (trs == 1) {  // Z = rho pf1
-            zr = rv.x * pp.x - rv.y * pp.y;
-            zi = rv.x * pp.y + rv.y * pp.x;
-          } else {         // Z = conj(rho) pf2
-            zr = rv.x * pp.x + rv.y * pp.y;
-            zi = rv.x * pp.y - rv.y * pp.x;
-          }
-          const double yr = accr[j][cb][v], yi = acci[j][cb][v];
-          sre[cb] += zr * yr - zi * yi;
-          sim[cb] += zr * yi + zi * yr;
-        }
-      }
-    }
-  }
-  // lanes of one column (li) hold their rows' sums: over lk, then the waves
-#pragma unroll
-  for (int cb = 0; cb < 2; ++cb)
-    for (int off = 16; off < 64; off <<= 1) {
-      sre[cb] += __shfl_xor(sre[cb], off);
-      sim[cb] += __shfl_xor(sim[cb], off);
-    }
-  if (lk == 0) {
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      red[cb * 16 + li][wave][0] = sre[cb];
-      red[cb * 16 + li][wave][1] = sim[cb];
-    }
+    sx[i][lane] = x;
+    sz[i][lane] = z;
   }
   __syncthreads();
-  for (int e = t; e < 2 * nvb; e += blockDim.x) {
-    const int p = e >> 1, part = e & 1;
-    double sum = 0.0;
-#pragma unroll
-    for (int wv = 0; wv < 8; ++wv) sum += red[p][wv][part];
-    const double2 sh = shell[(size_t)q * nv + c0 + p];
-    double2* o = funcw + ((size_t)q * nen + w) * nv + c0 + p;
-    if (part == 0) o->x = sum + sh.x;
-    else o->y = sum + sh.y;
+  for (int i = row; i < 32; i += 8) {  // columns along the lanes
+    const int b = b0 + i, c = c0 + lane;
+    if (b >= nbp || c >= cpad) continue;
+    const double2 x = sx[lane][i];
+    xs[g.xoff + (size_t)b * cpad + c] = x;
+    if (b < g.nge) zs[g.zoff + (size_t)b * cpad + c] = sz[lane][i];
   }
 }
 
-// calc_j3d func / shell (calc_intJ.F:680-690): per (q, p) sum_G |rho_p(G)|^2 as
-// rho conj(rho).  grid: (ntq, npair), 256 threads; out [q][p].
-__global__ void __launch_bounds__(256) k_j_func(const double2* __restrict__ rho,
-                                                const long long* __restrict__ rho_off,
-                                                const int4* __restrict__ qinfo, int np,
-                                                double2* __restrict__ func,
-                                                double2* __restrict__ shell) {
-  const int q = blockIdx.x, p = blockIdx.y;
-  const int4 qi = qinfo[q];
-  const int nge = qi.x, ngpsi = qi.y;
-  const double2* r = rho + rho_off[q] + (size_t)p * ngpsi;
-  __shared__ double red[256];
-  double f[4] = {0, 0, 0, 0};
-  for (int g = threadIdx.x; g < ngpsi; g += blockDim.x) {
-    const double2 a = r[g];
-    const double pr = a.x * a.x + a.y * a.y, pi = a.y * a.x - a.x * a.y;
-    f[0] += pr;
-    f[1] += pi;
-    if (g >= nge) { f[2] += pr; f[3] += pi; }
-  }
+// NR row blocks from block rb on by the column block cb of a staged chunk.
+template <int NR>
+__device__ __forceinline__ void j_chunk(const double* pe, const double* px, int rb, int cb, int li,
+                                        int lk, jd4 (&acc)[3][NR]) {
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    red[threadIdx.x] = f[c];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+  for (int k0 = 0; k0 < kJKC; k0 += 4)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      const int o = p * kJPlane + (k0 + lk) * kJRow + li;
+      const double x = px[o + 16 * cb];
+      double e[NR];
+#pragma unroll
+      for (int a = 0; a < NR; ++a) e[a] = pe[o + 16 * (rb + a)];
+#pragma unroll
+      for (int a = 0; a < NR; ++a)
+        acc[p][a] = __builtin_amdgcn_mfma_f64_16x16x4f64(e[a], x, acc[p][a], 0, 0, 0);
+    }
+}
+
+// grid: (nen, groups, column tiles of the widest group x nrs), 256 threads; row
+// tile t of a workgroup with row share s (of nrs) is taken when t % nrs == s.
+// out[s][R][q][w][p]: the partial sums over that share's rows.
+__global__ void __launch_bounds__(256, 3) k_j_contract(
+    const float2* __restrict__ eps, const long long* __restrict__ eps_off,
+    const JGroup* __restrict__ grp, const int* __restrict__ gmem, const double2* __restrict__ xs,
+    const double2* __restrict__ zs, int np, int nr, int nrs, int ntq, int nen,
+    double2* __restrict__ out) {
+  __shared__ double se[3 * kJPlane], sx[3 * kJPlane];
+  __shared__ double2 red[4][16];
+  const int w = blockIdx.x, rs = (int)blockIdx.z % nrs, tc = (int)blockIdx.z / nrs;
+  const JGroup g = grp[blockIdx.y];
+  const int ncb = (g.ncol + 15) / 16, nct = (ncb + 3) / 4, cpad = 16 * ncb;
+  if (tc >= nct) return;  // uniform
+  const int hb = tc * ncb / nct, nc = (tc + 1) * ncb / nct - hb;  // column blocks, dealt evenly
+  const int nab = (g.nge + 15) / 16, nat = (nab + 3) / 4;
+  const int ld = w3d_eps_ld(g.nge), nbp = (g.nge + kJKC - 1) / kJKC * kJKC;
+  const float2* E = eps + eps_off[g.iqir] + (size_t)w * ld * g.nge;
+  const double2* X = xs + g.xoff;
+  const double2* Z = zs + g.zoff;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int part = (wave + (int)(blockIdx.x + blockIdx.y)) & 3;
+  const int li = lane & 15, lk = lane >> 4;
+  // this wave's column block and share of a tile's row blocks
+  const int cb = nc >= 3 ? part : (nc == 2 ? part & 1 : 0);
+  const int nsh = nc >= 3 ? 1 : (nc == 2 ? 2 : 4), sh = nc >= 3 ? 0 : (nc == 2 ? part >> 1 : part);
+  const int xc = min(16 * hb + lane, cpad - 1);
+  float2 ev[kJKC / 4];
+  double2 xv[kJKC / 4];
+  auto load = [&](int a0, int b0) {
+    const int a = min(a0 + lane, ld - 1);
+#pragma unroll
+    for (int e = 0; e < kJKC / 4; ++e) {
+      const int b = b0 + wave + 4 * e;
+      ev[e] = (E + (size_t)min(b, g.nge - 1) * ld)[a];  // X is zero past NG_eps
+      xv[e] = (X + (size_t)b * cpad)[xc];
+    }
+  };
+  double sre = 0.0, sim = 0.0;  // this lane's rows of column 16 (hb + cb) + li
+  if (rs < nat) load(16 * (rs * nab / nat), 0);
+  // one row tile for a wave with NR of its row blocks, from rb on (0: it only
+  // stages); next: first row of the workgroup's next tile, < 0 for none
+  auto tile = [&](auto rows, int ab, int rb, int next) {
+    constexpr int NR = decltype(rows)::value;
+    jd4 acc[3][NR > 0 ? NR : 1];
+#pragma unroll
+    for (int p = 0; p < 3; ++p)
+#pragma unroll
+      for (int a = 0; a < NR; ++a) acc[p][a] = jd4{0, 0, 0, 0};
+    for (int b0 = 0; b0 < nbp; b0 += kJKC) {
+#pragma unroll
+      for (int e = 0; e < kJKC / 4; ++e) {
+        const int o = (wave + 4 * e) * kJRow + lane;
+        const double er = ev[e].x, ei = ev[e].y;
+        se[o] = er;
+        se[kJPlane + o] = ei;
+        se[2 * kJPlane + o] = er + ei;
+        sx[o] = xv[e].x;
+        sx[kJPlane + o] = xv[e].y;
+        sx[2 * kJPlane + o] = xv[e].x + xv[e].y;
+      }
+      __syncthreads();
+      if (b0 + kJKC < nbp) load(16 * ab, b0 + kJKC);
+      else if (next >= 0) load(next, 0);
+      if constexpr (NR > 0) j_chunk<NR>(se, sx, rb, cb, li, lk, acc);
       __syncthreads();
     }
-    if (threadIdx.x == 0) {
-      double2* o = (c < 2 ? func : shell) + (size_t)q * np + p;
-      if (c % 2 == 0) o->x = red[0];
-      else o->y = red[0];
+    const int c = 16 * (hb + cb) + li;
+#pragma unroll
+    for (int a = 0; a < NR; ++a) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int ar = 16 * (ab + rb + a) + lk + 4 * v;
+        if (ar >= g.nge) continue;
+        const double yr = acc[0][a][v] - acc[1][a][v];
+        const double yi = acc[2][a][v] - acc[0][a][v] - acc[1][a][v];
+        const double2 z = Z[(size_t)ar * cpad + c];
+        sre += z.x * yr - z.y * yi;
+        sim += z.x * yi + z.y * yr;
+        if (v & 1) __builtin_amdgcn_sched_barrier(0);  // few Z in registers at a time: no spills
+      }
     }
-    __syncthreads();
+  };
+  using std::integral_constant;
+  for (int t = rs; t < nat; t += nrs) {
+    const int ab = t * nab / nat, na = (t + 1) * nab / nat - ab;
+    const int rb = na * sh / nsh, nrb = cb < nc ? na * (sh + 1) / nsh - rb : 0;
+    const int next = t + nrs < nat ? 16 * ((t + nrs) * nab / nat) : -1;
+    if (nrb == 4) tile(integral_constant<int, 4>{}, ab, rb, next);
+    else if (nrb == 3) tile(integral_constant<int, 3>{}, ab, rb, next);
+    else if (nrb == 2) tile(integral_constant<int, 2>{}, ab, rb, next);
+    else if (nrb == 1) tile(integral_constant<int, 1>{}, ab, rb, next);
+    else tile(integral_constant<int, 0>{}, ab, rb, next);
   }
+  for (int off = 16; off < 64; off <<= 1) {
+    sre += __shfl_xor(sre, off);
+    sim += __shfl_xor(sim, off);
+  }
+  if (lk == 0) red[part][li] = make_double2(sre, sim);
+  __syncthreads();
+  for (int e = threadIdx.x; e < 16 * nc; e += 256) {
+    const int k = e / 16, c = 16 * (hb + k) + e % 16;
+    if (c >= g.ncol) continue;
+    double2 v = red[k][e % 16];  // the shares of column block k: parts k, k + 4 / nsh, ...
+    for (int i = 1; i < nsh; ++i) {
+      const double2 u = red[k + i * (4 / nsh)][e % 16];
+      v.x += u.x;
+      v.y += u.y;
+    }
+    const int m = c / (nr * np), r = c / np % nr, p = c % np;
+    const int q = gmem[g.mbeg + m];
+    out[((((size_t)rs * nr + r) * ntq + q) * nen + w) * np + p] = v;
+  }
+}
+
+// calc_j3d func / shell (calc_intJ.F:680-690): per (R, q, p) sum_G |rho_p(G)|^2
+// (real) over every G and over the shell beyond the eps sphere.  A wave per
+// (R, q, p); out [R][q][p] as (all, shell).
+__global__ void __launch_bounds__(256) k_j_func(const double2* __restrict__ rho,
+                                                const long long* __restrict__ rho_off,
+                                                long long rho_r, const int4* __restrict__ qinfo,
+                                                int np, int ntq, int nr,
+                                                double2* __restrict__ func) {
+  const int u = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (u >= nr * ntq * np) return;  // uniform per wave
+  const int p = u % np, q = u / np % ntq, r = u / (np * ntq);
+  const int4 qi = qinfo[q];
+  const double2* v = rho + (long long)r * rho_r + rho_off[q] + (long long)p * qi.y;
+  double f = 0.0, sh = 0.0;
+  for (int g = lane; g < qi.y; g += 64) {
+    const double2 a = v[g];
+    const double m = a.x * a.x + a.y * a.y;
+    f += m;
+    if (g >= qi.x) sh += m;
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    f += __shfl_xor(f, off);
+    sh += __shfl_xor(sh, off);
+  }
+  if (lane == 0) func[u] = make_double2(f, sh);
 }
 
 // X_ij(R) (slot w = nen) and J_ij(R, w) = 2*2pi sum_q f(q) / V / NTQ, heads on
-// i = j at R = 0 (calc_intJ.F:830-904).  One R: grid (nen + 1), threads over p.
-// out: X [p] and J [w * wstride + p] at this R's slot.
-__global__ void __launch_bounds__(64) k_j_sum(const double2* __restrict__ func,
-                                              const double2* __restrict__ funcw, int ntq, int nwf,
-                                              int nen, int r0, double volume, double chead,
-                                              const double2* __restrict__ cheadw,
-                                              double2* __restrict__ xmat,
-                                              double2* __restrict__ jmat, size_t wstride) {
-  const int w = blockIdx.x;
+// i = j at R = 0 (calc_intJ.F:830-904); f(q) is func, or the contraction's row
+// shares plus the shell.  grid (nen + 1, R of the batch), 256 threads: the q are
+// dealt to nq threads per pair and their sums meet in LDS, pair by pair in turn.
+// out: X [p] and J [w * wstride + p] at each R's slot.
+__global__ void __launch_bounds__(256) k_j_sum(const double2* __restrict__ func,
+                                               const double2* __restrict__ funcw, int ntq, int nwf,
+                                               int nen, int nr, int nrs,
+                                               const int* __restrict__ isr0, double volume,
+                                               double chead, const double2* __restrict__ cheadw,
+                                               double2* __restrict__ xmat,
+                                               double2* __restrict__ jmat, size_t wstride) {
+  const int w = blockIdx.x, r = blockIdx.y, np = nwf * nwf;
   const bool isx = w == nen;
-  const int np = nwf * nwf;
   const double tpi = 2.0 * 3.141592653589793238462643383279502884;
-  for (int p = threadIdx.x; p < np; p += blockDim.x) {
+  __shared__ double2 red[256];
+  const int pb = np < 256 ? np : 256, nq = 256 / pb;  // pairs at a time, threads per pair
+  for (int p0 = 0; p0 < np; p0 += pb) {
+    const int p = p0 + (int)threadIdx.x % pb, ql = (int)threadIdx.x / pb;
     double sr = 0.0, si = 0.0;
-    for (int q = 0; q < ntq; ++q) {
-      const double2 f = isx ? func[(size_t)q * np + p] : funcw[((size_t)q * nen + w) * np + p];
-      sr += f.x;
-      si += f.y;
-    }
-    double xr = 2.0 * tpi * sr / volume / (double)ntq, xi = 2.0 * tpi * si / volume / (double)ntq;
-    const bool diag = r0 && (p % nwf) == (p / nwf);
-    if (isx) {
-      if (diag) xr += chead;
-      xmat[p] = make_double2(xr, xi);
-    } else {
-      if (diag) { xr += cheadw[w].x; xi += cheadw[w].y; }
-      jmat[(size_t)w * wstride + p] = make_double2(xr, xi);
+    if (ql < nq && p < np)
+      for (int q = ql; q < ntq; q += nq) {
+        const double2 f = func[((size_t)r * ntq + q) * np + p];
+        if (isx) {
+          sr += f.x;
+        } else {
+          sr += f.y;
+          for (int s = 0; s < nrs; ++s) {
+            const double2 v = funcw[((((size_t)s * nr + r) * ntq + q) * nen + w) * np + p];
+            sr += v.x;
+            si += v.y;
+          }
+        }
+      }
+    __syncthreads();
+    red[threadIdx.x] = make_double2(sr, si);
+    __syncthreads();
+    if (ql == 0 && p < np) {
+      for (int k = 1; k < nq; ++k) {
+        sr += red[threadIdx.x + k * pb].x;
+        si += red[threadIdx.x + k * pb].y;
+      }
+      double xr = 2.0 * tpi * sr / volume / (double)ntq, xi = 2.0 * tpi * si / volume / (double)ntq;
+      const bool diag = isr0[r] && (p % nwf) == (p / nwf);
+      if (isx) {
+        if (diag) xr += chead;
+        xmat[(size_t)r * np + p] = make_double2(xr, xi);
+      } else {
+        if (diag) { xr += cheadw[w].x; xi += cheadw[w].y; }
+        jmat[(size_t)w * wstride + (size_t)r * np + p] = make_double2(xr, xi);
+      }
     }
   }
 }
@@ -602,35 +653,58 @@ void launch_w_contract(const float2* eps, const long long* eps_off, const double
   RP_HIP(hipGetLastError());
 }
 
+// Elements of X and of Z that a group of nge rows and ncol columns takes.
+size_t j_x_elems(int nge, int ncol) {
+  return (size_t)((nge + kJKC - 1) / kJKC * kJKC) * ((ncol + 15) / 16 * 16);
+}
+size_t j_z_elems(int nge, int ncol) { return (size_t)nge * ((ncol + 15) / 16 * 16); }
+
+// Shares of the row tiles (1..4): workgroups for a few rounds of four per CU.
+int j_row_shares(int ngroups, int nen, int max_ncol, int max_nge, int ncu) {
+  const long wgs = (long)ngroups * nen * ((max_ncol + kJT - 1) / kJT);
+  const int nat = (max_nge + kJT - 1) / kJT;
+  const long want = (4L * 4 * ncu + wgs - 1) / std::max(1L, wgs);
+  return (int)std::min<long>(std::min(4, nat), std::max(1L, want));
+}
+
+// groups: device array of ngroups {nge, iq_irr, first member, columns, X offset,
+// Z offset} as pack_j_groups lays them out; nr R of the batch, rho_r apart.
+size_t j_group_bytes() { return sizeof(JGroup); }
+void pack_j_group(void* at, int nge, int iqir, int mbeg, int ncol, long long xoff, long long zoff) {
+  *(JGroup*)at = JGroup{nge, iqir, mbeg, ncol, xoff, zoff};
+}
+
 void launch_j_contract(const float2* eps, const long long* eps_off, const double2* rho,
-                       const long long* rho_off, const int4* qinfo, const int* minv,
-                       const double2* pf1, const double2* pf2, const long long* map_off,
-                       double2* xg, const double2* shell, int ntq, int npair, int nen,
-                       double2* funcw, hipStream_t s) {
-  const int groups = (npair + 31) / 32;
-  const int g32 = 32 * groups;
-  hipLaunchKernelGGL(k_j_xvec, dim3(ntq), dim3(256), 0, s, rho, rho_off, qinfo, minv, pf1, pf2,
-                     map_off, npair, g32, xg);
-  hipLaunchKernelGGL(k_j_contract, dim3(nen, ntq, groups), dim3(512), 0, s, eps, eps_off, rho,
-                     rho_off, qinfo, minv, pf1, pf2, map_off, (const double2*)xg, g32, shell,
-                     npair, nen, funcw);
+                       const long long* rho_off, long long rho_r, const int4* qinfo,
+                       const int* minv, const double2* pf1, const double2* pf2,
+                       const long long* map_off, const void* groups, const int* gmem, int ngroups,
+                       int max_nge, int max_ncol, int npair, int nr, int nrs, int ntq, int nen,
+                       double2* xs, double2* zs, double2* funcw, hipStream_t s) {
+  RP_CHECK(ngroups >= 1 && ngroups <= 65535 && max_nge >= 1 && max_ncol >= 1,
+           "J contraction: bad group sizes");
+  const int cpad = (max_ncol + 15) / 16 * 16, nbp = (max_nge + kJKC - 1) / kJKC * kJKC;
+  hipLaunchKernelGGL(k_j_vecs, dim3((cpad + 31) / 32, (nbp + 31) / 32, ngroups), dim3(256), 0, s, rho,
+                     rho_off, rho_r, qinfo, minv, pf1, pf2, map_off, (const JGroup*)groups, gmem,
+                     npair, nr, xs, zs);
+  hipLaunchKernelGGL(k_j_contract, dim3(nen, ngroups, (cpad + kJT - 1) / kJT * nrs), dim3(256), 0, s,
+                     eps, eps_off, (const JGroup*)groups, gmem, (const double2*)xs,
+                     (const double2*)zs, npair, nr, nrs, ntq, nen, funcw);
   RP_HIP(hipGetLastError());
 }
 
-size_t j_contract_scratch(size_t sum_nge, int npair) { return sum_nge * 32 * ((npair + 31) / 32); }
-
-void launch_j_func(const double2* rho, const long long* rho_off, const int4* qinfo, int ntq,
-                   int npair, double2* func, double2* shell, hipStream_t s) {
-  hipLaunchKernelGGL(k_j_func, dim3(ntq, npair), dim3(256), 0, s, rho, rho_off, qinfo, npair, func,
-                     shell);
+void launch_j_func(const double2* rho, const long long* rho_off, long long rho_r, const int4* qinfo,
+                   int ntq, int npair, int nr, double2* func, hipStream_t s) {
+  const long units = (long)nr * ntq * npair;
+  hipLaunchKernelGGL(k_j_func, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, rho, rho_off, rho_r,
+                     qinfo, npair, ntq, nr, func);
   RP_HIP(hipGetLastError());
 }
 
-void launch_j_sum(const double2* func, const double2* funcw, int ntq, int nwf, int nen, int r0,
-                  double volume, double chead, const double2* cheadw, double2* xmat,
+void launch_j_sum(const double2* func, const double2* funcw, int ntq, int nwf, int nen, int nr, int nrs,
+                  const int* isr0, double volume, double chead, const double2* cheadw, double2* xmat,
                   double2* jmat, size_t wstride, hipStream_t s) {
-  hipLaunchKernelGGL(k_j_sum, dim3(nen + 1), dim3(64), 0, s, func, funcw, ntq, nwf, nen, r0, volume,
-                     chead, cheadw, xmat, jmat, wstride);
+  hipLaunchKernelGGL(k_j_sum, dim3(nen + 1, nr), dim3(256), 0, s, func, funcw, ntq, nwf, nen, nr, nrs,
+                     isr0, volume, chead, cheadw, xmat, jmat, wstride);
   RP_HIP(hipGetLastError());
 }
 
