@@ -22,43 +22,42 @@
 namespace rp {
 
 // Per q: func (all G of the psi list) and the shell part of funcw (G beyond the
-// eps sphere).  grid: ntq blocks of 256; out [q][j][i].
+// eps sphere).  A wave per (q, i <= j), its lanes along G; (j, i) is the complex
+// conjugate.  out [q][j][i].  64 q of five functions: 6 us, against 82 us of one
+// workgroup per q that took the pairs in turn.
 __global__ void __launch_bounds__(256) k_w_func(const double2* __restrict__ rho,
                                                 const long long* __restrict__ rho_off,
-                                                const int4* __restrict__ qinfo, int nwf,
+                                                const int4* __restrict__ qinfo, int nwf, int ntq,
                                                 double2* __restrict__ func,
                                                 double2* __restrict__ shell) {
-  const int q = blockIdx.x;
+  const int np = nwf * (nwf + 1) / 2;
+  const int u = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (u >= ntq * np) return;  // uniform per wave
+  const int q = u / np;
+  int i = u % np, j = 0;
+  while (i > j) i -= ++j;  // u % np = j (j + 1) / 2 + i, i <= j
   const int4 qi = qinfo[q];  // (ng_eps, ng_psi, iq_irr, trs)
-  const double2* r = rho + rho_off[q];
   const int ngpsi = qi.y, nge = qi.x;
-  __shared__ double red[256];
-  for (int ij = 0; ij < nwf * nwf; ++ij) {
-    const int i = ij % nwf, j = ij / nwf;
-    const double2* ri = r + (size_t)i * ngpsi;
-    const double2* rj = r + (size_t)j * ngpsi;
-    double f[4] = {0, 0, 0, 0};  // func re/im, shell re/im
-    for (int g = threadIdx.x; g < ngpsi; g += blockDim.x) {
-      const double2 a = ri[g], b = rj[g];
-      const double pr = a.x * b.x + a.y * b.y, pi = a.y * b.x - a.x * b.y;  // a conj(b)
-      f[0] += pr;
-      f[1] += pi;
-      if (g >= nge) { f[2] += pr; f[3] += pi; }
-    }
+  const double2* ri = rho + rho_off[q] + (size_t)i * ngpsi;
+  const double2* rj = rho + rho_off[q] + (size_t)j * ngpsi;
+  double f[4] = {0, 0, 0, 0};  // func re/im, shell re/im
+  for (int g = lane; g < ngpsi; g += 64) {
+    const double2 a = ri[g], b = rj[g];
+    const double pr = a.x * b.x + a.y * b.y, pi = a.y * b.x - a.x * b.y;  // a conj(b)
+    f[0] += pr;
+    f[1] += pi;
+    if (g >= nge) { f[2] += pr; f[3] += pi; }
+  }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      red[threadIdx.x] = f[c];
-      __syncthreads();
-      for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-        __syncthreads();
-      }
-      if (threadIdx.x == 0) {
-        double2* o = (c < 2 ? func : shell) + ((size_t)q * nwf + j) * nwf + i;
-        if (c % 2 == 0) o->x = red[0];
-        else o->y = red[0];
-      }
-      __syncthreads();
+  for (int c = 0; c < 4; ++c)
+    for (int off = 32; off > 0; off >>= 1) f[c] += __shfl_xor(f[c], off);
+  if (lane == 0) {
+    const size_t ij = ((size_t)q * nwf + j) * nwf + i, ji = ((size_t)q * nwf + i) * nwf + j;
+    func[ij] = make_double2(f[0], f[1]);
+    shell[ij] = make_double2(f[2], f[3]);
+    if (i != j) {
+      func[ji] = make_double2(f[0], -f[1]);
+      shell[ji] = make_double2(f[2], -f[3]);
     }
   }
 }
@@ -85,13 +84,14 @@ typedef double jd4 __attribute__((ext_vector_type(4)));
 constexpr int kMaxWf = 16;     // Wannier functions of calc_w3d and calc_j3d
 constexpr int kWcVec = 16;     // vectors of a group: one MFMA column block
 constexpr int kWA = 3;         // row blocks per wave and pass of the W contraction
+constexpr int kWD = 2;         // steps its loads run ahead
 template <int NV>
 constexpr int wc_members() { return kWcVec / NV; }
 int w_contract_members(int nwf) { return kWcVec / nwf; }
 int w_contract_vectors(int) { return kWcVec; }
 
 // X_c(b) of every group, [nge][vb] at xw + vb * map_off[first member] (zero
-// past the group's vectors).  grid: ngroups, 256 threads.
+// past the group's vectors).  grid: (ceil(largest nge / 16), ngroups), 256 threads.
 __global__ void __launch_bounds__(256) k_w_xvec(const double2* __restrict__ rho,
                                                 const long long* __restrict__ rho_off,
                                                 const int4* __restrict__ qinfo,
@@ -102,12 +102,13 @@ __global__ void __launch_bounds__(256) k_w_xvec(const double2* __restrict__ rho,
                                                 const int* __restrict__ goff,
                                                 const int* __restrict__ gmem, int nv, int vb,
                                                 double2* __restrict__ xw) {
-  const int grp = blockIdx.x;
+  const int grp = blockIdx.y;
   const int mbeg = goff[grp], nvt = (goff[grp + 1] - mbeg) * nv;
   const int q0 = gmem[mbeg];
   const int nge = qinfo[q0].x;
   double2* out = xw + map_off[q0] * vb;
-  for (int e = threadIdx.x; e < vb * nge; e += blockDim.x) {
+  const int e1 = min(vb * nge, ((int)blockIdx.x + 1) * 16 * vb);
+  for (int e = (int)blockIdx.x * 16 * vb + (int)threadIdx.x; e < e1; e += blockDim.x) {
     const int b = e / vb, c = e % vb;
     double2 v = make_double2(0.0, 0.0);
     if (c < nvt) {
@@ -159,43 +160,46 @@ __global__ void __launch_bounds__(512) k_w_contract(
   // up to kWA row blocks per wave and pass (ab = a0 + wave + 8 j) share each
   // load of X; blocks past the last are skipped (uniform per wave)
   for (int a0 = 0; a0 < nab; a0 += 8 * kWA) {
-    jd4 accr[kWA], acci[kWA];
+    jd4 t1[kWA], t2[kWA], t3[kWA];
     int arow[kWA];
 #pragma unroll
     for (int j = 0; j < kWA; ++j) {
-      accr[j] = acci[j] = jd4{0.0, 0.0, 0.0, 0.0};
+      t1[j] = t2[j] = t3[j] = jd4{0.0, 0.0, 0.0, 0.0};
       // rows nge .. ld-1 are the zero padding; their sums are never used
       arow[j] = (a0 + wave + 8 * j) * 16 + li;
     }
     const int nj = min(kWA, (nab - a0 - wave + 7) / 8);  // live blocks of this wave
-    // the next step's X and E are loaded during this step's MFMAs (the last
-    // step loads itself again); columns past nge contribute zero
-    int bn = lk < nge ? lk : nge - 1;
-    double2 xn = Xg[(size_t)bn * kWcVec + li];
-    float2 en[kWA];
+    // X and E of the step kWD steps ahead are loaded during a step's MFMAs;
+    // columns past nge contribute zero
+    double2 xq[kWD];
+    float2 eq[kWD][kWA];
+    auto fetch = [&](int b0, int slot) {
+      const int b = min(b0 + lk, nge - 1);
+      xq[slot] = Xg[(size_t)b * kWcVec + li];
 #pragma unroll
-    for (int j = 0; j < kWA; ++j) en[j] = j < nj ? E[(size_t)bn * ld + arow[j]] : make_float2(0.f, 0.f);
-    for (int b0 = 0; b0 < nge; b0 += 4) {
-      const bool bv = b0 + lk < nge;
-      const double2 xv = xn;
-      float2 ec[kWA];
+      for (int j = 0; j < kWA; ++j) eq[slot][j] = j < nj ? E[(size_t)b * ld + arow[j]] : make_float2(0.f, 0.f);
+    };
 #pragma unroll
-      for (int j = 0; j < kWA; ++j) ec[j] = en[j];
-      const int b1 = (b0 + 4 < nge ? b0 + 4 : b0) + lk;
-      bn = b1 < nge ? b1 : nge - 1;
-      xn = Xg[(size_t)bn * kWcVec + li];
+    for (int d = 0; d < kWD; ++d) fetch(4 * d, d);
+    for (int b0 = 0; b0 < nge; b0 += 4 * kWD) {
 #pragma unroll
-      for (int j = 0; j < kWA; ++j)
-        if (j < nj) en[j] = E[(size_t)bn * ld + arow[j]];
-      const double xr = bv ? xv.x : 0.0, xi = bv ? xv.y : 0.0, nxi = -xi;
+      for (int d = 0; d < kWD; ++d) {
+        const bool bv = b0 + 4 * d + lk < nge;
+        const double xr = bv ? xq[d].x : 0.0, xi = bv ? xq[d].y : 0.0, xs = xr + xi;
+        double er[kWA], ei[kWA];
 #pragma unroll
-      for (int j = 0; j < kWA; ++j) {
-        if (j >= nj) break;  // uniform
-        const double er = ec[j].x, ei = ec[j].y;
-        accr[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er, xr, accr[j], 0, 0, 0);
-        accr[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei, nxi, accr[j], 0, 0, 0);
-        acci[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er, xi, acci[j], 0, 0, 0);
-        acci[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei, xr, acci[j], 0, 0, 0);
+        for (int j = 0; j < kWA; ++j) {
+          er[j] = eq[d][j].x;
+          ei[j] = eq[d][j].y;
+        }
+        fetch(b0 + 4 * (d + kWD), d);
+#pragma unroll
+        for (int j = 0; j < kWA; ++j) {
+          if (j >= nj) break;  // uniform
+          t1[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[j], xr, t1[j], 0, 0, 0);
+          t2[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[j], xi, t2[j], 0, 0, 0);
+          t3[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[j] + ei[j], xs, t3[j], 0, 0, 0);
+        }
       }
     }
     // Z_i(a) Y(a, c) for this lane's rows a = 16 ab + lk + 4 v and vector c = li
@@ -209,7 +213,7 @@ __global__ void __launch_bounds__(512) k_w_contract(
           const int ar = ab * 16 + lk + 4 * v;
           if (ar >= nge) continue;
           const int g = minv[mom + ar];
-          const double yr = accr[j][v], yi = acci[j][v];
+          const double yr = t1[j][v] - t2[j][v], yi = t3[j][v] - t1[j][v] - t2[j][v];
           const double2 pp = qim.w == 1 ? pf1[mom + g] : pf2[mom + g];
 #pragma unroll
           for (int i = 0; i < NV; ++i) {
@@ -624,7 +628,9 @@ int w3d_max_wannier() { return kMaxWf; }
 
 void launch_w_func(const double2* rho, const long long* rho_off, const int4* qinfo, int ntq,
                    int nwf, double2* func, double2* shell, hipStream_t s) {
-  hipLaunchKernelGGL(k_w_func, dim3(ntq), dim3(256), 0, s, rho, rho_off, qinfo, nwf, func, shell);
+  const int units = ntq * (nwf * (nwf + 1) / 2);
+  hipLaunchKernelGGL(k_w_func, dim3((units + 3) / 4), dim3(256), 0, s, rho, rho_off, qinfo, nwf, ntq, func,
+                     shell);
   RP_HIP(hipGetLastError());
 }
 
@@ -637,7 +643,7 @@ void launch_w_contract(const float2* eps, const long long* eps_off, const double
   RP_CHECK(nwf >= 1 && nwf <= kMaxWf, "W contraction supports 1..16 Wannier functions");
   RP_CHECK(max_nge >= 1, "W contraction: empty eps sphere");
   if (ngroups <= 0) return;
-  hipLaunchKernelGGL(k_w_xvec, dim3(ngroups), dim3(256), 0, s, rho, rho_off, qinfo, minv, pf1,
+  hipLaunchKernelGGL(k_w_xvec, dim3((max_nge + 15) / 16, ngroups), dim3(256), 0, s, rho, rho_off, qinfo, minv, pf1,
                      pf2, map_off, goff, gmem, nwf, w_contract_vectors(nwf), xw);
   switch (nwf) {
 #define RP_WC(NV)                                                                             \
