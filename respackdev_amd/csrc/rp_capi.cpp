@@ -584,9 +584,13 @@ void issue_weights(rp_ctx* h) {
   grow(h, h->d_w, (size_t)h->nen * h->kpad, "weight buffer");
   launch_zero(h->d_w.p, sizeof(double2) * h->nen * h->kpad, s);
   if (!h->capturing) launch_zero(h->d_status.p, sizeof(int), s);
+  int ncut = 0;  // pairs whose tetrahedra the Fermi level can cut
+  if (h->n_pocc > 0)
+    for (int p = 0; p < h->npair; ++p)
+      ncut += h->win[h->pocc[p]] == 1 || h->win[h->pvir[p]] == 1;
   launch_tetra_weights(h->ntk, h->nkb[0], h->nkb[1], h->nkb[2], h->d_imt.p, h->d_index.p, h->d_pocc.p,
                        h->d_pvir.p, h->d_ikq.p, h->d_eband.p, h->d_pband.p, h->ef, h->delt, h->dmna,
-                       h->dmnr, h->nen, h->d_em.p, h->kpad, h->npair, h->n_pocc > 0 ? 1 : 0,
+                       h->dmnr, h->nen, h->d_em.p, h->kpad, h->npair, ncut, h->ncu,
                        h->d_status.p, h->d_w.p, s);
 }
 

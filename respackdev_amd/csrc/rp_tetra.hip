@@ -829,14 +829,23 @@ __device__ __forceinline__ bool node_kept(const CutNode& n, const double (&val)[
 //
 // A plane moves one more vertex onto itself with every cut and needs two
 // unmoved vertices to cut again, so a tree has at most 3 cut levels per plane:
-// at most 2^6 pieces.  Each thread owns one tetrahedron and walks the leaves
-// of its tree depth first, rebuilding each from the root along its path of
-// child bits, so the pieces never need storage; both signs dsgn share the
-// pieces and the degeneracy class (chk1 depends on |g_p - g_q| and |g_p + g_q|).
+// at most 2^6 pieces.  Each thread owns one tetrahedron at a time and walks the
+// leaves of its tree depth first, rebuilding each from the root along its path
+// of child bits; both signs dsgn share the pieces and the degeneracy class (chk1
+// depends on |g_p - g_q| and |g_p + g_q|).  The walk only lists pieces in LDS; when
+// the list is nearly full, the block's threads share its (piece, frequency) pairs
+// evenly.  The closed forms take nearly all of the time, and a thread that did all
+// those of its tetrahedron would have the block wait for the few that have dozens
+// of pieces: with both kernels, a metal of 500 pairs, 20 frequencies and 64 k took
+// 3.30 ms so and 0.95 ms with the list, one of 660 pairs, 27 frequencies and 27 k
+// 9.3 and 1.05 ms.
 //
-// grid as k_tetra_weights, which must have run first: the pieces are added
-// to the weights it wrote, with the same 1/NTK and cRPA factor.  Status bit 2
-// as there; bit 8 if a tree had more leaves than the bound (cannot happen).
+// grid (npair, slices of nf frequencies).  k_tetra_weights must have run first: the
+// pieces are added to the weights it wrote, with the same 1/NTK and cRPA factor.
+// Status bit 2 as there; bit 8 if a tree had more leaves than the bound (cannot
+// happen).
+constexpr int kPieces = 256;  // the LDS list's length
+
 __global__ void __launch_bounds__(256) k_tetra_cut(
     int ntk, int n1, int n2, int n3, const int* __restrict__ imt,
     const int* __restrict__ index_kpt, const int* __restrict__ pocc,
@@ -850,8 +859,11 @@ __global__ void __launch_bounds__(256) k_tetra_cut(
   double2* x = lds;                              // [nk3][nf]
   double* e1 = (double*)(x + (size_t)nk3 * nf);  // [nk3]
   double* e2 = e1 + nk3;                         // [nk3]
-  int* list = (int*)(e2 + nk3);                  // [ntet]
-  __shared__ int count;
+  double* pr = e2 + nk3;                         // [17][kPieces]: r[v][c], volume of a piece
+  int2* pc = (int2*)(pr + 17 * kPieces);         // [kPieces]: its tetrahedron and class
+  int* list = (int*)(pc + kPieces);              // [ntet]
+  __shared__ int count, npiece, nbusy;
+  if (threadIdx.x == 0) npiece = 0;
   const int p = blockIdx.x;
   const int f0 = blockIdx.y * nf, nfb = min(nf, nen - f0);
   const int jo = pocc[p], iv = pvir[p];
@@ -872,19 +884,17 @@ __global__ void __launch_bounds__(256) k_tetra_cut(
   __syncthreads();
   const int ncut = count;
   if (ncut == 0) return;  // uniform over the block
-  for (int j = threadIdx.x; j < ncut; j += blockDim.x) {
-    const int t = list[j];
-    const int c0 = imt[4 * t], c1 = imt[4 * t + 1], c2 = imt[4 * t + 2], c3 = imt[4 * t + 3];
-    const double de2[4] = {e2[c0], e2[c1], e2[c2], e2[c3]};
-    const double de1[4] = {e1[c0], e1[c1], e1[c2], e1[c3]};
-    double2* y0 = x + (size_t)c0 * nf;
-    double2* y1 = x + (size_t)c1 * nf;
-    double2* y2 = x + (size_t)c2 * nf;
-    double2* y3 = x + (size_t)c3 * nf;
-    unsigned path = 0;
-    bool more = true;
-#pragma unroll 1
-    for (int leaf = 0; leaf < 64 && more; ++leaf) {
+  int j = threadIdx.x, leaf = 0;  // this thread's tetrahedron and leaf
+  unsigned path = 0;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) nbusy = 0;
+    __syncthreads();
+    if (j < ncut) {
+      const int t = list[j];
+      const int c0 = imt[4 * t], c1 = imt[4 * t + 1], c2 = imt[4 * t + 2], c3 = imt[4 * t + 3];
+      const double de2[4] = {e2[c0], e2[c1], e2[c2], e2[c3]};
+      const double de1[4] = {e1[c0], e1[c1], e1[c2], e1[c3]};
       CutNode n;
 #pragma unroll
       for (int v = 0; v < 4; ++v)
@@ -920,6 +930,7 @@ __global__ void __launch_bounds__(256) k_tetra_cut(
           }
         }
       }
+      bool taken = true;  // false: the list is full, the same leaf again next round
       if (keep) {
         double s[4];
 #pragma unroll
@@ -931,39 +942,79 @@ __global__ void __launch_bounds__(256) k_tetra_cut(
         if ((code & 15) == kBad) {
           atomicOr(status, 2);
         } else {
-#pragma unroll 1
-          for (int f = 0; f < nfb; ++f) {
-            const zd e = mkz(em[f0 + f].x, em[f0 + f].y);
-            zd T0 = mkz(0, 0), T1 = mkz(0, 0), T2 = mkz(0, 0), T3 = mkz(0, 0);
-#pragma unroll 1
-            for (int sg = 0; sg < 2; ++sg) {  // dsgn = +1, then -1: g -> -g, f -> -f
-              const double ds = sg == 0 ? 1.0 : -1.0;
-              zd t0, t1, t2, t3;
-              calc_terms(code, g[0] * ds, g[1] * ds, g[2] * ds, g[3] * ds, e, t0, t1, t2, t3);
-              T0 = T0 + t0 * ds;
-              T1 = T1 + t1 * ds;
-              T2 = T2 + t2 * ds;
-              T3 = T3 + t3 * ds;
-            }
-            T0 = T0 * n.vol;
-            T1 = T1 * n.vol;
-            T2 = T2 * n.vol;
-            T3 = T3 * n.vol;
-            // corner c: sum_v T_v dwgt(c, v)
-            lds_add(y0 + f, T0 * n.r[0][0] + T1 * n.r[1][0] + T2 * n.r[2][0] + T3 * n.r[3][0]);
-            lds_add(y1 + f, T0 * n.r[0][1] + T1 * n.r[1][1] + T2 * n.r[2][1] + T3 * n.r[3][1]);
-            lds_add(y2 + f, T0 * n.r[0][2] + T1 * n.r[1][2] + T2 * n.r[2][2] + T3 * n.r[3][2]);
-            lds_add(y3 + f, T0 * n.r[0][3] + T1 * n.r[1][3] + T2 * n.r[2][3] + T3 * n.r[3][3]);
+          const int i = atomicAdd(&npiece, 1);
+          taken = i < kPieces;
+          if (taken) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+              for (int c = 0; c < 4; ++c) pr[(4 * v + c) * kPieces + i] = n.r[v][c];
+            pr[16 * kPieces + i] = n.vol;
+            pc[i] = make_int2(t, code);
           }
         }
       }
       // next leaf in depth-first order: flip the deepest 0 bit of the path
       int b = depth - 1;
       while (b >= 0 && ((path >> b) & 1u)) --b;
-      if (b < 0) more = false;
-      else path = (path & ((1u << b) - 1u)) | (1u << b);
+      if (!taken) {
+      } else if (b >= 0 && ++leaf < 64) {
+        path = (path & ((1u << b) - 1u)) | (1u << b);
+      } else {
+        if (b >= 0) atomicOr(status, 8);
+        j += blockDim.x;
+        leaf = 0;
+        path = 0;
+      }
+      if (j < ncut) nbusy = 1;
     }
-    if (more) atomicOr(status, 8);
+    __syncthreads();
+    const bool more = nbusy != 0;  // uniform, as np
+    const int np = min(npiece, kPieces);
+    if (more && np < 3 * kPieces / 4) continue;
+    for (int u = threadIdx.x; u < np * nfb; u += blockDim.x) {
+      const int i = u / nfb, f = u % nfb;
+      const int2 tc = pc[i];
+      const int t = tc.x;
+      const int c0 = imt[4 * t], c1 = imt[4 * t + 1], c2 = imt[4 * t + 2], c3 = imt[4 * t + 3];
+      const double d0 = e2[c0] - e1[c0], d1 = e2[c1] - e1[c1], d2 = e2[c2] - e1[c2],
+                   d3 = e2[c3] - e1[c3];
+      double sv[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        sv[v] = d0 * pr[(4 * v) * kPieces + i] + d1 * pr[(4 * v + 1) * kPieces + i] +
+                d2 * pr[(4 * v + 2) * kPieces + i] + d3 * pr[(4 * v + 3) * kPieces + i];
+      const zd e = mkz(em[f0 + f].x, em[f0 + f].y);
+      zd T0 = mkz(0, 0), T1 = mkz(0, 0), T2 = mkz(0, 0), T3 = mkz(0, 0);
+#pragma unroll 1
+      for (int sg = 0; sg < 2; ++sg) {  // dsgn = +1, then -1: g -> -g, f -> -f
+        const double ds = sg == 0 ? 1.0 : -1.0;
+        zd t0, t1, t2, t3;
+        calc_terms(tc.y, mkz(-sv[0], delt) * ds, mkz(-sv[1], delt) * ds, mkz(-sv[2], delt) * ds,
+                   mkz(-sv[3], delt) * ds, e, t0, t1, t2, t3);
+        T0 = T0 + t0 * ds;
+        T1 = T1 + t1 * ds;
+        T2 = T2 + t2 * ds;
+        T3 = T3 + t3 * ds;
+      }
+      const double vol = pr[16 * kPieces + i];
+      T0 = T0 * vol;
+      T1 = T1 * vol;
+      T2 = T2 * vol;
+      T3 = T3 * vol;
+      // corner c: sum_v T_v dwgt(c, v)
+      auto corner = [&](int c, int k) {
+        lds_add(x + (size_t)k * nf + f, T0 * pr[c * kPieces + i] + T1 * pr[(4 + c) * kPieces + i] +
+                                            T2 * pr[(8 + c) * kPieces + i] + T3 * pr[(12 + c) * kPieces + i]);
+      };
+      corner(0, c0);
+      corner(1, c1);
+      corner(2, c2);
+      corner(3, c3);
+    }
+    __syncthreads();
+    if (!more) break;
+    if (threadIdx.x == 0) npiece = 0;  // no one adds before the next barrier
   }
   __syncthreads();
   const double inv_ntk = 1.0 / (double)ntk;
@@ -1099,24 +1150,31 @@ size_t tetra_lds_bytes(int nk3, int nf) {
          sizeof(int2) * 6 * (size_t)nk3 + sizeof(int) * (size_t)tetra_queue_len(nk3, nf);
 }
 
-// Frequencies per workgroup: as many as keep two workgroups per CU (the
-// register budget allows two waves per SIMD), evened out over the slices.
-int tetra_freqs_per_block(int nk3, int nen) {
+// Frequencies per workgroup: as many as keep two workgroups per CU by LDS (the
+// register budget allows two waves per SIMD), and few enough that the pairs'
+// slices make five workgroups per CU, evened out over the slices.  A workgroup
+// is a chain of long FP64 closed forms, so few of them leave the chip idle:
+// 6 pairs of 14 frequencies on 8 k 93 us with one slice, 44 with 14; 192 pairs of
+// 16 on 64 k 358 and 192 us; 20 of 16 on 125 k 311 and 99 us; from about 1000
+// workgroups on more slices only repeat the classification and the logarithms
+// (2448 pairs of 19: 257 us with one, 331 with five).
+int tetra_freqs_per_block(int nk3, int nen, int npair, int ncu) {
   const size_t fixed = tetra_lds_bytes(nk3, 0), per = tetra_lds_bytes(nk3, 1) - fixed;
   const size_t target = 80 * 1024;
   int nf = target > fixed ? (int)((target - fixed) / per) : 1;
   nf = std::max(1, std::min(nf, nen));
-  const int nslice = (nen + nf - 1) / nf;
+  const int fill = std::min(nen, (5 * ncu + npair - 1) / npair);
+  const int nslice = std::max((nen + nf - 1) / nf, fill);
   return (nen + nslice - 1) / nslice;
 }
 
 void launch_tetra_weights(int ntk, int n1, int n2, int n3, const int* imt, const int* index_kpt,
                           const int* pocc, const int* pvir, const int* ikq, const double* eband,
                           const double2* pband, double ef, double delt, double dmna, double dmnr,
-                          int nen, const double2* em, size_t ldd, int npair, int cuts, int* status,
-                          double2* dout, hipStream_t s) {
+                          int nen, const double2* em, size_t ldd, int npair, int ncut, int ncu,
+                          int* status, double2* dout, hipStream_t s) {
   const int nk3 = n1 * n2 * n3;
-  const int nf = tetra_freqs_per_block(nk3, nen);
+  int nf = tetra_freqs_per_block(nk3, nen, npair, ncu);
   const size_t lds = tetra_lds_bytes(nk3, nf);
   RP_CHECK(lds <= 160 * 1024, "k mesh too large for the LDS accumulator of the tetrahedron kernel");
   if (lds > 65536)
@@ -1125,16 +1183,22 @@ void launch_tetra_weights(int ntk, int n1, int n2, int n3, const int* imt, const
   const dim3 grid(npair, (nen + nf - 1) / nf);
   hipLaunchKernelGGL(k_tetra_weights, grid, dim3(256), lds, s, ntk, n1, n2, n3, imt, index_kpt,
                      pocc, pvir, ikq, eband, pband, ef, delt, dmna, dmnr, nen, nf, em, ldd,
-                     cuts ? 1 : 0, tetra_queue_len(nk3, nf), status, dout);
+                     ncut > 0 ? 1 : 0, tetra_queue_len(nk3, nf), status, dout);
   RP_HIP(hipGetLastError());
-  if (!cuts) return;
-  // x[nk3][nf], e1, e2, the cut list (<= lds of the uncut kernel)
+  if (ncut == 0) return;
+  // Only the pairs with a partially occupied band have pieces: slices of their own,
+  // as many as give those pairs the two workgroups per CU that the registers allow
+  // (500 pairs, 96 of them cut, 20 frequencies on 64 k: 0.92 ms for 1 to 3
+  // slices, 0.98 for 6; 660, 102, 27 on 27 k: 1.61, 1.31 and 1.01).
+  nf = std::min(nf, std::max(1, nen * ncut / (2 * ncu)));
+  // x[nk3][nf], e1, e2, the pieces of a round and the cut list
   const size_t lcut = sizeof(double2) * (size_t)nk3 * nf + 2 * sizeof(double) * (size_t)nk3 +
-                      sizeof(int) * 6 * (size_t)nk3;
+                      (17 * sizeof(double) + sizeof(int2)) * kPieces + sizeof(int) * 6 * (size_t)nk3;
+  RP_CHECK(lcut <= 160 * 1024, "k mesh too large for the LDS accumulator of the cut tetrahedra");
   if (lcut > 65536)
     RP_HIP(hipFuncSetAttribute((const void*)k_tetra_cut,
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lcut));
-  hipLaunchKernelGGL(k_tetra_cut, grid, dim3(256), lcut, s, ntk, n1, n2, n3, imt, index_kpt, pocc,
+  hipLaunchKernelGGL(k_tetra_cut, dim3(npair, (nen + nf - 1) / nf), dim3(256), lcut, s, ntk, n1, n2, n3, imt, index_kpt, pocc,
                      pvir, ikq, eband, pband, ef, delt, dmna, dmnr, nen, nf, em, ldd, status, dout);
   RP_HIP(hipGetLastError());
 }
