@@ -4,13 +4,11 @@
 //
 // The inversion is Gauss-Jordan with partial pivoting by |Re|+|Im| (the pivot
 // rule of LAPACK's izamax in zgetrf, which the reference calls through
-// invZGE.F90:1-23), blocked by panels of up to 16 columns: one workgroup per
-// matrix factors a panel (in registers for n <= 768, else in LDS), a batched
-// kernel applies the panel's rank-nb update to all other columns (for n <= 768
-// in the same launch as the factoring of the next panel), and a final kernel
-// undoes the row interchanges as column swaps.
+// invZGE.F90:1-23), blocked by panels: one workgroup per matrix factors a panel (for
+// n <= 768 32 columns in registers, else up to 16 in LDS), a batched kernel applies
+// the panel's transform to all other columns (for n <= 768 in the same launch as the
+// factoring of the next panel), and a final kernel puts the columns in order.
 #include <algorithm>
-
 #include <utility>
 
 #include "rp_common.h"
@@ -190,26 +188,51 @@ __global__ void __launch_bounds__(1024) k_gj_panel(double2* __restrict__ a, int 
   if (tid == 0) mv[0] = singular ? -1 : nb + nmove;
 }
 
-// The same panel step for full panels (nb = 16) of n <= 768 rows, with the
-// panel in registers: thread i starts with row i of the 16 panel columns.  The
-// 16 column steps are expanded at compile time (gj_reg_step<L>), so every
-// register index is a constant.  Rows are never exchanged between threads:
-// each thread carries the matrix row it holds (lr), the pivot search takes the
-// largest |Re|+|Im| over rows lr >= c with the smallest row on ties (izamax),
-// and the interchange of rows c and p only swaps the two threads' row numbers.
-// The pivot row goes to the others through LDS: two barriers per column.  The
-// elimination multiplies by 1/piv once per row, r - (r_L/piv) rowp, where
-// k_gj_panel scales the pivot row first, r - r_L (rowp/piv): the same
-// arithmetic up to the order of one product.  The rows go back to the matrix at
-// their row numbers (gj_reg_store).
-struct GjRegShared {
-  double wv[16];
-  int wi[16];
-  double2 rowp[kPanelMax];
-  double2 pinv;  // 1/piv, formed by the pivot row's thread
-  int orig[768];
-  int origb[768];  // the rows' sources since the last reset (one half of a 32-column panel)
-  int nmove;
+// ---------------------------------------------------------------------------
+// n <= 768: steps of 32 columns.  Each launch applies the rank-32 transform of
+// one 32-column panel to every other column; one block per matrix brings the
+// next panel up to date and factors it in the same launch (look-ahead), as two
+// halves of 16 columns in registers: half A, half B after A's transform, then A
+// after B's.  The transform of the two halves together differs from the identity
+// in the panel's columns only, so every other column j becomes
+//   a'(:,j) = P a(:,j) with the panel rows zeroed + W (P a)(panel rows, j),
+// W the panel's final columns and P the panel's row interchanges (B's act on
+// rows below A's panel rows only, so A's transform commutes past them).  The last
+// panel is as narrow as what is left of the columns.
+//
+// The panel blocks are the critical path: 32 column steps one after the other,
+// each about 2400 clocks of latency (pivot search 300, reciprocal 200, offering the
+// candidates' rows and meeting at the barrier 800, comparing them 300, the rank-1
+// update 700 to 850).  A thread holds R rows (256 R >= n), so that a block has four
+// waves, one per SIMD, which meet quickly and take the update's time together.
+// Rows are not exchanged between threads: a thread keeps the number lr of the
+// matrix row that its values are (-1: no row), and an interchange swaps the
+// numbers.  Per launch, 16 to 24 matrices, with a thread per row, two barriers per
+// column and the update on the vector unit before: NG 106, first panel 64 -> 49 us,
+// a step 59 -> 35; NG 586, 100 -> 85 and 146 -> 120 us.  The last panel in the same
+// way instead of by k_gj_panel and k_gj_update: NG 17, all of it, 75 -> 28 us; NG 586
+// 107 -> 38 us of one step that has no next panel.
+constexpr int kSuper = 32;
+constexpr int kHalf = 16;
+constexpr int kMoveMax32 = 2 * kSuper;           // panel rows and rows they displaced
+constexpr int kMoveInts32 = 1 + 2 * kMoveMax32;  // {count, dst[64], src[64]}
+constexpr int kGjThreads = 256;
+constexpr int kGjRows = 768;
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+struct GjShared {
+  // every wave's candidate for the pivot, by the parity of the column: |Re|+|Im|, the
+  // row's number, its reciprocal and its other columns
+  double2 wv[2][2];
+  int4 wi[2];
+  double2 rowp[2][4][kHalf];
+  int orig[kGjRows];   // the row whose content is now in row i: by the panel, by its half B
+  int orig2[kGjRows];
+  short slot[kGjRows];  // where row i comes from: -1 itself, -2 zero (panel row), e: vals[e]
+  double2 vals[kMoveMax32][kSuper];  // old values of the moved rows
+  int dst[kMoveMax32], src[kMoveMax32];
+  int nm;
   int singular;
 };
 
@@ -230,413 +253,355 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// A zero pivot sets the matrix's status bit and sh.singular and the steps go
-// on (on values that are then discarded): every thread runs the same steps and
-// meets the same barriers, and no branch keeps an older copy of the registers.
-template <int L>
-__device__ __forceinline__ void gj_reg_step(double2 (&r)[kPanelMax], int& lr, GjRegShared& sh,
-                                            int i, int n, int c0, bool mine, int b,
-                                            int* __restrict__ ipiv, int* __restrict__ status) {
-  constexpr int NB = kPanelMax;
-  const int lane = i & 63, wave = i >> 6, nwave = (int)(blockDim.x >> 6);
-  const int c = c0 + L;
-  // pivot: largest |Re|+|Im| in rows c..n-1, first row on ties (izamax)
-  const double own = (mine && lr >= c) ? fabs(r[L].x) + fabs(r[L].y) : -1.0;
+// Lane Q of every row of 16 lanes, in all of them.
+template <int Q>
+__device__ __forceinline__ double2 gj_bcast(double2 v) {
+  return make_double2(__builtin_amdgcn_update_dpp(0.0, v.x, 0x150 + Q, 0xf, 0xf, false),
+                      __builtin_amdgcn_update_dpp(0.0, v.y, 0x150 + Q, 0xf, 0xf, false));
+}
+
+// Columns 1.. of the rows less f times the pivot row (entry q in lane q), moved up
+// by one.
+template <int R, int... Q>
+__device__ __forceinline__ void gj_rank1(std::integer_sequence<int, Q...>,
+                                         double2 (&r)[R][kHalf], const double2 (&f)[R], double2 v) {
+  (
+      [&] {
+        const double2 u = gj_bcast<Q + 1>(v);
+#pragma unroll
+        for (int k = 0; k < R; ++k) r[k][Q] = cfms(r[k][Q + 1], f[k], u);
+      }(),
+      ...);
+}
+
+// 1/z by Smith's scaling without a branch.
+__device__ __forceinline__ double2 gj_inv(double2 z) {
+  const bool xb = fabs(z.x) >= fabs(z.y);
+  const double g = xb ? z.x : z.y, l = xb ? z.y : z.x;
+  const double q = l / g, t = 1.0 / fma(l, q, g);
+  return xb ? make_double2(t, -q * t) : make_double2(q * t, -t);
+}
+
+// The step of column c of a half panel.  The column is in r[.][0], the others
+// follow in turn; the step leaves them moved up by one and its own column last, so
+// that one loop body of constant register indices serves all columns.  The reciprocal
+// of every thread's own candidate is formed while the search runs, which waits on
+// latency; only the winner's is used.  Every wave offers its candidate's whole row
+// before the one barrier of the step.  A zero pivot sets the status bit and
+// sh.singular and the steps go on (on values that are then discarded): every
+// thread runs the same steps and meets the same barriers.
+template <int R>
+__device__ __forceinline__ void gj_step(double2 (&r)[R][kHalf], int (&lr)[R], GjShared& sh, int n,
+                                        int c, int* __restrict__ status) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int par = c & 1;
+  // pivot: largest |Re|+|Im| in rows c..n-1, first row on ties (izamax); -1: none
+  double ob = -1.0;
+  int ol = n;
+  double2 z = make_double2(1.0, 0.0);
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const double v = fabs(r[k][0].x) + fabs(r[k][0].y);
+    const bool g = (lr[k] >= c) & ((v > ob) | ((v == ob) & (lr[k] < ol)));
+    ob = g ? v : ob;
+    ol = g ? lr[k] : ol;
+    z.x = g ? r[k][0].x : z.x;
+    z.y = g ? r[k][0].y : z.y;
+  }
+  const double2 zi = gj_inv(z);
   // wave maximum: butterfly within rows of 16 lanes (DPP), then the four rows
-  double best = own;
+  double best = ob;
   best = fmax(best, dpp_d<0xB1>(best));   // quad_perm [1,0,3,2]
   best = fmax(best, dpp_d<0x4E>(best));   // quad_perm [2,3,0,1]
   best = fmax(best, dpp_d<0x124>(best));  // row_ror:4
   best = fmax(best, dpp_d<0x128>(best));  // row_ror:8
   best = fmax(fmax(readlane_d(best, 0), readlane_d(best, 16)),
               fmax(readlane_d(best, 32), readlane_d(best, 48)));
-  // the smallest row holding it (n: no candidate here)
-  int key = (best >= 0.0 && own == best) ? lr : n;
-  key = min(key, __builtin_amdgcn_update_dpp(key, key, 0xB1, 0xf, 0xf, false));
-  key = min(key, __builtin_amdgcn_update_dpp(key, key, 0x4E, 0xf, 0xf, false));
-  key = min(key, __builtin_amdgcn_update_dpp(key, key, 0x124, 0xf, 0xf, false));
-  key = min(key, __builtin_amdgcn_update_dpp(key, key, 0x128, 0xf, 0xf, false));
-  key = min(min(__builtin_amdgcn_readlane(key, 0), __builtin_amdgcn_readlane(key, 16)),
-            min(__builtin_amdgcn_readlane(key, 32), __builtin_amdgcn_readlane(key, 48)));
-  if (lane == 0) { sh.wv[wave] = best; sh.wi[wave] = key; }
-  __syncthreads();
-  best = sh.wv[0];
-  int bi = sh.wi[0];
-  for (int w = 1; w < nwave; ++w)
-    if (sh.wv[w] > best || (sh.wv[w] == best && sh.wi[w] < bi)) { best = sh.wv[w]; bi = sh.wi[w]; }
-  const int p = bi < n ? bi : c;  // no candidate compared (NaN column): keep row c
-  if (i == 0) {
-    ipiv[(size_t)b * n + c] = p;
-    const int t = sh.orig[c];
-    sh.orig[c] = sh.orig[p];
-    sh.orig[p] = t;
-    const int tb = sh.origb[c];
-    sh.origb[c] = sh.origb[p];
-    sh.origb[p] = tb;
-  }
-  const bool is_p = mine && lr == p;
-  if (is_p) {
+  const unsigned long long at = __ballot(ob == best);
+  int row = __builtin_amdgcn_readlane(ol, __ffsll(at) - 1);
+  if (best >= 0.0)
+    for (unsigned long long m = at & (at - 1); m; m &= m - 1)  // ties
+      row = min(row, __builtin_amdgcn_readlane(ol, __ffsll(m) - 1));
+  // one lane of the wave, or none (a row number is in one lane only; n in none)
 #pragma unroll
-    for (int q = 0; q < NB; ++q) sh.rowp[q] = r[q];
-    const zd pz = mkz(1.0, 0.0) / mkz(r[L].x, r[L].y);
-    sh.pinv = make_double2(pz.x, pz.y);
-    if (r[L].x == 0.0 && r[L].y == 0.0) {
-      atomicOr(status, 4);
-      sh.singular = 1;
+  for (int k = 0; k < R; ++k)
+    if (lr[k] == row) {
+      double2* o = sh.rowp[par][wave];
+      o[0] = zi;
+#pragma unroll
+      for (int q = 1; q < kHalf; ++q) o[q] = r[k][q];
     }
+  if (lane == 0) {
+    ((double*)sh.wv[par])[wave] = best;
+    ((int*)&sh.wi[par])[wave] = row;
   }
   __syncthreads();
-  const double2 pinv = sh.pinv;
-  if (is_p) {
-    // the pivot row becomes row c, scaled (its column L becomes 1/piv)
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-      r[q] = q == L ? pinv : cfma(make_double2(0.0, 0.0), r[q], pinv);
-    lr = c;
-  } else if (mine) {
-    if (lr == c) lr = p;  // row c's content is row p's now
-    const double2 s = cfma(make_double2(0.0, 0.0), r[L], pinv);
-#pragma unroll
-    for (int q = 0; q < NB; ++q)
-      r[q] = q == L ? make_double2(-s.x, -s.y) : cfms(r[q], s, sh.rowp[q]);
+  const double2 w01 = sh.wv[par][0], w23 = sh.wv[par][1];
+  const int4 wi = sh.wi[par];
+  const bool b1 = (w01.y > w01.x) | ((w01.y == w01.x) & (wi.y < wi.x));
+  const bool b3 = (w23.y > w23.x) | ((w23.y == w23.x) & (wi.w < wi.z));
+  const double va = b1 ? w01.y : w01.x, vb = b3 ? w23.y : w23.x;
+  const int pa = b1 ? wi.y : wi.x, pb = b3 ? wi.w : wi.z;
+  const bool bb = (vb > va) | ((vb == va) & (pb < pa));
+  best = bb ? vb : va;
+  int p = bb ? pb : pa;
+  // lane l of a row of 16 lanes reads entry l and the others get it by DPP: read by
+  // every lane, an entry costs each wave a read of LDS (first panel of NG 586:
+  // 94 us so, 86 this way)
+  double2 v = sh.rowp[par][bb ? 2 + b3 : (int)b1][lane & 15];
+  if (best < 0.0) {  // no candidate compared (NaN column): keep row c, all becomes NaN
+    p = c;
+    v.x = v.y = __builtin_nan("");
   }
-}
-
-template <int... L>
-__device__ __forceinline__ void gj_reg_steps(std::integer_sequence<int, L...>, double2 (&r)[kPanelMax],
-                                             int& lr, GjRegShared& sh, int i, int n, int c0,
-                                             bool mine, int b, int* __restrict__ ipiv,
-                                             int* __restrict__ status) {
-  (gj_reg_step<L>(r, lr, sh, i, n, c0, mine, b, ipiv, status), ...);
-}
-
-// Columns [c0, c0+16) of the rows the threads hold, back to the matrix at
-// their row numbers.
-__device__ __forceinline__ void gj_reg_store(const double2 (&r)[kPanelMax], int lr, bool mine,
-                                             double2* __restrict__ m, int n, int c0) {
-  if (mine)
-#pragma unroll
-    for (int q = 0; q < kPanelMax; ++q) m[lr + (size_t)n * (c0 + q)] = r[q];
-}
-
-// Factors the panel [c0, c0+16) of matrix m held in r (row i of the panel in
-// thread i), writes it back and leaves the move list in mv.
-__device__ __forceinline__ void gj_reg_factor(double2 (&r)[kPanelMax], GjRegShared& sh, int i,
-                                              int n, int c0, bool mine, int b,
-                                              double2* __restrict__ m, int* __restrict__ ipiv,
-                                              int* __restrict__ mv, int* __restrict__ status) {
-  constexpr int NB = kPanelMax;
-  if (mine) sh.orig[i] = i;
-  if (i == 0) { sh.nmove = 0; sh.singular = 0; }
-  __syncthreads();
-  int lr = i;
-  gj_reg_steps(std::make_integer_sequence<int, NB>{}, r, lr, sh, i, n, c0, mine, b, ipiv, status);
-  __syncthreads();
-  const bool singular = sh.singular != 0;
-  if (!singular) gj_reg_store(r, lr, mine, m, n, c0);
-  // move list: the nb panel rows first (in order), then other rows whose
-  // content changed
-  if (i < NB) {
-    mv[1 + i] = c0 + i;
-    mv[1 + kMoveMax + i] = sh.orig[c0 + i];
+  if (best == 0.0 && threadIdx.x == 0) {
+    atomicOr(status, 4);
+    sh.singular = 1;
   }
-  if (mine && (i < c0 || i >= c0 + NB) && sh.orig[i] != i) {
-    const int e = NB + atomicAdd(&sh.nmove, 1);
-    mv[1 + e] = i;
-    mv[1 + kMoveMax + e] = sh.orig[i];
-  }
-  __syncthreads();
-  if (i == 0) mv[0] = singular ? -1 : NB + sh.nmove;
-}
-
-__global__ void __launch_bounds__(768) k_gj_panel_reg(double2* __restrict__ a, int n, int c0,
-                                                      int* __restrict__ ipiv,
-                                                      int* __restrict__ moves,
-                                                      int* __restrict__ status) {
-  constexpr int NB = kPanelMax;
-  __shared__ GjRegShared sh;
-  const int b = blockIdx.x, i = threadIdx.x;
-  double2* m = a + (size_t)b * n * n;
-  const bool mine = i < n;
-  double2 r[NB];
 #pragma unroll
-  for (int q = 0; q < NB; ++q) r[q] = mine ? m[i + (size_t)n * (c0 + q)] : make_double2(0.0, 0.0);
-  gj_reg_factor(r, sh, i, n, c0, mine, b, m, ipiv, moves + (size_t)b * kMoveInts, status);
+  for (int k = 0; k < R; ++k)
+    // the pivot row becomes row c, scaled: zero less the row times -1/pivot
+    if (lr[k] == p)
+#pragma unroll
+      for (int q = 0; q < kHalf; ++q) r[k][q] = make_double2(0.0, 0.0);
+  const double2 pinv = gj_bcast<0>(v);
+  double2 f[R];  // what multiplies the pivot row
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const double2 g = cfma(make_double2(0.0, 0.0), r[k][0], pinv);
+    const bool is = lr[k] == p;
+    f[k] = make_double2(is ? -pinv.x : g.x, is ? -pinv.y : g.y);
+    lr[k] = is ? c : lr[k] == c ? p : lr[k];  // row c's content is row p's now
+  }
+  gj_rank1(std::make_integer_sequence<int, kHalf - 1>{}, r, f, v);
+#pragma unroll
+  for (int k = 0; k < R; ++k) r[k][kHalf - 1] = make_double2(-f[k].x, -f[k].y);
 }
 
-// One step of the register path (n <= 768, full panels) with look-ahead: the
-// rank-16 update of panel k (columns [ck, ck+16), factored by the previous
-// launch, its move list in moves_k) and, when next is set, the factoring of
-// panel k+1 in the same launch.  Blocks [0, nbatch) (next set) are panel
-// blocks: they apply panel k's update to the 16 columns of panel k+1 in
-// registers and factor them at once (gj_reg_factor), writing the move list to
-// moves_next.  Every other block updates one group of up to 16 other columns
-// of one matrix: the columns outside [ck, ck + 16 (1 + next)), in groups of
-// 16, ngroups per matrix.  The two kinds touch disjoint columns and read
-// panel k's columns only, so nothing in the launch waits for anything else:
-// the panel factoring (one block per matrix, latency-bound) runs beside the
-// bandwidth-bound update instead of after it.  Thread i handles row i; the
-// arithmetic is k_gj_update's, operation for operation.  The rows the move
-// list names (at most 32) are staged in LDS first; after that each thread
-// reads and writes its own row only, so the waves run without further
-// barriers and one wave's loads overlap another's arithmetic.  With nbatch a
-// multiple of 8 the update blocks of matrix b run on XCD b mod 8 (blocks are
-// dealt to the XCDs round-robin), so each XCD's L2 holds its matrices' panels.
-struct GjStepShared {
-  GjRegShared p;
-  // old values of the moved rows in the block's columns: vals[e][t] = a(src_e, cj + t);
-  // the first 16 entries are panel k's pivot rows
-  double2 vals[kMoveMax][kPanelMax];
-  int dst[kMoveMax], src[kMoveMax];
-};
-
-__global__ void __launch_bounds__(768) k_gj_step(double2* __restrict__ a, int n, int ck, int next,
-                                                 int nbatch, int ngroups, int* __restrict__ ipiv,
-                                                 const int* __restrict__ moves_k,
-                                                 int* __restrict__ moves_next,
-                                                 int* __restrict__ status) {
-  constexpr int NB = kPanelMax;
-  __shared__ GjStepShared sh;
-  const int i = threadIdx.x;
-  const bool mine = i < n;
-  const bool panel = next && (int)blockIdx.x < nbatch;
-  int b, cj, ntj;
-  if (panel) {
-    b = blockIdx.x;
-    cj = ck + NB;
-    ntj = NB;
-  } else {
-    const int u = (int)blockIdx.x - (next ? nbatch : 0);
-    int t;
-    if (nbatch % 8 == 0) {
-      const int x = u % 8, s = u / 8;
-      b = x + 8 * (s / ngroups);
-      t = s % ngroups;
-    } else {
-      b = u / ngroups;
-      t = u % ngroups;
+// Factors columns [c, c + w), w <= 16, in registers and puts them back; map[i]
+// becomes the row whose content is in row i.  Ends with a barrier.
+template <int R>
+__device__ __forceinline__ void gj_half(GjShared& sh, int* map, double2* m, int n, int c, int w,
+                                        int* __restrict__ status) {
+  double2 r[R][kHalf];
+  int lr[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int i = threadIdx.x + kGjThreads * k;
+    lr[k] = i < n ? i : -1;
+#pragma unroll
+    for (int q = 0; q < kHalf; ++q)
+      r[k][q] = i < n && q < w ? m[i + (size_t)n * (c + q)] : make_double2(0.0, 0.0);
+  }
+#pragma unroll 1
+  for (int l = 0; l < w; ++l) gj_step<R>(r, lr, sh, n, c + l, status);
+  // column l is now in r[.][16 - w + l]
+#pragma unroll
+  for (int k = 0; k < R; ++k)
+    if (lr[k] >= 0) {
+      map[lr[k]] = threadIdx.x + kGjThreads * k;
+#pragma unroll
+      for (int q = 0; q < kHalf; ++q)
+        if (q >= kHalf - w) m[lr[k] + (size_t)n * (c + q - (kHalf - w))] = r[k][q];
     }
-    const int skip = NB * (1 + next);  // columns [ck, ck + skip) are not in the groups
-    const int t0 = t * NB;             // groups never straddle ck (both multiples of 16)
-    cj = t0 < ck ? t0 : t0 + skip;
-    ntj = min(NB, n - skip - t0);
-  }
-  double2* m = a + (size_t)b * n * n;
-  const int* mv = moves_k + (size_t)b * kMoveInts;
-  const int nm = mv[0];
-  if (nm < 0) {  // a zero pivot earlier (the host reports it): nothing more for this matrix
-    if (panel && i == 0) moves_next[(size_t)b * kMoveInts] = -1;
-    return;  // uniform: every thread read the same word
-  }
-  if (i < nm) {
-    sh.dst[i] = mv[1 + i];
-    sh.src[i] = mv[1 + kMoveMax + i];
-  }
   __syncthreads();
-  // the only rows a thread reads besides its own: those the move list names
-  for (int x = i; x < nm * NB; x += blockDim.x) {
-    const int e = x / NB, t = x % NB;
-    sh.vals[e][t] = t < ntj ? m[sh.src[e] + (size_t)n * (cj + t)] : make_double2(0.0, 0.0);
-  }
-  __syncthreads();  // after this each thread reads and writes its own row only
-  const bool inpanel = i >= ck && i < ck + NB;
-  int slot = -1;
-  if (!inpanel)
-    for (int e = NB; e < nm; ++e)
-      if (sh.dst[e] == i) slot = e;
-  double2 r[NB];
-#pragma unroll
-  for (int t = 0; t < NB; ++t)
-    r[t] = (!mine || inpanel || t >= ntj) ? make_double2(0.0, 0.0)
-           : slot >= 0                    ? sh.vals[slot][t]
-                                          : m[i + (size_t)n * (cj + t)];
-  if (mine) {
-    for (int q = 0; q < NB; ++q) {
-      const double2 wq = m[i + (size_t)n * (ck + q)];
-#pragma unroll
-      for (int t = 0; t < NB; ++t) r[t] = cfma(r[t], wq, sh.vals[q][t]);
-    }
-  }
-  if (!panel) {
-    if (mine)
-#pragma unroll
-      for (int t = 0; t < NB; ++t)
-        if (t < ntj) m[i + (size_t)n * (cj + t)] = r[t];
-    return;  // uniform per block
-  }
-  gj_reg_factor(r, sh.p, i, n, cj, mine, b, m, ipiv, moves_next + (size_t)b * kMoveInts, status);
 }
 
-// ---------------------------------------------------------------------------
-// Register path with 32-column steps (n <= 768).  Each launch applies the
-// rank-32 transform of one 32-column panel (two 16-column halves factored by
-// the previous launch) to every other column: half the passes over the
-// matrices of 16-column steps.  One block per matrix brings the next panel up
-// to date and factors it in the same launch (look-ahead), as two halves in
-// registers: half A, then half B after A's transform, then A after B's.
-// The transform of the two halves together differs from the identity in the
-// 32 panel columns only, so every other column j becomes
-//   a'(:,j) = P a(:,j) with the panel rows zeroed + W (P a)(panel rows, j),
-// W the panel's 32 final columns and P the panel's row interchanges (B's act
-// on rows below A's panel rows only, so A's transform commutes past them).
-constexpr int kSuper = 32;
-constexpr int kMoveMax32 = 2 * kSuper;          // panel rows and rows they displaced
-constexpr int kMoveInts32 = 1 + 2 * kMoveMax32;  // {count, dst[64], src[64]}
+// The move list of the rows that map moves, the nb panel rows [c0, c0 + nb)
+// first, into sh.dst/src/nm.  Ends with a barrier.
+__device__ __forceinline__ void gj_list(GjShared& sh, const int* map, int n, int c0, int nb) {
+  if (threadIdx.x == 0) sh.nm = nb;
+  if ((int)threadIdx.x < nb) {
+    sh.dst[threadIdx.x] = c0 + threadIdx.x;
+    sh.src[threadIdx.x] = map[c0 + threadIdx.x];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += kGjThreads)
+    if ((i < c0 || i >= c0 + nb) && map[i] != i) {
+      const int e = atomicAdd(&sh.nm, 1);  // at most nb of them
+      sh.dst[e] = i;
+      sh.src[e] = map[i];
+    }
+  __syncthreads();
+}
 
-constexpr int kUpdCols = 32;  // columns per update workgroup of a 32-column step
-
-struct Gj32Shared {
-  GjRegShared p;
-  double2 vals[kMoveMax32][kUpdCols];  // old values of the moved rows in up to 32 columns
-  int dst[kMoveMax32], src[kMoveMax32];
-  int nm;
-};
-
-// Loads into sh.vals the old values of the nm moved rows (sources sh.src) in
-// columns [cj, cj + ntj) of a CW-column group and ends with a barrier.
-template <int CW>
-__device__ __forceinline__ void gj32_stage(Gj32Shared& sh, const double2* __restrict__ m, int n,
-                                           int cj, int ntj, int nm) {
-  for (int x = threadIdx.x; x < nm * CW; x += blockDim.x) {
+// Columns [cj, cj + nt) of m, nt <= 16 CT, after the transform of the panel
+// [ck, ck + w), w <= 4 KQ, with the move list in sh: C = P a with the panel rows
+// zeroed, plus W times the panel rows of P a, on the matrix cores (FP64
+// 16x16x4, four real products per complex one).  A wave takes tiles of 16 rows, W and
+// C from memory with the next tile's in flight.  On the vector unit every fourth multiply-add needs one of
+// the panel rows' values broadcast from LDS.  NG 586, 32 columns of a block: 38 us, of which 17 are the products at the
+// rate of the matrix cores.  Begins with writes to LDS that earlier readers must be done with,
+// ends with a barrier.
+template <int KQ, int CT>
+__device__ __forceinline__ void gj_apply(GjShared& sh, double2* m, int n, int ck, int w, int cj,
+                                         int nt) {
+  constexpr int CW = 16 * CT;
+  const int nm = sh.nm;
+  for (int x = threadIdx.x; x < nm * CW; x += kGjThreads) {
     const int e = x / CW, t = x % CW;
-    sh.vals[e][t] = t < ntj ? m[sh.src[e] + (size_t)n * (cj + t)] : make_double2(0.0, 0.0);
+    sh.vals[e][t] = t < nt ? m[sh.src[e] + (size_t)n * (cj + t)] : make_double2(0.0, 0.0);
   }
+  for (int i = threadIdx.x; i < n; i += kGjThreads) sh.slot[i] = -1;
   __syncthreads();
-}
-
-// Row i of columns [cj, cj + ntj) (at most CW) after the rank-W transform of
-// the panel [ck, ck + W): the staged move list (sh.dst/sh.vals, its first W
-// entries the panel rows in order) and the panel columns W(i, q) read from m.
-template <int W, int CW>
-__device__ __forceinline__ void gj32_apply(double2 (&r)[CW], const Gj32Shared& sh,
-                                           const double2* __restrict__ m, int n, int ck, int cj,
-                                           int ntj, int nm, int i, bool mine) {
-  const bool inpanel = i >= ck && i < ck + W;
-  int slot = -1;
-  if (!inpanel)
-    for (int e = W; e < nm; ++e)
-      if (sh.dst[e] == i) slot = e;
+  if ((int)threadIdx.x < nm) sh.slot[sh.dst[threadIdx.x]] = (int)threadIdx.x < w ? -2 : threadIdx.x;
+  __syncthreads();
+  const int lane = threadIdx.x & 63, lo = lane & 15, hi = lane >> 4;
+  // loads without conditions, at clamped addresses: what a row or column takes
+  // instead of its own value is put in when the value is used
+  double2 wn[KQ], cn[CT][4];
+  int sn = -1;
+  auto load = [&](int tile) {
+    const int i = min(16 * tile + lo, n - 1);
+    sn = sh.slot[i];
 #pragma unroll
-  for (int t = 0; t < CW; ++t)
-    r[t] = (!mine || inpanel || t >= ntj) ? make_double2(0.0, 0.0)
-           : slot >= 0                    ? sh.vals[slot][t]
-                                          : m[i + (size_t)n * (cj + t)];
-  if (!mine) return;
-  for (int q = 0; q < W; ++q) {
-    const double2 wq = m[i + (size_t)n * (ck + q)];
+    for (int k = 0; k < KQ; ++k) wn[k] = m[i + (size_t)n * (ck + min(4 * k + hi, w - 1))];
 #pragma unroll
-    for (int t = 0; t < CW; ++t) r[t] = cfma(r[t], wq, sh.vals[q][t]);
-  }
-}
-
-// The move list of rows whose source differs from themselves in map (orig or
-// origb of sh.p), the nb panel rows [c0, c0 + nb) first, into sh.dst/src/nm.
-__device__ __forceinline__ void gj32_list(Gj32Shared& sh, const int* map, int n, int c0, int nb,
-                                          int i, bool mine) {
-  if (i == 0) sh.nm = nb;
-  if (i < nb) {
-    sh.dst[i] = c0 + i;
-    sh.src[i] = map[c0 + i];
-  }
-  __syncthreads();
-  if (mine && (i < c0 || i >= c0 + nb) && map[i] != i) {
-    const int e = atomicAdd(&sh.nm, 1);
-    sh.dst[e] = i;
-    sh.src[e] = map[i];
-  }
-  __syncthreads();
-}
-
-// Factors the 32-column panel [c, c + 32) of matrix b: half A's columns are
-// in r (up to date), half B's in m (up to date).  Leaves the panel's final
-// columns in m and its move list in mv.
-__device__ __forceinline__ void gj32_chain(double2 (&r)[kPanelMax], Gj32Shared& sh, double2* m,
-                                           int n, int c, int b, int* __restrict__ ipiv,
-                                           int* __restrict__ mv, int* __restrict__ status) {
-  const int i = threadIdx.x;
-  const bool mine = i < n;
-  if (mine) sh.p.orig[i] = sh.p.origb[i] = i;
-  if (i == 0) sh.p.singular = 0;
-  __syncthreads();
-  // half A
-  int lr = i;
-  gj_reg_steps(std::make_integer_sequence<int, kPanelMax>{}, r, lr, sh.p, i, n, c, mine, b, ipiv,
-               status);
-  __syncthreads();
-  if (sh.p.singular) {
-    if (i == 0) mv[0] = -1;
-    return;  // uniform
-  }
-  gj_reg_store(r, lr, mine, m, n, c);
-  // half B after A's transform (A's moves: origb since the reset)
-  gj32_list(sh, sh.p.origb, n, c, kPanelMax, i, mine);
-  gj32_stage<kPanelMax>(sh, m, n, c + kPanelMax, kPanelMax, sh.nm);
-  gj32_apply<kPanelMax, kPanelMax>(r, sh, m, n, c, c + kPanelMax, kPanelMax, sh.nm, i, mine);
-  if (mine) sh.p.origb[i] = i;
-  __syncthreads();
-  lr = i;
-  gj_reg_steps(std::make_integer_sequence<int, kPanelMax>{}, r, lr, sh.p, i, n, c + kPanelMax, mine,
-               b, ipiv, status);
-  __syncthreads();
-  if (sh.p.singular) {
-    if (i == 0) mv[0] = -1;
-    return;  // uniform
-  }
-  gj_reg_store(r, lr, mine, m, n, c + kPanelMax);
-  // half A after B's transform (B's moves: origb since its reset)
-  gj32_list(sh, sh.p.origb, n, c + kPanelMax, kPanelMax, i, mine);
-  gj32_stage<kPanelMax>(sh, m, n, c, kPanelMax, sh.nm);
-  gj32_apply<kPanelMax, kPanelMax>(r, sh, m, n, c + kPanelMax, c, kPanelMax, sh.nm, i, mine);
-  __syncthreads();  // every staged read of A is done before A is overwritten
-  if (mine)
+    for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-    for (int q = 0; q < kPanelMax; ++q) m[i + (size_t)n * (c + q)] = r[q];
-  // the panel's move list: its 32 rows, then the rows they displaced
-  gj32_list(sh, sh.p.orig, n, c, kSuper, i, mine);
-  for (int e = i; e < sh.nm; e += blockDim.x) {
-    mv[1 + e] = sh.dst[e];
-    mv[1 + kMoveMax32 + e] = sh.src[e];
-  }
-  if (i == 0) mv[0] = sh.nm;
-}
-
-// The first panel [0, 32): one block per matrix.
-__global__ void __launch_bounds__(768) k_gj_first32(double2* __restrict__ a, int n,
-                                                    int* __restrict__ ipiv, int* __restrict__ moves,
-                                                    int* __restrict__ status) {
-  __shared__ Gj32Shared sh;
-  const int b = blockIdx.x, i = threadIdx.x;
-  double2* m = a + (size_t)b * n * n;
-  double2 r[kPanelMax];
+      for (int v = 0; v < 4; ++v)
+        cn[ct][v] = m[i + (size_t)n * (cj + min(16 * ct + hi + 4 * v, nt - 1))];
+  };
+  const int ntile = (n + 15) / 16;
+  int tile = threadIdx.x >> 6;
+  if (tile < ntile) load(tile);
+  for (; tile < ntile; tile += kGjThreads / 64) {
+    double2 wc[KQ];
+    d4 re[CT], im[CT];
 #pragma unroll
-  for (int q = 0; q < kPanelMax; ++q) r[q] = i < n ? m[i + (size_t)n * q] : make_double2(0.0, 0.0);
-  gj32_chain(r, sh, m, n, 0, b, ipiv, moves + (size_t)b * kMoveInts32, status);
+    for (int k = 0; k < KQ; ++k) {
+      const bool in = 4 * k + hi < w;
+      wc[k] = make_double2(in ? wn[k].x : 0.0, in ? wn[k].y : 0.0);
+    }
+    const int slot = sn;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        re[ct][v] = slot == -2 ? 0.0 : cn[ct][v].x;
+        im[ct][v] = slot == -2 ? 0.0 : cn[ct][v].y;
+      }
+    if (__ballot(slot >= 0) != 0) {  // few tiles
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const double2 o = sh.vals[max(slot, 0)][16 * ct + hi + 4 * v];
+          re[ct][v] = slot >= 0 ? o.x : re[ct][v];
+          im[ct][v] = slot >= 0 ? o.y : im[ct][v];
+        }
+    }
+    if (tile + kGjThreads / 64 < ntile) load(tile + kGjThreads / 64);
+#pragma unroll
+    for (int k = 0; k < KQ; ++k) {
+      double2 v[CT];
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        v[ct] = 4 * k + hi < w ? sh.vals[4 * k + hi][16 * ct + lo] : make_double2(0.0, 0.0);
+        re[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[ct].x, wc[k].x, re[ct], 0, 0, 0);
+        im[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[ct].x, wc[k].y, im[ct], 0, 0, 0);
+      }
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        re[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(-v[ct].y, wc[k].y, re[ct], 0, 0, 0);
+        im[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[ct].y, wc[k].x, im[ct], 0, 0, 0);
+      }
+    }
+    const int i = 16 * tile + lo;
+    if (i < n)
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int t = 16 * ct + hi + 4 * v;
+          if (t < nt) m[i + (size_t)n * (cj + t)] = make_double2(re[ct][v], im[ct][v]);
+        }
+  }
+  __syncthreads();
 }
 
-// One 32-column step: the rank-32 transform of panel k (columns [ck, ck+32),
-// move list moves_k) on every other column and, when next is set, the
-// factoring of panel k+1.  Blocks [0, nbatch) (next set) are panel blocks:
-// they update the 32 columns of panel k+1 (half B to HBM, half A kept in
-// registers) and factor it (gj32_chain).  Every other block updates 32 other
-// columns of one matrix (fewer in the last group): those outside
-// [ck, ck + 32 (1 + next)), ngroups per matrix, so a block reads the panel's
-// 32 columns once for 32 of its own.  The two kinds touch disjoint columns and
-// read panel k's columns only.  With nbatch a multiple of 8 the update blocks
-// of matrix b run on XCD b mod 8.
-__global__ void __launch_bounds__(768) k_gj_step32(double2* __restrict__ a, int n, int ck, int next,
-                                                   int nbatch, int ngroups, int* __restrict__ ipiv,
-                                                   const int* __restrict__ moves_k,
-                                                   int* __restrict__ moves_next,
-                                                   int* __restrict__ status) {
-  __shared__ Gj32Shared sh;
-  const int i = threadIdx.x;
-  const bool mine = i < n;
-  const bool panel = next && (int)blockIdx.x < nbatch;
-  int b, cj = 0, ntj = kPanelMax;
+// Factors the panel [c, c + w), w <= 32, of one matrix, its columns up to date
+// in m.  Leaves the panel's final columns in m, its move list in mv (count -1 after
+// a zero pivot) and in perm[i] the row of the given matrix that is now row i.
+template <int R>
+__device__ __forceinline__ void gj_panel32(GjShared& sh, double2* m, int n, int c, int w,
+                                           int* __restrict__ perm, int* __restrict__ mv,
+                                           int* __restrict__ status) {
+  const int wa = min(w, kHalf), wb = w - wa;
+  if (c == 0)
+    for (int i = threadIdx.x; i < n; i += kGjThreads) perm[i] = i;
+  if (threadIdx.x == 0) sh.singular = 0;
+  gj_half<R>(sh, sh.orig, m, n, c, wa, status);
+  if (wb > 0) {
+    gj_list(sh, sh.orig, n, c, wa);
+    gj_apply<kHalf / 4, 1>(sh, m, n, c, wa, c + wa, wb);
+    gj_half<R>(sh, sh.orig2, m, n, c + wa, wb, status);
+    gj_list(sh, sh.orig2, n, c + wa, wb);
+    gj_apply<kHalf / 4, 1>(sh, m, n, c + wa, wb, c, wa);
+  }
+  if (sh.singular) {  // uniform: set before the barriers above
+    if (threadIdx.x == 0) mv[0] = -1;
+    return;
+  }
+  int o[R], pn[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int i = threadIdx.x + kGjThreads * k;
+    if (i < n) {
+      o[k] = sh.orig[wb > 0 ? sh.orig2[i] : i];
+      pn[k] = perm[o[k]];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int i = threadIdx.x + kGjThreads * k;
+    if (i < n) {
+      sh.orig[i] = o[k];
+      perm[i] = pn[k];
+    }
+  }
+  __syncthreads();
+  gj_list(sh, sh.orig, n, c, w);
+  if ((int)threadIdx.x < sh.nm) {
+    mv[1 + threadIdx.x] = sh.dst[threadIdx.x];
+    mv[1 + kMoveMax32 + threadIdx.x] = sh.src[threadIdx.x];
+  }
+  if (threadIdx.x == 0) mv[0] = sh.nm;
+}
+
+// The first panel: one block per matrix.
+template <int R>
+__global__ void __launch_bounds__(kGjThreads, R < 3 ? 2 : 1)
+    k_gj_first(double2* __restrict__ a, int n, int* __restrict__ perm, int* __restrict__ moves,
+               int* __restrict__ status) {
+  __shared__ GjShared sh;
+  const int b = blockIdx.x;
+  gj_panel32<R>(sh, a + (size_t)b * n * n, n, 0, min(n, kSuper), perm + (size_t)b * n,
+                moves + (size_t)b * kMoveInts32, status);
+}
+
+// One step: the transform of panel k (columns [ck, ck + w), move list moves_k)
+// on every other column and, when wn > 0, the factoring of panel k + 1, columns
+// [ck + 32, ck + 32 + wn).  Blocks [0, nbatch) (wn > 0) are panel blocks.  Every
+// other block updates up to 32 columns of one matrix outside both panels, ngroups
+// groups per matrix.  The two kinds touch disjoint columns and read panel k's
+// columns only, so nothing in the launch waits for anything else.  With nbatch a
+// multiple of 8 the update blocks of matrix b run on XCD b mod 8 (blocks are dealt
+// to the XCDs round-robin), so each XCD's L2 holds its matrices' panels.
+template <int R>
+__global__ void __launch_bounds__(kGjThreads, R < 3 ? 2 : 1)
+    k_gj_step32(double2* __restrict__ a, int n, int ck, int w, int wn, int nbatch, int ngroups,
+                int* __restrict__ perm, const int* __restrict__ moves_k,
+                int* __restrict__ moves_next, int* __restrict__ status) {
+  __shared__ GjShared sh;
+  const bool panel = wn > 0 && (int)blockIdx.x < nbatch;
+  int b, cj, nt;
   if (panel) {
     b = blockIdx.x;
+    cj = ck + w;
+    nt = wn;
   } else {
-    const int u = (int)blockIdx.x - (next ? nbatch : 0);
+    const int u = (int)blockIdx.x - (wn > 0 ? nbatch : 0);
     int t;
     if (nbatch % 8 == 0) {
       const int x = u % 8, s = u / 8;
@@ -646,46 +611,44 @@ __global__ void __launch_bounds__(768) k_gj_step32(double2* __restrict__ a, int 
       b = u / ngroups;
       t = u % ngroups;
     }
-    const int skip = kSuper * (1 + next);  // columns [ck, ck + skip) are not in the groups
-    const int t0 = t * kUpdCols;           // groups never straddle ck (multiples of 32)
+    const int skip = w + wn;      // columns [ck, ck + skip) are not in the groups
+    const int t0 = t * kSuper;    // groups never straddle ck (multiples of 32)
     cj = t0 < ck ? t0 : t0 + skip;
-    ntj = min(kUpdCols, n - skip - t0);
+    nt = min(kSuper, n - skip - t0);
   }
   double2* m = a + (size_t)b * n * n;
   const int* mv = moves_k + (size_t)b * kMoveInts32;
   const int nm = mv[0];
   if (nm < 0) {  // a zero pivot earlier (the host reports it): nothing more for this matrix
-    if (panel && i == 0) moves_next[(size_t)b * kMoveInts32] = -1;
+    if (panel && threadIdx.x == 0) moves_next[(size_t)b * kMoveInts32] = -1;
     return;  // uniform: every thread read the same word
   }
-  if (i < nm) {
-    sh.dst[i] = mv[1 + i];
-    sh.src[i] = mv[1 + kMoveMax32 + i];
+  if ((int)threadIdx.x < nm) {
+    sh.dst[threadIdx.x] = mv[1 + threadIdx.x];
+    sh.src[threadIdx.x] = mv[1 + kMoveMax32 + threadIdx.x];
   }
+  if (threadIdx.x == 0) sh.nm = nm;
   __syncthreads();
-  if (!panel) {
-    double2 ru[kUpdCols];
-    gj32_stage<kUpdCols>(sh, m, n, cj, ntj, nm);
-    gj32_apply<kSuper, kUpdCols>(ru, sh, m, n, ck, cj, ntj, nm, i, mine);
-    if (mine)
-#pragma unroll
-      for (int t = 0; t < kUpdCols; ++t)
-        if (t < ntj) m[i + (size_t)n * (cj + t)] = ru[t];
-    return;  // uniform per block
-  }
-  double2 r[kPanelMax];
-  // panel k+1: half B brought up to date into HBM, then half A into registers
-  const int c = ck + kSuper;
-  gj32_stage<kPanelMax>(sh, m, n, c + kPanelMax, kPanelMax, nm);
-  gj32_apply<kSuper, kPanelMax>(r, sh, m, n, ck, c + kPanelMax, kPanelMax, nm, i, mine);
-  __syncthreads();  // staged reads of B done before B is overwritten
-  if (mine)
-#pragma unroll
-    for (int t = 0; t < kPanelMax; ++t) m[i + (size_t)n * (c + kPanelMax + t)] = r[t];
-  gj32_stage<kPanelMax>(sh, m, n, c, kPanelMax, nm);
-  gj32_apply<kSuper, kPanelMax>(r, sh, m, n, ck, c, kPanelMax, nm, i, mine);
-  __syncthreads();  // every thread's B row is written before the chain stages B rows
-  gj32_chain(r, sh, m, n, c, b, ipiv, moves_next + (size_t)b * kMoveInts32, status);
+  gj_apply<kSuper / 4, 2>(sh, m, n, ck, w, cj, nt);
+  if (panel)  // uniform per block
+    gj_panel32<R>(sh, m, n, cj, nt, perm + (size_t)b * n, moves_next + (size_t)b * kMoveInts32,
+                  status);
+}
+
+// The columns back in the given matrix's order: with row i of P a the row perm[i]
+// of a, column i of (P a)^-1 is column perm[i] of a^-1.  grid (ceil(n / 8),
+// nbatch): a block moves eight rows through LDS.
+constexpr int kPermRows = 8;
+__global__ void __launch_bounds__(512) k_gj_colperm(double2* __restrict__ a, int n,
+                                                    const int* __restrict__ perm) {
+  extern __shared__ double2 lds[];
+  const int b = blockIdx.y, row = blockIdx.x * kPermRows + (threadIdx.x % kPermRows);
+  double2* m = a + (size_t)b * n * n;
+  for (int x = threadIdx.x; x < n * kPermRows; x += 512)
+    if (row < n) lds[x] = m[row + (size_t)n * (x / kPermRows)];
+  __syncthreads();
+  for (int x = threadIdx.x; x < n * kPermRows; x += 512)
+    if (row < n) m[row + (size_t)n * perm[(size_t)b * n + x / kPermRows]] = lds[x];
 }
 
 // Rank-nb update of every column outside the panel.  grid: (ceil((n-nb)/TJ),
@@ -792,48 +755,44 @@ void launch_eps_build(const double2* chi, const double* qn, int n, int nbatch, i
 // blocks write panel k+1's.
 size_t gauss_jordan_work_ints(int nbatch) { return 2 * (size_t)nbatch * kMoveInts32; }
 
+template <int R>
+static void launch_gj32(double2* a, int n, int nbatch, int* perm, int* work, int* status,
+                        hipStream_t s) {
+  auto moves = [&](int k) { return work + (size_t)(k & 1) * nbatch * kMoveInts32; };
+  hipLaunchKernelGGL(k_gj_first<R>, dim3(nbatch), dim3(kGjThreads), 0, s, a, n, perm, moves(0),
+                     status);
+  for (int k = 0, ck = 0; ck < n; ++k, ck += kSuper) {
+    const int w = std::min(kSuper, n - ck), wn = std::min(kSuper, n - ck - w);
+    const int ngroups = (n - w - wn + kSuper - 1) / kSuper;
+    const int nblk = (wn > 0 ? nbatch : 0) + nbatch * ngroups;
+    if (nblk > 0)
+      hipLaunchKernelGGL(k_gj_step32<R>, dim3(nblk), dim3(kGjThreads), 0, s, a, n, ck, w, wn, nbatch,
+                         ngroups, perm, (const int*)moves(k), moves(k + 1), status);
+  }
+}
+
+// ipiv: n ints per matrix; work: gauss_jordan_work_ints(nbatch).
 void launch_gauss_jordan(double2* a, int n, int nbatch, int* ipiv, int* work, int* status,
                          hipStream_t s) {
+  if (n <= kGjRows) {
+    RP_CHECK(n >= 1, "Dyson: empty matrix");
+    if (n <= kGjThreads) launch_gj32<1>(a, n, nbatch, ipiv, work, status, s);
+    else if (n <= 2 * kGjThreads) launch_gj32<2>(a, n, nbatch, ipiv, work, status, s);
+    else launch_gj32<3>(a, n, nbatch, ipiv, work, status, s);
+    const size_t lds = sizeof(double2) * kPermRows * n;
+    if (lds > 65536)
+      RP_HIP(hipFuncSetAttribute((const void*)k_gj_colperm,
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_gj_colperm, dim3((n + kPermRows - 1) / kPermRows, nbatch), dim3(512), lds,
+                       s, a, n, (const int*)ipiv);
+    RP_HIP(hipGetLastError());
+    return;
+  }
   // move list of panel number k: work + (k & 1) * nbatch * kMoveInts
   auto moves = [&](int k) { return work + (size_t)(k & 1) * nbatch * kMoveInts; };
   int c0 = 0, panel = 0;
-  if (n <= 768 && n >= kSuper) {
-    // a thread per row (at least 256: the steps stage 64 x 16 moved-row values)
-    const int nt = std::max(256, (n + 63) / 64 * 64);
-    auto moves32 = [&](int k) { return work + (size_t)(k & 1) * nbatch * kMoveInts32; };
-    const int nfull = n / kSuper;
-    hipLaunchKernelGGL(k_gj_first32, dim3(nbatch), dim3(nt), 0, s, a, n, ipiv, moves32(0), status);
-    for (int k = 0; k < nfull; ++k) {
-      const int next = k + 1 < nfull ? 1 : 0;
-      const int nrest = n - kSuper * (1 + next);
-      const int ngroups = (nrest + kUpdCols - 1) / kUpdCols;
-      const int nblk = (next ? nbatch : 0) + nbatch * ngroups;
-      if (nblk > 0)
-        hipLaunchKernelGGL(k_gj_step32, dim3(nblk), dim3(nt), 0, s, a, n, k * kSuper, next, nbatch,
-                           ngroups, ipiv, (const int*)moves32(k), moves32(k + 1), status);
-    }
-    c0 = nfull * kSuper;
-    panel = nfull;  // the LDS path's move lists continue the alternation
-  } else if (n <= 768 && n >= kPanelMax) {
-    // a thread per row (at least 256: the step stages 16 x 16 pivot-row values)
-    const int nt = std::max(256, (n + 63) / 64 * 64);
-    // full panels in registers, each launch updating panel k and factoring k+1
-    const int nfull = n / kPanelMax;
-    hipLaunchKernelGGL(k_gj_panel_reg, dim3(nbatch), dim3(nt), 0, s, a, n, 0, ipiv, moves(0), status);
-    for (int k = 0; k < nfull; ++k) {
-      const int next = k + 1 < nfull ? 1 : 0;
-      const int nrest = n - kPanelMax * (1 + next);
-      const int ngroups = (nrest + kPanelMax - 1) / kPanelMax;
-      const int nblk = (next ? nbatch : 0) + nbatch * ngroups;
-      if (nblk > 0)
-        hipLaunchKernelGGL(k_gj_step, dim3(nblk), dim3(nt), 0, s, a, n, k * kPanelMax, next,
-                           nbatch, ngroups, ipiv, (const int*)moves(k), moves(k + 1), status);
-    }
-    c0 = panel = nfull;
-    c0 *= kPanelMax;
-  }
-  // the remaining columns (every column when n > 768): panels in LDS, as many
-  // columns as fit next to the row map, at most 16, then a rank-nb update
+  // panels in LDS, as many columns as fit next to the row map, at most 16, then a
+  // rank-nb update
   const size_t budget = 160 * 1024 - 1024 - sizeof(int) * (size_t)n;
   const int nb = (int)std::min<size_t>(kPanelMax, budget / (sizeof(double2) * (size_t)n));
   RP_CHECK(nb >= 1, "Dyson: matrix too large for the LDS panel");
