@@ -43,6 +43,15 @@ void launch_pair_densities_pruned(const float2* ur, int ntk, const int* pocc, co
 void launch_pair_rsum(const float2* ur, int ntk, int nwf, bool full, int nx, int ny, int nz,
                       const int* ikq, const int* shift, const unsigned* kqs, const double2* wk,
                       int nq, double2* P, hipStream_t s);
+// The same on a regular k mesh n[3] that pair_kfft_mesh takes: kpos[k] is the mesh
+// position of k (first axis fastest, relative to k = 0), qof[position] the q whose
+// k+q lie that far from k or -1 (q0 .. q0+nq-1 are wanted), sk0[k][3] the k points,
+// qvec[position][3] the q vector there.
+bool pair_kfft_mesh(const int n[3], int ntk);
+void launch_pair_kfft(const float2* ur, int ntk, int nwf, bool full, int nx, int ny, int nz,
+                      const int n[3], const int* kpos, const int* qof, int q0, int nq,
+                      const double* sk0, const double* qvec, const double2* wk, double2* P,
+                      hipStream_t s);
 // k+q index (< 2^20) and umklapp vector (components -8..7) in one word, or
 // false when they do not fit
 inline bool pair_rsum_pack(int ikq, const int* d, unsigned* out) {

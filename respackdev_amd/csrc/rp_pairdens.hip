@@ -934,6 +934,182 @@ void launch_pair_densities_pruned(const float2* ur, int ntk, const int* pocc, co
   }
 }
 
+// The same sums on a regular k mesh of at most kKfftMax points as correlations over
+// the mesh: with psi_k = u_k e^{i 2pi k.r/N}, which is periodic in k,
+//   P(q, r) = e^{i 2pi q.r/N} sum_k w_k conj(psi_iw,k+q) psi_jw,k
+//           = e^{i 2pi q.r/N} / NTK  sum_m conj(A_i(m)) C_j(m) e^{-i 2pi q.m/n},
+// A and C the forward transforms over the mesh of psi_iw and w psi_jw.  That is NTK
+// (n1 + n2 + n3) products per (pair, r) instead of NTK^2.  A workgroup takes tr
+// grid points: A, C, the phases of q.r and pg pairs at a time in LDS, a thread one
+// line of up to eight mesh points in registers.  Bound by LDS (every axis reads and
+// writes each point once); rho with its transforms, 5 functions, k_pair_rsum_tile
+// before: 64 k, plane waves to 20 Ry in a 7 bohr cube, 70 -> 29 us (diagonal), 135 -> 60
+// (all pairs); 216 k, 30 Ry 851 -> 150 and 2140 -> 427; 8 k, 20 Ry 17 -> 16 and 24 -> 22.  More k do not fit with
+// every function's transforms; the line is drawn without regard to their number, so
+// that the same pairs among others come out the same.
+constexpr int kKfftMax = 256, kKfftAxis = 8;
+
+// Forward transform of a line, tw[m] = e^{-i 2pi m/N}.
+template <int N>
+__device__ __forceinline__ void kfft_line(const double2 (&v)[N], double2 (&o)[N], const double2* tw) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    double2 s = v[0];
+#pragma unroll
+    for (int j = 1; j < N; ++j) {
+      const int m = j * k % N;
+      if (m == 0) s = make_double2(s.x + v[j].x, s.y + v[j].y);
+      else if (2 * m == N) s = make_double2(s.x - v[j].x, s.y - v[j].y);
+      else if (4 * m == N) s = make_double2(s.x + v[j].y, s.y - v[j].x);
+      else if (4 * m == 3 * N) s = make_double2(s.x - v[j].y, s.y + v[j].x);
+      else {
+        const double2 t = tw[m];
+        s.x += v[j].x * t.x - v[j].y * t.y;
+        s.y += v[j].x * t.y + v[j].y * t.x;
+      }
+    }
+    o[k] = s;
+  }
+}
+
+// Every line of one axis (stride st) of `count` arrays of ntk x tr points: load(array,
+// point of the line) and store the same.
+template <int N, class Load, class Store>
+__device__ __forceinline__ void kfft_lines(int count, int ntk, int tr, int st, const double2* tw,
+                                           Load load, Store store) {
+  const int nl = ntk / N;
+  for (int x = threadIdx.x; x < count * nl * tr; x += 256) {
+    const int r = x % tr, l = x / tr, arr = l / nl, rem = l % nl;
+    const int p0 = rem / st * st * N + rem % st;
+    double2 v[N], o[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) v[j] = load(arr, p0 + j * st, r);
+    kfft_line<N>(v, o, tw);
+#pragma unroll
+    for (int j = 0; j < N; ++j) store(arr, p0 + j * st, r, o[j]);
+  }
+  __syncthreads();
+}
+
+template <class Load, class Store>
+__device__ __forceinline__ void kfft_axis(int n, int count, int ntk, int tr, int st,
+                                          const double2* tw, Load load, Store store) {
+  switch (n) {  // uniform
+    case 1: kfft_lines<1>(count, ntk, tr, st, tw, load, store); break;
+    case 2: kfft_lines<2>(count, ntk, tr, st, tw, load, store); break;
+    case 3: kfft_lines<3>(count, ntk, tr, st, tw, load, store); break;
+    case 4: kfft_lines<4>(count, ntk, tr, st, tw, load, store); break;
+    case 5: kfft_lines<5>(count, ntk, tr, st, tw, load, store); break;
+    case 6: kfft_lines<6>(count, ntk, tr, st, tw, load, store); break;
+    case 7: kfft_lines<7>(count, ntk, tr, st, tw, load, store); break;
+    default: kfft_lines<8>(count, ntk, tr, st, tw, load, store); break;
+  }
+}
+
+// grid (ceil(nr / tr)), 256 threads.  mesh: kpos[k], then qof[position]: the q of this
+// launch there, or -1; vec: sk0 of every k, then the vector of every position.
+__global__ void __launch_bounds__(256) k_pair_kfft(
+    const float2* __restrict__ ur, int ntk, int nwf, int full, int nx, int ny, int nz, int n1, int n2,
+    int n3, const int* __restrict__ kpos, const int* __restrict__ qof, int q0, int nq,
+    const double* __restrict__ sk0, const double* __restrict__ qvec, const double2* __restrict__ wk,
+    int tr, int pg, double2* __restrict__ P) {
+  extern __shared__ double2 kf[];
+  const int row = ntk * tr;
+  double2* tw = kf;                           // e^{-i 2pi m/n} per axis
+  double2* ph = tw + 3 * kKfftAxis;           // e^{i 2pi q.r/N} / NTK
+  double2* buf = ph + row;                    // [pg][ntk][tr]
+  double2* A = buf + (size_t)pg * row;        // [nwf][ntk][tr]
+  double2* C = wk ? A + (size_t)nwf * row : A;
+  const double tpi = 2.0 * 3.141592653589793238462643383279502884;
+  const int nr = nx * ny * nz, r0 = blockIdx.x * tr, t = threadIdx.x;
+  if (t < 3 * kKfftAxis) {
+    const int ax = t / kKfftAxis, m = t % kKfftAxis, n = ax == 0 ? n1 : (ax == 1 ? n2 : n3);
+    double sn, cs;
+    sincos(tpi * ((double)m / (double)n), &sn, &cs);
+    tw[t] = make_double2(cs, -sn);
+  }
+  for (int e = t; e < row; e += 256) {
+    const int k = e / tr, r = min(r0 + e % tr, nr - 1);
+    const double x = (double)(r % nx) / nx, y = (double)(r / nx % ny) / ny,
+                 z = (double)(r / (nx * ny)) / nz;
+    double sn, cs;
+    sincos(tpi * (qvec[3 * k] * x + qvec[3 * k + 1] * y + qvec[3 * k + 2] * z), &sn, &cs);
+    ph[e] = make_double2(cs / ntk, sn / ntk);
+    sincos(tpi * (sk0[3 * k] * x + sk0[3 * k + 1] * y + sk0[3 * k + 2] * z), &sn, &cs);
+    const double2 wv = wk ? wk[k] : make_double2(1.0, 0.0);
+    const int o = kpos[k] * tr + e % tr;
+    for (int w = 0; w < nwf; ++w) {
+      const float2 u = ur[((size_t)w * ntk + k) * nr + r];
+      const double2 v = make_double2((double)u.x * cs - (double)u.y * sn,
+                                     (double)u.x * sn + (double)u.y * cs);
+      A[w * row + o] = v;
+      if (wk) C[w * row + o] = make_double2(v.x * wv.x - v.y * wv.y, v.x * wv.y + v.y * wv.x);
+    }
+  }
+  __syncthreads();
+  {
+    auto at = [&](int a, int p, int r) { return A[a * row + p * tr + r]; };
+    auto put = [&](int a, int p, int r, double2 v) { A[a * row + p * tr + r] = v; };
+    const int na = wk ? 2 * nwf : nwf;  // C follows A
+    kfft_axis(n1, na, ntk, tr, 1, tw, at, put);
+    kfft_axis(n2, na, ntk, tr, n1, tw + kKfftAxis, at, put);
+    kfft_axis(n3, na, ntk, tr, n1 * n2, tw + 2 * kKfftAxis, at, put);
+  }
+  const int npair = full ? nwf * nwf : nwf;
+  auto at = [&](int a, int p, int r) { return buf[a * row + p * tr + r]; };
+  auto put = [&](int a, int p, int r, double2 v) { buf[a * row + p * tr + r] = v; };
+  for (int pb = 0; pb < npair; pb += pg) {
+    const int np = min(pg, npair - pb);
+    auto product = [&](int a, int p, int r) {
+      const int pr = pb + a, iw = full ? pr % nwf : pr, jw = full ? pr / nwf : pr;
+      const double2 b = A[iw * row + p * tr + r], c = C[jw * row + p * tr + r];
+      return make_double2(b.x * c.x + b.y * c.y, b.x * c.y - b.y * c.x);
+    };
+    auto out = [&](int a, int p, int r, double2 v) {
+      const int q = qof[p] - q0;
+      if (q < 0 || q >= nq || r0 + r >= nr) return;
+      const double2 f = ph[p * tr + r];
+      P[((size_t)q * npair + pb + a) * nr + r0 + r] =
+          make_double2(v.x * f.x - v.y * f.y, v.x * f.y + v.y * f.x);
+    };
+    kfft_axis(n1, np, ntk, tr, 1, tw, product, put);
+    kfft_axis(n2, np, ntk, tr, n1, tw + kKfftAxis, at, put);
+    kfft_axis(n3, np, ntk, tr, n1 * n2, tw + 2 * kKfftAxis, at, out);
+  }
+}
+
+bool pair_kfft_mesh(const int n[3], int ntk) {
+  return n[0] * n[1] * n[2] == ntk && ntk <= kKfftMax && std::max({n[0], n[1], n[2]}) <= kKfftAxis;
+}
+
+void launch_pair_kfft(const float2* ur, int ntk, int nwf, bool full, int nx, int ny, int nz,
+                      const int n[3], const int* kpos, const int* qof, int q0, int nq,
+                      const double* sk0, const double* qvec, const double2* wk, double2* P,
+                      hipStream_t s) {
+  RP_CHECK(nwf >= 1 && nwf <= 16, "Wannier pair sums take at most 16 Wannier functions");
+  RP_CHECK(pair_kfft_mesh(n, ntk), "k mesh too large for the correlation sums");
+  if (nq <= 0) return;
+  const int nr = nx * ny * nz;
+  // As many grid points (up to 8) as leave two workgroups per CU, and as many pairs at
+  // a time (up to 8) as have a line each for the threads.
+  const size_t unit = sizeof(double2) * (size_t)ntk, fixed = sizeof(double2) * 3 * kKfftAxis;
+  const size_t arrays = 1 + (wk ? 2 : 1) * (size_t)nwf;
+  int tr = 8;
+  while (tr > 1 && fixed + unit * tr * (arrays + 4) > kLdsBytes / 2) tr /= 2;
+  const int lines = ntk / std::min({n[0], n[1], n[2]}) * tr;
+  const int room = (int)((kLdsBytes - fixed) / (unit * tr)) - (int)arrays;
+  const int pg = std::max(1, std::min({8, 256 / lines, room}));
+  const size_t lds = fixed + unit * tr * (arrays + pg);
+  RP_CHECK(lds <= kLdsBytes, "k mesh too large for the correlation sums");
+  if (lds > 65536)
+    RP_HIP(hipFuncSetAttribute((const void*)k_pair_kfft, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+  hipLaunchKernelGGL(k_pair_kfft, dim3((nr + tr - 1) / tr), dim3(256), lds, s, ur, ntk, nwf,
+                     full ? 1 : 0, nx, ny, nz, n[0], n[1], n[2], kpos, qof, q0, nq, sk0, qvec, wk, tr,
+                     pg, P);
+  RP_HIP(hipGetLastError());
+}
+
 void launch_pair_rsum(const float2* ur, int ntk, int nwf, bool full, int nx, int ny, int nz,
                       const int* ikq, const int* shift, const unsigned* kqs, const double2* wk,
                       int nq, double2* P, hipStream_t s) {

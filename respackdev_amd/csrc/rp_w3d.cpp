@@ -68,6 +68,10 @@ struct W3d {
   DevBuf<int> d_geo_ikq, d_geo_shift, d_geo_plan, d_geo_g0, d_ngpsi, d_geo_lg;
   DevBuf<unsigned> d_geo_kqs;  // ikq and shift packed (pair_rsum_pack; empty if they do not fit)
   DevBuf<long long> d_geo_qg_off, d_geo_plan_off;
+  // the k mesh of launch_pair_kfft (geo_mesh[0] = 0: not one it takes)
+  int geo_mesh[3] = {0, 0, 0};
+  DevBuf<int> d_geo_kpos, d_geo_qof;
+  DevBuf<double> d_geo_sk0, d_geo_qvec;
   // summed pair-density grids P[q][p][r] of a chunk of q (launch_pair_rsum)
   DevBuf<double2> d_P;
   // exchange (rp_j3d_run): work buffers kept between calls, sized to a batch of R
@@ -216,6 +220,52 @@ QGeom q_geometry(const W3d& w, int iq) {
   return r;
 }
 
+// The k points as a regular mesh, for the pair sums as correlations over it: true if
+// every k is at a mesh position of its own, k + q at that of k moved by the same
+// amount for every k, and k + q less its umklapp vector the same q.  kpos, qof and
+// qvec as launch_pair_kfft takes them.
+bool mesh_plan(const W3d& w, const std::vector<int>& ikq, const std::vector<int>& shift, int n[3],
+               std::vector<int>& kpos, std::vector<int>& qof, std::vector<double>& qvec) {
+  for (int d = 0; d < 3; ++d) n[d] = w.nkb[d];
+  if (n[0] < 1 || n[1] < 1 || n[2] < 1 || !pair_kfft_mesh(n, w.ntk)) return false;
+  kpos.assign(w.ntk, 0);
+  std::vector<char> seen(w.ntk, 0);
+  std::vector<int> m(3 * (size_t)w.ntk);
+  for (int k = 0; k < w.ntk; ++k) {
+    for (int d = 0; d < 3; ++d) {
+      const double x = (w.sk0[3 * k + d] - w.sk0[d]) * n[d], r = std::round(x);
+      if (!(std::fabs(x - r) < 1e-6 * n[d])) return false;
+      m[3 * k + d] = (((int)r) % n[d] + n[d]) % n[d];
+    }
+    kpos[k] = m[3 * k] + n[0] * (m[3 * k + 1] + n[1] * m[3 * k + 2]);
+    if (seen[kpos[k]]++) return false;
+  }
+  qof.assign(w.ntk, -1);
+  qvec.assign(3 * (size_t)w.ntk, 0.0);
+  for (int q = 0; q < w.ntq; ++q) {
+    int mq[3];
+    double v[3];
+    for (int k = 0; k < w.ntk; ++k) {
+      const size_t i = (size_t)q * w.ntk + k;
+      for (int d = 0; d < 3; ++d) {
+        const int dm = (m[3 * ikq[i] + d] - m[3 * k + d] + n[d]) % n[d];
+        const double dv = w.sk0[3 * ikq[i] + d] + shift[3 * i + d] - w.sk0[3 * k + d];
+        if (k == 0) {
+          mq[d] = dm;
+          v[d] = dv;
+        } else if (dm != mq[d] || !(std::fabs(dv - v[d]) < 1e-12)) {
+          return false;
+        }
+      }
+    }
+    const int p = mq[0] + n[0] * (mq[1] + n[1] * mq[2]);
+    if (qof[p] >= 0) return false;
+    qof[p] = q;
+    for (int d = 0; d < 3; ++d) qvec[3 * p + d] = v[d];
+  }
+  return true;
+}
+
 // Every q's pair-density inputs in HBM, so that the loops over q only launch.
 void ensure_geometry(W3d& w, hipStream_t s) {
   if (w.geo_ready) return;
@@ -253,6 +303,16 @@ void ensure_geometry(W3d& w, hipStream_t s) {
   for (size_t i = 0; i < ikq.size() && packed; ++i) packed = pair_rsum_pack(ikq[i], &shift[3 * i], &kqs[i]);
   if (packed) w.d_geo_kqs.upload(kqs, s);
   else w.d_geo_kqs.release();
+  std::vector<int> kpos, qof;
+  std::vector<double> qvec;
+  if (mesh_plan(w, ikq, shift, w.geo_mesh, kpos, qof, qvec)) {
+    w.d_geo_kpos.upload(kpos, s);
+    w.d_geo_qof.upload(qof, s);
+    w.d_geo_sk0.upload(w.sk0, s);
+    w.d_geo_qvec.upload(qvec, s);
+  } else {
+    w.geo_mesh[0] = 0;
+  }
   w.d_geo_plan.upload(plan, s);
   w.d_geo_qg_off.upload(w.geo_qg_off, s);
   w.d_geo_plan_off.upload(w.geo_plan_off, s);
@@ -279,7 +339,12 @@ void rho_all_q(W3d& w, bool full, const double2* wk, const long long* d_rho_off,
   w.d_P.reserve((size_t)qchunk * npair * nr);
   for (int q0 = 0; q0 < w.ntq; q0 += qchunk) {
     const int nq = std::min(qchunk, w.ntq - q0);
-    launch_pair_rsum(w.d_ur.p, w.ntk, w.nwf, full, w.nw[0], w.nw[1], w.nw[2],
+    if (w.geo_mesh[0] > 0)  // faster at every size it takes
+      launch_pair_kfft(w.d_ur.p, w.ntk, w.nwf, full, w.nw[0], w.nw[1], w.nw[2], w.geo_mesh,
+                       w.d_geo_kpos.p, w.d_geo_qof.p, q0, nq, w.d_geo_sk0.p, w.d_geo_qvec.p, wk,
+                       w.d_P.p, s);
+    else
+      launch_pair_rsum(w.d_ur.p, w.ntk, w.nwf, full, w.nw[0], w.nw[1], w.nw[2],
                      w.d_geo_ikq.p + (size_t)q0 * w.ntk, w.d_geo_shift.p + (size_t)3 * q0 * w.ntk,
                      w.d_geo_kqs.n ? w.d_geo_kqs.p + (size_t)q0 * w.ntk : nullptr, wk, nq,
                      w.d_P.p, s);
