@@ -2,7 +2,7 @@
 // integrals V_ij(R), W_ij(R,w) of calc_intW.F:636-985.
 //
 // rho_w(q+G) = (1/NTK) sum_k M_ww,k(G) / |q+G| comes from the pair-density
-// kernels of rp_pairdens.hip (k_pair_rsum, k_rho_from_grid: the products summed
+// kernels of rp_pairdens.hip (k_pair_kfft or k_pair_rsum, k_rho_from_grid: the products summed
 // over k on the grid, one transform per (q, pair)).  Then per full-mesh q (all
 // q of one launch):
 //   func_ij(q)     = sum_{G in psi} rho_i(G) conj(rho_j(G))                (k_w_func)
