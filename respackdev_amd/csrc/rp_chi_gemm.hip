@@ -1,18 +1,16 @@
 // chi_GG'(q,w) = sum_K conj(A[K][G]) d[w][K] A[K][G'] on gfx950 MFMA.
 //
 // This is the accumulation of chiqw.F:1397-1410 restated as a rank-K update
-// per frequency (K = pair*NTK + k).  The complex product is mapped onto real
-// MFMA by doubling K: with a = A[K][G], b = d A[K][G'],
-//   Re chi += Re a Re b + Im a Im b,   Im chi += Re a Im b - Im a Re b,
-// i.e. one real GEMM whose k-slots hold (Re a | Im a) against (Re b | Im b)
-// for the real part and (Im b | -Re b) for the imaginary part.
+// per frequency (K = pair*NTK + k), a = A[K][G], b = d A[K][G'],
+//   Re chi += Re a Re b + Im a Im b,   Im chi += Re a Im b - Im a Re b.
 //
-// Workgroup: 256 threads (2x2 waves), tile 64 G x 64 G' for one frequency;
-// each wave owns 2x2 MFMA blocks of 16x16.  Precisions:
+// Workgroup: 256 threads, tile 64 G x 64 G' for one frequency.  Precisions:
 //   FP64   k_chi_f64: v_mfma_f64_16x16x4f64, FP64 accumulators, the complex
-//          product as three real ones.
-//   FP32   k_chi_gemm: v_mfma_f32_16x16x4f32; FP32 accumulators flushed into
-//          FP64 ones every kFlush chunks.
+//          product as three real ones, the tile's 16-blocks dealt to the waves.
+//   FP32   k_chi_gemm: v_mfma_f32_16x16x4f32, 2x2 waves of 2x2 blocks; one real
+//          product of twice the K, whose k-slots hold (Re a | Im a) against
+//          (Re b | Im b) for the real part and (Im b | -Re b) for the imaginary
+//          part; FP32 accumulators flushed into FP64 ones every kFlush chunks.
 // (The split-BF16 precision has its own kernel, k_chi_bf16x3.)
 // The K range may be split over gridDim.z; partial tiles are summed in fixed
 // order by k_chi_reduce (deterministic), which also divides by the volume.
@@ -147,8 +145,13 @@ __global__ void __launch_bounds__(256) k_chi_gemm(const float2* __restrict__ A, 
 // One output tile in FP64.  With b = d a(G') the complex product conj(a) b is
 // three real ones (three real MFMAs per block and 4 K where the direct form
 // needs four):
-//   T1 = ar br,  T2 = ai bi,  T3 = (ar - ai)(br + bi),
-//   Re = T1 + T2,  Im = T3 - T1 + T2.
+//   T1 = ar bi,  T2 = ai br,  T3 = (ar + ai)(br + bi),
+//   Im = T1 - T2,  Re = T3 - T1 - T2.
+// T1 and T2 have terms of either sign (the phase of a row of A is its
+// eigenvectors' arbitrary one) and stay of the order of Im, so that Im carries no
+// rounding of the many times larger Re.  (With T1 = ar br, T2 = ai bi and
+// T3 = (ar - ai)(br + bi), T1 - T2 is small and T1, T2 are half of Re each: Im is
+// then off by three to five times as much.)
 // FP64 MFMAs and FP64 vector instructions share one unit per SIMD (run
 // together they reach 58 TFLOP/s, the MFMAs alone 79), so every vector
 // operation on the operands costs matrix time: the three left and three right
@@ -163,9 +166,10 @@ __global__ void __launch_bounds__(256) k_chi_gemm(const float2* __restrict__ A, 
 // 108.5 ms).  Four workgroups per CU hide the staging, hence 8 K per chunk and
 // 128 registers: three (more registers, 8 K) 68.3 ms, two (16 K) 71 ms, two with
 // 128 x 64 tiles and fewer vector operations 75.6 ms, two double-buffered 78 ms.
-// Error against long double, relative norm: 7.8e-16 (direct form 6.6e-15; the
-// imaginary part alone, 50 times smaller than the real part here, 3e-14 against
-// 9e-15 of its own norm).
+// Error against long double, each part by its own norm, at that size: Re 7e-16 to
+// 1e-15, Im 1.3e-15 to 3.1e-15 (direct form 5e-15 to 7e-15 and 1.0e-14; the other
+// three products 3.2e-15 to 1.6e-14 for Im); K 1296 to 6144, NG 81 to 126: Re 2.0e-16,
+// Im 2.9e-16 to 4.7e-16 (2.0e-16 and 4.1e-16 to 6.2e-16; 1.0e-15 to 1.4e-15).
 //
 // The right block is the MFMA's first operand, so that D(row, col) =
 // (G', G) and the lanes of a result run along G, the fastest index of out.
@@ -253,11 +257,11 @@ __global__ void __launch_bounds__(256, 4) k_chi_f64(const float2* __restrict__ A
       const double ar = la[e].x, ai = la[e].y;
       sl[o] = ar;
       sl[kF64Plane + o] = ai;
-      sl[2 * kF64Plane + o] = ar - ai;
+      sl[2 * kF64Plane + o] = ar + ai;
       const double cr = ra[e].x, ci = ra[e].y;
       const double br = dv[e].x * cr - dv[e].y * ci, bi = dv[e].x * ci + dv[e].y * cr;
-      sr[o] = br;
-      sr[kF64Plane + o] = bi;
+      sr[o] = bi;
+      sr[kF64Plane + o] = br;
       sr[2 * kF64Plane + o] = br + bi;
     }
   };
@@ -290,7 +294,7 @@ __global__ void __launch_bounds__(256, 4) k_chi_f64(const float2* __restrict__ A
           const int hj = h0 + (cb + b) * 16 + lk + 4 * v;
           const int i = a * NC + b;
           const double t1 = acc[0][i][v], t2 = acc[1][i][v], t3 = acc[2][i][v];
-          if (gi < ng && hj < ncol) o[(size_t)hj * ng + gi] = make_double2(t1 + t2, t3 - t1 + t2);
+          if (gi < ng && hj < ncol) o[(size_t)hj * ng + gi] = make_double2(t3 - t1 - t2, t1 - t2);
         }
   };
   using std::integral_constant;
@@ -362,7 +366,9 @@ __global__ void k_chi_reduce_cross(const double2* __restrict__ part, int ng, int
 int chi_tile() { return kTile; }
 int chi_kchunk() { return kKC; }
 
-// K splits.  FP32: enough for 2048 workgroups.  FP64: with W workgroups per
+// K splits.  FP32: enough for 2048 workgroups.  FP64: at least as many, for the
+// rounding of a sum falls with its splits (K 1296, NG 81: 9 splits left the real
+// part off by 2.6e-16, 37 by 1.9e-16), and more where they are faster: with W workgroups per
 // split, S = 4 resident per CU and C chunks of 32 K, a launch takes about
 //   (W sp / S + 1/2 round of tail) (C / sp + 2 chunks of start and end)
 // chunk times of a full CU (5.2 us: four workgroups' MFMAs), plus the traffic
@@ -376,7 +382,8 @@ int chi_gemm_nsplit(int prec, int ng, int nen, size_t kpad, int ncu) {
   const double per = 16.0 * ng * ng * nen;  // bytes of one partial set
   const double cost = 2.0 * (double)wgs / (4.0 * ncu) + 2.0 * per / 4.5e6 / 5.2;
   const double sp = std::min(std::sqrt(0.5 * (double)kchunks / cost), 2147483648.0 / per);
-  return (int)std::max(1.0, std::min((double)std::min<long>(kchunks, 64), std::round(sp)));
+  const long fast = (long)std::max(1.0, std::min(64.0, std::round(sp)));
+  return (int)std::min(kchunks, std::max(fast, (2048 + wgs - 1) / wgs));
 }
 
 void launch_chi_gemm(int prec, const float2* A, size_t lda, const double2* dw, size_t ldd,
@@ -440,8 +447,9 @@ void launch_chi_head(const float2* A, size_t lda, const double2* dw, size_t ldd,
                      double2* partial, size_t room, double2* chi, hipStream_t s) {
   const int ntile = (ng + kTile - 1) / kTile, ctile = (2 * nen + kTile - 1) / kTile;
   const size_t kchunks = kpad / kF64KC;
-  // a split of at least 16 chunks each, at most 64, within the partials' room
-  size_t nsplit = std::min<size_t>(std::max<size_t>(1, kchunks / 16), 64);
+  // splits of at least 4 chunks (short sums round less), at most 64 of them, within the
+  // partials' room
+  size_t nsplit = std::min<size_t>(std::max<size_t>(1, kchunks / 4), 64);
   nsplit = std::min(nsplit, room / ((size_t)2 * nen * ng));
   RP_CHECK(nsplit >= 1, "chi head: no room for its partials");
   const size_t per = (kchunks + nsplit - 1) / nsplit;
