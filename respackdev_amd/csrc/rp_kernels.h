@@ -163,7 +163,10 @@ void launch_w_contract(const float2* eps, const long long* eps_off, const double
                        const double2* shell, const int* goff, const int* gmem, int ngroups,
                        int nwf, int nen, int max_nge, double2* xw, double2* funcw,
                        hipStream_t s);
-// xg: scratch of j_contract_scratch(sum over q of NG_eps, npair) complex values
+// The exchange contraction of a batch of nr R (rp_w3d.hip): groups holds one
+// pack_j_group entry (j_group_bytes) per irreducible q, gmem their members; xs and zs
+// have room for the groups' j_x_elems and j_z_elems, funcw for nrs (j_row_shares)
+// partial sums per (R, q, w, pair).
 size_t j_x_elems(int nge, int ncol);
 size_t j_z_elems(int nge, int ncol);
 int j_row_shares(int ngroups, int nen, int max_ncol, int max_nge, int ncu);

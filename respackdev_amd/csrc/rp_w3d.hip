@@ -75,16 +75,20 @@ __global__ void __launch_bounds__(256) k_w_func(const double2* __restrict__ rho,
 // k_j_contract (Re Y = Er Xr - Ei Xi, Im Y = Er Xi + Ei Xr, v_mfma_f64_16x16x4,
 // the group's vectors as one 16-column block): lane l supplies A(l % 16, l / 16)
 // and B(l / 16, l % 16) and holds D(l / 16 + 4 v, l % 16).  X of every group
-// is formed once (k_w_xvec, independent of w).  A wave takes one 16-row block
-// of E per pass over all columns; then each lane multiplies its four Y(a, c)
+// is formed once (k_w_xvec, independent of w).  A wave takes up to kWA 16-row
+// blocks of E per pass over all columns; then each lane multiplies its Y(a, c)
 // by the Z_i(a) of c's member and keeps NV sums, reduced over the lanes of
 // c and the waves at the end.
+// Bound by the FP64 matrix cores, with 10 to 15 of the 16 columns in use: 64 q, 20
+// frequencies, five functions, NG_eps ~ 310: 190 us with three row blocks per wave, 243
+// with two, 218 with four; with the loads two steps ahead instead of one 212.  Three real
+// products per complex one take 187 us, but Im Y = T3 - T1 - T2 left Im W of a diagonal
+// pair 4 to 10 times further off by its own norm.
 // grid: (nen, ngroups), 512 threads; group g has the q gmem[goff[g] .. goff[g+1]).
 typedef double jd4 __attribute__((ext_vector_type(4)));
 constexpr int kMaxWf = 16;     // Wannier functions of calc_w3d and calc_j3d
 constexpr int kWcVec = 16;     // vectors of a group: one MFMA column block
 constexpr int kWA = 3;         // row blocks per wave and pass of the W contraction
-constexpr int kWD = 2;         // steps its loads run ahead
 template <int NV>
 constexpr int wc_members() { return kWcVec / NV; }
 int w_contract_members(int nwf) { return kWcVec / nwf; }
@@ -160,46 +164,43 @@ __global__ void __launch_bounds__(512) k_w_contract(
   // up to kWA row blocks per wave and pass (ab = a0 + wave + 8 j) share each
   // load of X; blocks past the last are skipped (uniform per wave)
   for (int a0 = 0; a0 < nab; a0 += 8 * kWA) {
-    jd4 t1[kWA], t2[kWA], t3[kWA];
+    jd4 accr[kWA], acci[kWA];
     int arow[kWA];
 #pragma unroll
     for (int j = 0; j < kWA; ++j) {
-      t1[j] = t2[j] = t3[j] = jd4{0.0, 0.0, 0.0, 0.0};
+      accr[j] = acci[j] = jd4{0.0, 0.0, 0.0, 0.0};
       // rows nge .. ld-1 are the zero padding; their sums are never used
       arow[j] = (a0 + wave + 8 * j) * 16 + li;
     }
     const int nj = min(kWA, (nab - a0 - wave + 7) / 8);  // live blocks of this wave
-    // X and E of the step kWD steps ahead are loaded during a step's MFMAs;
-    // columns past nge contribute zero
-    double2 xq[kWD];
-    float2 eq[kWD][kWA];
-    auto fetch = [&](int b0, int slot) {
+    // X and E of the next step are loaded during a step's MFMAs; columns past nge
+    // contribute zero
+    double2 xq;
+    float2 eq[kWA];
+    auto fetch = [&](int b0) {
       const int b = min(b0 + lk, nge - 1);
-      xq[slot] = Xg[(size_t)b * kWcVec + li];
+      xq = Xg[(size_t)b * kWcVec + li];
 #pragma unroll
-      for (int j = 0; j < kWA; ++j) eq[slot][j] = j < nj ? E[(size_t)b * ld + arow[j]] : make_float2(0.f, 0.f);
+      for (int j = 0; j < kWA; ++j) eq[j] = j < nj ? E[(size_t)b * ld + arow[j]] : make_float2(0.f, 0.f);
     };
+    fetch(0);
+    for (int b0 = 0; b0 < nge; b0 += 4) {
+      const bool bv = b0 + lk < nge;
+      const double xr = bv ? xq.x : 0.0, xi = bv ? xq.y : 0.0, nxi = -xi;
+      double er[kWA], ei[kWA];
 #pragma unroll
-    for (int d = 0; d < kWD; ++d) fetch(4 * d, d);
-    for (int b0 = 0; b0 < nge; b0 += 4 * kWD) {
+      for (int j = 0; j < kWA; ++j) {
+        er[j] = eq[j].x;
+        ei[j] = eq[j].y;
+      }
+      fetch(b0 + 4);
 #pragma unroll
-      for (int d = 0; d < kWD; ++d) {
-        const bool bv = b0 + 4 * d + lk < nge;
-        const double xr = bv ? xq[d].x : 0.0, xi = bv ? xq[d].y : 0.0, xs = xr + xi;
-        double er[kWA], ei[kWA];
-#pragma unroll
-        for (int j = 0; j < kWA; ++j) {
-          er[j] = eq[d][j].x;
-          ei[j] = eq[d][j].y;
-        }
-        fetch(b0 + 4 * (d + kWD), d);
-#pragma unroll
-        for (int j = 0; j < kWA; ++j) {
-          if (j >= nj) break;  // uniform
-          t1[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[j], xr, t1[j], 0, 0, 0);
-          t2[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[j], xi, t2[j], 0, 0, 0);
-          t3[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[j] + ei[j], xs, t3[j], 0, 0, 0);
-        }
+      for (int j = 0; j < kWA; ++j) {
+        if (j >= nj) break;  // uniform
+        accr[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[j], xr, accr[j], 0, 0, 0);
+        acci[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[j], xi, acci[j], 0, 0, 0);
+        accr[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[j], nxi, accr[j], 0, 0, 0);
+        acci[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[j], xr, acci[j], 0, 0, 0);
       }
     }
     // Z_i(a) Y(a, c) for this lane's rows a = 16 ab + lk + 4 v and vector c = li
@@ -213,7 +214,7 @@ __global__ void __launch_bounds__(512) k_w_contract(
           const int ar = ab * 16 + lk + 4 * v;
           if (ar >= nge) continue;
           const int g = minv[mom + ar];
-          const double yr = t1[j][v] - t2[j][v], yi = t3[j][v] - t1[j][v] - t2[j][v];
+          const double yr = accr[j][v], yi = acci[j][v];
           const double2 pp = qim.w == 1 ? pf1[mom + g] : pf2[mom + g];
 #pragma unroll
           for (int i = 0; i < NV; ++i) {
@@ -275,17 +276,17 @@ __global__ void __launch_bounds__(512) k_w_contract(
 // q and seven R all but two of 352).
 //
 // k_j_vecs forms once per batch, for every group, X [nbp][cpad] (nbp: NG_eps
-// rounded up to 8 rows, cpad: the columns to 16, zero beyond) and Z [NG_eps][cpad].  k_j_contract then takes 64 columns of one
-// (group, w): Y = E X as three real products, Re Y = T1 - T2, Im Y = T3 - T1 - T2
-// with T1 = er xr, T2 = ei xi, T3 = (er + ei)(xr + xi), over tiles of up to 64
-// rows and 8 columns of E at a time staged in LDS, and folds each tile into the
-// sums over rows Z_c(a) Y(a, c).  A wave takes one column block of 16 and every
-// row block of the tile (with fewer column blocks the rows are dealt out).
-// Bound by the FP64 MFMAs (shared with the FP64 vector unit, hence planes formed
-// once per workgroup): 64 q, 16 frequencies, 25 pairs, NG_eps ~310: seven
-// R 2.01 ms (52 TFLOP/s executed; 4.20 ms with every (q, R) on its own and four
-// real products), one R 0.37 ms (0.59).  Three workgroups per CU; two take 2.18
-// ms, four spill.
+// rounded up to 8 rows, cpad: the columns to 16, zero beyond) and Z [NG_eps][cpad].
+// k_j_contract then takes 64 columns of one (group, w): Y = E X as real products
+// (Re Y = Er Xr - Ei Xi, Im Y = Er Xi + Ei Xr) over tiles of up to 64 rows and 8
+// columns of E at a time staged in LDS, and folds each tile into the sums over rows
+// Z_c(a) Y(a, c).  A wave takes one column block of 16 and every row block of the
+// tile (with fewer column blocks the rows are dealt out).  Bound by the FP64 MFMAs
+// (shared with the FP64 vector unit, hence E and X widened once per workgroup): 64 q,
+// 16 frequencies, 25 pairs, NG_eps ~310, seven R: 2.28 ms (60 TFLOP/s; 4.16 ms with
+// every (q, R) on its own).  Four workgroups per CU; three take 2.41 ms; 12 columns of E
+// at a time 2.55.  Three real products per complex one take 1.98 ms, but leave Im J
+// further off (as Im W of k_w_contract).
 constexpr int kJT = 64, kJKC = 8;                 // rows / columns of a tile, K per chunk
 constexpr int kJRow = kJT + 16, kJPlane = kJKC * kJRow;
 
@@ -343,31 +344,39 @@ __global__ void __launch_bounds__(256) k_j_vecs(const double2* __restrict__ rho,
 // NR row blocks from block rb on by the column block cb of a staged chunk.
 template <int NR>
 __device__ __forceinline__ void j_chunk(const double* pe, const double* px, int rb, int cb, int li,
-                                        int lk, jd4 (&acc)[3][NR]) {
+                                        int lk, jd4 (&re)[NR], jd4 (&im)[NR]) {
 #pragma unroll
-  for (int k0 = 0; k0 < kJKC; k0 += 4)
+  for (int k0 = 0; k0 < kJKC; k0 += 4) {
+    const int o = (k0 + lk) * kJRow + li;
+    const double xr = px[o + 16 * cb], xi = px[kJPlane + o + 16 * cb], nxi = -xi;
+    double er[NR], ei[NR];
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      const int o = p * kJPlane + (k0 + lk) * kJRow + li;
-      const double x = px[o + 16 * cb];
-      double e[NR];
-#pragma unroll
-      for (int a = 0; a < NR; ++a) e[a] = pe[o + 16 * (rb + a)];
-#pragma unroll
-      for (int a = 0; a < NR; ++a)
-        acc[p][a] = __builtin_amdgcn_mfma_f64_16x16x4f64(e[a], x, acc[p][a], 0, 0, 0);
+    for (int a = 0; a < NR; ++a) {
+      er[a] = pe[o + 16 * (rb + a)];
+      ei[a] = pe[kJPlane + o + 16 * (rb + a)];
     }
+#pragma unroll
+    for (int a = 0; a < NR; ++a) {
+      re[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[a], xr, re[a], 0, 0, 0);
+      im[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(er[a], xi, im[a], 0, 0, 0);
+    }
+#pragma unroll
+    for (int a = 0; a < NR; ++a) {
+      re[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[a], nxi, re[a], 0, 0, 0);
+      im[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(ei[a], xr, im[a], 0, 0, 0);
+    }
+  }
 }
 
 // grid: (nen, groups, column tiles of the widest group x nrs), 256 threads; row
 // tile t of a workgroup with row share s (of nrs) is taken when t % nrs == s.
 // out[s][R][q][w][p]: the partial sums over that share's rows.
-__global__ void __launch_bounds__(256, 3) k_j_contract(
+__global__ void __launch_bounds__(256, 4) k_j_contract(
     const float2* __restrict__ eps, const long long* __restrict__ eps_off,
     const JGroup* __restrict__ grp, const int* __restrict__ gmem, const double2* __restrict__ xs,
     const double2* __restrict__ zs, int np, int nr, int nrs, int ntq, int nen,
     double2* __restrict__ out) {
-  __shared__ double se[3 * kJPlane], sx[3 * kJPlane];
+  __shared__ double se[2 * kJPlane], sx[2 * kJPlane];
   __shared__ double2 red[4][16];
   const int w = blockIdx.x, rs = (int)blockIdx.z % nrs, tc = (int)blockIdx.z / nrs;
   const JGroup g = grp[blockIdx.y];
@@ -404,27 +413,22 @@ __global__ void __launch_bounds__(256, 3) k_j_contract(
   // stages); next: first row of the workgroup's next tile, < 0 for none
   auto tile = [&](auto rows, int ab, int rb, int next) {
     constexpr int NR = decltype(rows)::value;
-    jd4 acc[3][NR > 0 ? NR : 1];
+    jd4 re[NR > 0 ? NR : 1], im[NR > 0 ? NR : 1];
 #pragma unroll
-    for (int p = 0; p < 3; ++p)
-#pragma unroll
-      for (int a = 0; a < NR; ++a) acc[p][a] = jd4{0, 0, 0, 0};
+    for (int a = 0; a < NR; ++a) re[a] = im[a] = jd4{0, 0, 0, 0};
     for (int b0 = 0; b0 < nbp; b0 += kJKC) {
 #pragma unroll
       for (int e = 0; e < kJKC / 4; ++e) {
         const int o = (wave + 4 * e) * kJRow + lane;
-        const double er = ev[e].x, ei = ev[e].y;
-        se[o] = er;
-        se[kJPlane + o] = ei;
-        se[2 * kJPlane + o] = er + ei;
+        se[o] = ev[e].x;
+        se[kJPlane + o] = ev[e].y;
         sx[o] = xv[e].x;
         sx[kJPlane + o] = xv[e].y;
-        sx[2 * kJPlane + o] = xv[e].x + xv[e].y;
       }
       __syncthreads();
       if (b0 + kJKC < nbp) load(16 * ab, b0 + kJKC);
       else if (next >= 0) load(next, 0);
-      if constexpr (NR > 0) j_chunk<NR>(se, sx, rb, cb, li, lk, acc);
+      if constexpr (NR > 0) j_chunk<NR>(se, sx, rb, cb, li, lk, re, im);
       __syncthreads();
     }
     const int c = 16 * (hb + cb) + li;
@@ -434,8 +438,7 @@ __global__ void __launch_bounds__(256, 3) k_j_contract(
       for (int v = 0; v < 4; ++v) {
         const int ar = 16 * (ab + rb + a) + lk + 4 * v;
         if (ar >= g.nge) continue;
-        const double yr = acc[0][a][v] - acc[1][a][v];
-        const double yi = acc[2][a][v] - acc[0][a][v] - acc[1][a][v];
+        const double yr = re[a][v], yi = im[a][v];
         const double2 z = Z[(size_t)ar * cpad + c];
         sre += z.x * yr - z.y * yi;
         sim += z.x * yi + z.y * yr;
@@ -674,7 +677,7 @@ int j_row_shares(int ngroups, int nen, int max_ncol, int max_nge, int ncu) {
 }
 
 // groups: device array of ngroups {nge, iq_irr, first member, columns, X offset,
-// Z offset} as pack_j_groups lays them out; nr R of the batch, rho_r apart.
+// Z offset} as pack_j_group lays them out; nr R of the batch, rho_r apart.
 size_t j_group_bytes() { return sizeof(JGroup); }
 void pack_j_group(void* at, int nge, int iqir, int mbeg, int ncol, long long xoff, long long zoff) {
   *(JGroup*)at = JGroup{nge, iqir, mbeg, ncol, xoff, zoff};
