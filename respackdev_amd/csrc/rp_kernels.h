@@ -45,13 +45,16 @@ void launch_pair_rsum(const float2* ur, int ntk, int nwf, bool full, int nx, int
                       int nq, double2* P, hipStream_t s);
 // The same on a regular k mesh n[3] that pair_kfft_mesh takes: kpos[k] is the mesh
 // position of k (first axis fastest, relative to k = 0), qof[position] the q whose
-// k+q lie that far from k or -1 (q0 .. q0+nq-1 are wanted), sk0[k][3] the k points,
-// qvec[position][3] the q vector there.
+// k+q lie that far from k or -1 (q0 .. q0+nq-1 are wanted), phase and L from kfft_plan.
 bool pair_kfft_mesh(const int n[3], int ntk);
+// mk[k][3], mq[position][3]: k less k = 0 and the q at a position, each times n (whole
+// numbers; k + q less its umklapp vector is then k's position plus q's exactly).  False
+// if the phases' common denominator L does not fit.
+bool kfft_plan(const int n[3], int ntk, const int nw[3], const std::vector<int>& mk,
+               const std::vector<int>& mq, std::vector<double>& phase, double* L);
 void launch_pair_kfft(const float2* ur, int ntk, int nwf, bool full, int nx, int ny, int nz,
                       const int n[3], const int* kpos, const int* qof, int q0, int nq,
-                      const double* sk0, const double* qvec, const double2* wk, double2* P,
-                      hipStream_t s);
+                      const double* phase, double L, const double2* wk, double2* P, hipStream_t s);
 // k+q index (< 2^20) and umklapp vector (components -8..7) in one word, or
 // false when they do not fit
 inline bool pair_rsum_pack(int ikq, const int* d, unsigned* out) {

@@ -19,6 +19,8 @@
 // for the LDS (e.g. 24^3 = 13824 points) runs as three passes of line DFTs
 // over HBM (k_line_dft).
 #include <algorithm>
+#include <cmath>
+#include <numeric>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -939,36 +941,62 @@ void launch_pair_densities_pruned(const float2* ur, int ntk, const int* pocc, co
 //   P(q, r) = e^{i 2pi q.r/N} sum_k w_k conj(psi_iw,k+q) psi_jw,k
 //           = e^{i 2pi q.r/N} / NTK  sum_m conj(A_i(m)) C_j(m) e^{-i 2pi q.m/n},
 // A and C the forward transforms over the mesh of psi_iw and w psi_jw.  That is NTK
-// (n1 + n2 + n3) products per (pair, r) instead of NTK^2.  A workgroup takes tr
+// (n1 + n2 + n3) products per (pair, r) instead of NTK^2.  k and q enter as whole
+// numbers of mesh steps (k from the first k), which cancel to the umklapp phases of
+// the sums exactly; phases from the list's digits left Im func 5 times further off on
+// 27 k, and up to 6e-12 with lists of 13 digits.  A workgroup takes tr
 // grid points: A, C, the phases of q.r and pg pairs at a time in LDS, a thread one
 // line of up to eight mesh points in registers.  Bound by LDS (every axis reads and
 // writes each point once); rho with its transforms, 5 functions, k_pair_rsum_tile
-// before: 64 k, plane waves to 20 Ry in a 7 bohr cube, 70 -> 29 us (diagonal), 135 -> 60
-// (all pairs); 216 k, 30 Ry 851 -> 150 and 2140 -> 427; 8 k, 20 Ry 17 -> 16 and 24 -> 22.  More k do not fit with
-// every function's transforms; the line is drawn without regard to their number, so
-// that the same pairs among others come out the same.
+// before: 64 k, plane waves to 20 Ry in a 7 bohr cube, 69 -> 28 us (diagonal), 133 -> 59
+// (all pairs); 216 k, 30 Ry 857 -> 142 and 2148 -> 418; 8 k, 20 Ry 17 -> 16 and 24 -> 22.
+// More k do not fit with every function's transforms; the line is drawn without regard
+// to their number, so that the same pairs among others come out the same.
 constexpr int kKfftMax = 256, kKfftAxis = 8;
+constexpr int kKfftTw = 2 * (kKfftAxis / 2 + 1);  // factors of an axis: m = 0 .. 4, high and low
 
-// Forward transform of a line, tw[m] = e^{-i 2pi m/N}.
+// Forward transform of a line: with p_j = v_j + v_{N-j} and d_j = v_j - v_{N-j}, outputs
+// k and N - k are v_0 + sum_j cos(2pi jk/N) p_j -+ i sum_j sin(2pi jk/N) d_j (with
+// (-1)^k v_{N/2} if N is even).  tw[2 m] = (cos, sin)(2pi m/N), tw[2 m + 1] what their
+// rounding left: a rounded factor is the same for every value that goes through it, and
+// the eight passes of an axis would add its error up (three points: rho off by 4.5e-16
+// instead of 1.6e-16).
 template <int N>
 __device__ __forceinline__ void kfft_line(const double2 (&v)[N], double2 (&o)[N], const double2* tw) {
+  constexpr int H = (N - 1) / 2;
+  double2 p[H + 1], d[H + 1];
 #pragma unroll
-  for (int k = 0; k < N; ++k) {
-    double2 s = v[0];
+  for (int j = 1; j <= H; ++j) {
+    p[j] = make_double2(v[j].x + v[N - j].x, v[j].y + v[N - j].y);
+    d[j] = make_double2(v[j].x - v[N - j].x, v[j].y - v[N - j].y);
+  }
 #pragma unroll
-    for (int j = 1; j < N; ++j) {
-      const int m = j * k % N;
-      if (m == 0) s = make_double2(s.x + v[j].x, s.y + v[j].y);
-      else if (2 * m == N) s = make_double2(s.x - v[j].x, s.y - v[j].y);
-      else if (4 * m == N) s = make_double2(s.x + v[j].y, s.y - v[j].x);
-      else if (4 * m == 3 * N) s = make_double2(s.x - v[j].y, s.y + v[j].x);
-      else {
-        const double2 t = tw[m];
-        s.x += v[j].x * t.x - v[j].y * t.y;
-        s.y += v[j].x * t.y + v[j].y * t.x;
+  for (int k = 0; k <= N / 2; ++k) {
+    double2 a = v[0], b = make_double2(0.0, 0.0);
+    if (N % 2 == 0 && N > 1) {
+      const double2 u = v[N / 2];
+      a = k % 2 == 0 ? make_double2(a.x + u.x, a.y + u.y) : make_double2(a.x - u.x, a.y - u.y);
+    }
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      const int m = j * k % N, n = m < N - m ? m : N - m;  // cos(m) = cos(n), sin(m) = -+ sin(n)
+      const double sg = m == n ? 1.0 : -1.0;
+      if (n == 0) {
+        a = make_double2(a.x + p[j].x, a.y + p[j].y);
+      } else if (2 * n == N) {
+        a = make_double2(a.x - p[j].x, a.y - p[j].y);
+      } else if (4 * n == N) {
+        b = make_double2(fma(sg, d[j].x, b.x), fma(sg, d[j].y, b.y));
+      } else {
+        const double2 h = tw[2 * n], l = tw[2 * n + 1];
+        a.x = fma(h.x, p[j].x, fma(l.x, p[j].x, a.x));
+        a.y = fma(h.x, p[j].y, fma(l.x, p[j].y, a.y));
+        b.x = fma(sg * h.y, d[j].x, fma(sg * l.y, d[j].x, b.x));
+        b.y = fma(sg * h.y, d[j].y, fma(sg * l.y, d[j].y, b.y));
       }
     }
-    o[k] = s;
+    o[k] = make_double2(a.x + b.y, a.y - b.x);
+    if (k > 0 && 2 * k < N) o[N - k] = make_double2(a.x - b.y, a.y + b.x);
   }
 }
 
@@ -1006,36 +1034,40 @@ __device__ __forceinline__ void kfft_axis(int n, int count, int ntk, int tr, int
   }
 }
 
-// grid (ceil(nr / tr)), 256 threads.  mesh: kpos[k], then qof[position]: the q of this
-// launch there, or -1; vec: sk0 of every k, then the vector of every position.
+// e^{i 2pi (a . r) / L} for a whole-number vector a (below L) and a grid point r: the
+// product is exact, so the phase carries the roundings of one quotient and sincospi.
+__device__ __forceinline__ double2 kfft_phase(const double* a, int x, int y, int z, double L) {
+  const double s = fma(a[0], (double)x, fma(a[1], (double)y, a[2] * (double)z));
+  double sn, cs;
+  sincospi(2.0 * (fma(-rint(s / L), L, s) / L), &sn, &cs);
+  return make_double2(cs, sn);
+}
+
+// grid (ceil(nr / tr)), 256 threads.  kpos[k] and qof[position] (the q there, or -1) as
+// launch_pair_kfft takes them; phase: the vectors of every k, those of every position
+// (kfft_phase), then the axes' factors (kfft_line) and 1 / NTK with what its rounding left.
 __global__ void __launch_bounds__(256) k_pair_kfft(
     const float2* __restrict__ ur, int ntk, int nwf, int full, int nx, int ny, int nz, int n1, int n2,
     int n3, const int* __restrict__ kpos, const int* __restrict__ qof, int q0, int nq,
-    const double* __restrict__ sk0, const double* __restrict__ qvec, const double2* __restrict__ wk,
-    int tr, int pg, double2* __restrict__ P) {
+    const double* __restrict__ phase, double L, const double2* __restrict__ wk, int tr, int pg,
+    double2* __restrict__ P) {
   extern __shared__ double2 kf[];
   const int row = ntk * tr;
-  double2* tw = kf;                           // e^{-i 2pi m/n} per axis
-  double2* ph = tw + 3 * kKfftAxis;           // e^{i 2pi q.r/N} / NTK
+  double2* tw = kf;                           // the axes' factors
+  double2* ph = tw + 3 * kKfftTw;             // e^{i 2pi q.r/N}
   double2* buf = ph + row;                    // [pg][ntk][tr]
   double2* A = buf + (size_t)pg * row;        // [nwf][ntk][tr]
   double2* C = wk ? A + (size_t)nwf * row : A;
-  const double tpi = 2.0 * 3.141592653589793238462643383279502884;
   const int nr = nx * ny * nz, r0 = blockIdx.x * tr, t = threadIdx.x;
-  if (t < 3 * kKfftAxis) {
-    const int ax = t / kKfftAxis, m = t % kKfftAxis, n = ax == 0 ? n1 : (ax == 1 ? n2 : n3);
-    double sn, cs;
-    sincos(tpi * ((double)m / (double)n), &sn, &cs);
-    tw[t] = make_double2(cs, -sn);
-  }
+  const double* tail = phase + 6 * ntk;
+  if (t < 3 * kKfftTw) tw[t] = make_double2(tail[2 * t], tail[2 * t + 1]);
+  const double rh = tail[6 * kKfftTw], rl = tail[6 * kKfftTw + 1];
   for (int e = t; e < row; e += 256) {
     const int k = e / tr, r = min(r0 + e % tr, nr - 1);
-    const double x = (double)(r % nx) / nx, y = (double)(r / nx % ny) / ny,
-                 z = (double)(r / (nx * ny)) / nz;
-    double sn, cs;
-    sincos(tpi * (qvec[3 * k] * x + qvec[3 * k + 1] * y + qvec[3 * k + 2] * z), &sn, &cs);
-    ph[e] = make_double2(cs / ntk, sn / ntk);
-    sincos(tpi * (sk0[3 * k] * x + sk0[3 * k + 1] * y + sk0[3 * k + 2] * z), &sn, &cs);
+    const int x = r % nx, y = r / nx % ny, z = r / (nx * ny);
+    ph[e] = kfft_phase(phase + 3 * (ntk + k), x, y, z, L);
+    const double2 pk = kfft_phase(phase + 3 * k, x, y, z, L);
+    const double cs = pk.x, sn = pk.y;
     const double2 wv = wk ? wk[k] : make_double2(1.0, 0.0);
     const int o = kpos[k] * tr + e % tr;
     for (int w = 0; w < nwf; ++w) {
@@ -1052,8 +1084,8 @@ __global__ void __launch_bounds__(256) k_pair_kfft(
     auto put = [&](int a, int p, int r, double2 v) { A[a * row + p * tr + r] = v; };
     const int na = wk ? 2 * nwf : nwf;  // C follows A
     kfft_axis(n1, na, ntk, tr, 1, tw, at, put);
-    kfft_axis(n2, na, ntk, tr, n1, tw + kKfftAxis, at, put);
-    kfft_axis(n3, na, ntk, tr, n1 * n2, tw + 2 * kKfftAxis, at, put);
+    kfft_axis(n2, na, ntk, tr, n1, tw + kKfftTw, at, put);
+    kfft_axis(n3, na, ntk, tr, n1 * n2, tw + 2 * kKfftTw, at, put);
   }
   const int npair = full ? nwf * nwf : nwf;
   auto at = [&](int a, int p, int r) { return buf[a * row + p * tr + r]; };
@@ -1069,13 +1101,43 @@ __global__ void __launch_bounds__(256) k_pair_kfft(
       const int q = qof[p] - q0;
       if (q < 0 || q >= nq || r0 + r >= nr) return;
       const double2 f = ph[p * tr + r];
+      const double2 w = make_double2(v.x * f.x - v.y * f.y, v.x * f.y + v.y * f.x);
       P[((size_t)q * npair + pb + a) * nr + r0 + r] =
-          make_double2(v.x * f.x - v.y * f.y, v.x * f.y + v.y * f.x);
+          make_double2(fma(rh, w.x, rl * w.x), fma(rh, w.y, rl * w.y));
     };
     kfft_axis(n1, np, ntk, tr, 1, tw, product, put);
-    kfft_axis(n2, np, ntk, tr, n1, tw + kKfftAxis, at, put);
-    kfft_axis(n3, np, ntk, tr, n1 * n2, tw + 2 * kKfftAxis, at, out);
+    kfft_axis(n2, np, ntk, tr, n1, tw + kKfftTw, at, put);
+    kfft_axis(n3, np, ntk, tr, n1 * n2, tw + 2 * kKfftTw, at, out);
   }
+}
+
+bool kfft_plan(const int n[3], int ntk, const int nw[3], const std::vector<int>& mk,
+               const std::vector<int>& mq, std::vector<double>& phase, double* L) {
+  if (!pair_kfft_mesh(n, ntk)) return false;
+  long long l = 1;
+  for (int d = 0; d < 3; ++d) l = std::lcm(l, (long long)n[d] * nw[d]);
+  // a . r stays a whole number in FP64
+  if (l > (1LL << 50) / (3LL * std::max({nw[0], nw[1], nw[2]}))) return false;
+  phase.clear();
+  for (const auto* m : {&mk, &mq})
+    for (size_t i = 0; i < m->size(); ++i) {
+      const long long c = (*m)[i] * (l / ((long long)n[i % 3] * nw[i % 3])) % l;
+      phase.push_back((double)(c < 0 ? c + l : c));
+    }
+  auto split = [&](long double x) {
+    const double h = (double)x;
+    return std::pair<double, double>(h, (double)(x - h));
+  };
+  for (int d = 0; d < 3; ++d)
+    for (int m = 0; m <= kKfftAxis / 2; ++m) {
+      const long double a = 2.0L * std::acos(-1.0L) * (m % n[d]) / n[d];
+      const auto c = split(std::cos(a)), b = split(std::sin(a));
+      phase.insert(phase.end(), {c.first, b.first, c.second, b.second});
+    }
+  const auto r = split(1.0L / ntk);
+  phase.insert(phase.end(), {r.first, r.second});
+  *L = (double)l;
+  return true;
 }
 
 bool pair_kfft_mesh(const int n[3], int ntk) {
@@ -1084,15 +1146,14 @@ bool pair_kfft_mesh(const int n[3], int ntk) {
 
 void launch_pair_kfft(const float2* ur, int ntk, int nwf, bool full, int nx, int ny, int nz,
                       const int n[3], const int* kpos, const int* qof, int q0, int nq,
-                      const double* sk0, const double* qvec, const double2* wk, double2* P,
-                      hipStream_t s) {
+                      const double* phase, double L, const double2* wk, double2* P, hipStream_t s) {
   RP_CHECK(nwf >= 1 && nwf <= 16, "Wannier pair sums take at most 16 Wannier functions");
   RP_CHECK(pair_kfft_mesh(n, ntk), "k mesh too large for the correlation sums");
   if (nq <= 0) return;
   const int nr = nx * ny * nz;
   // As many grid points (up to 8) as leave two workgroups per CU, and as many pairs at
   // a time (up to 8) as have a line each for the threads.
-  const size_t unit = sizeof(double2) * (size_t)ntk, fixed = sizeof(double2) * 3 * kKfftAxis;
+  const size_t unit = sizeof(double2) * (size_t)ntk, fixed = sizeof(double2) * 3 * kKfftTw;
   const size_t arrays = 1 + (wk ? 2 : 1) * (size_t)nwf;
   int tr = 8;
   while (tr > 1 && fixed + unit * tr * (arrays + 4) > kLdsBytes / 2) tr /= 2;
@@ -1105,8 +1166,8 @@ void launch_pair_kfft(const float2* ur, int ntk, int nwf, bool full, int nx, int
     RP_HIP(hipFuncSetAttribute((const void*)k_pair_kfft, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds));
   hipLaunchKernelGGL(k_pair_kfft, dim3((nr + tr - 1) / tr), dim3(256), lds, s, ur, ntk, nwf,
-                     full ? 1 : 0, nx, ny, nz, n[0], n[1], n[2], kpos, qof, q0, nq, sk0, qvec, wk, tr,
-                     pg, P);
+                     full ? 1 : 0, nx, ny, nz, n[0], n[1], n[2], kpos, qof, q0, nq, phase, L, wk, tr, pg,
+                     P);
   RP_HIP(hipGetLastError());
 }
 

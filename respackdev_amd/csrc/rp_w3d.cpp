@@ -71,7 +71,8 @@ struct W3d {
   // the k mesh of launch_pair_kfft (geo_mesh[0] = 0: not one it takes)
   int geo_mesh[3] = {0, 0, 0};
   DevBuf<int> d_geo_kpos, d_geo_qof;
-  DevBuf<double> d_geo_sk0, d_geo_qvec;
+  DevBuf<double> d_geo_phase;
+  double geo_phase_den = 0;
   // summed pair-density grids P[q][p][r] of a chunk of q (launch_pair_rsum)
   DevBuf<double2> d_P;
   // exchange (rp_j3d_run): work buffers kept between calls, sized to a batch of R
@@ -221,49 +222,45 @@ QGeom q_geometry(const W3d& w, int iq) {
 }
 
 // The k points as a regular mesh, for the pair sums as correlations over it: true if
-// every k is at a mesh position of its own, k + q at that of k moved by the same
-// amount for every k, and k + q less its umklapp vector the same q.  kpos, qof and
-// qvec as launch_pair_kfft takes them.
+// every k is at a mesh position of its own and k + q less its umklapp vector at k's
+// position moved by the same whole numbers of mesh steps for every k.  The positions
+// are rounded from the list (within what search_kq takes for equal) and the phases
+// formed from them, so that the digits of the list do not matter, as they do not to
+// the sums over k.  kpos, qof, phase and den as launch_pair_kfft takes them.
 bool mesh_plan(const W3d& w, const std::vector<int>& ikq, const std::vector<int>& shift, int n[3],
-               std::vector<int>& kpos, std::vector<int>& qof, std::vector<double>& qvec) {
+               std::vector<int>& kpos, std::vector<int>& qof, std::vector<double>& phase, double* den) {
   for (int d = 0; d < 3; ++d) n[d] = w.nkb[d];
   if (n[0] < 1 || n[1] < 1 || n[2] < 1 || !pair_kfft_mesh(n, w.ntk)) return false;
+  auto wrap = [&](int x, int d) { return (x % n[d] + n[d]) % n[d]; };
   kpos.assign(w.ntk, 0);
   std::vector<char> seen(w.ntk, 0);
-  std::vector<int> m(3 * (size_t)w.ntk);
+  std::vector<int> mk(3 * (size_t)w.ntk), mq(3 * (size_t)w.ntk, 0);
   for (int k = 0; k < w.ntk; ++k) {
     for (int d = 0; d < 3; ++d) {
       const double x = (w.sk0[3 * k + d] - w.sk0[d]) * n[d], r = std::round(x);
-      if (!(std::fabs(x - r) < 1e-6 * n[d])) return false;
-      m[3 * k + d] = (((int)r) % n[d] + n[d]) % n[d];
+      if (!(std::fabs(x - r) < 1e-6 * n[d]) || std::fabs(r) > 1e6) return false;
+      mk[3 * k + d] = (int)r;
     }
-    kpos[k] = m[3 * k] + n[0] * (m[3 * k + 1] + n[1] * m[3 * k + 2]);
+    kpos[k] = wrap(mk[3 * k], 0) + n[0] * (wrap(mk[3 * k + 1], 1) + n[1] * wrap(mk[3 * k + 2], 2));
     if (seen[kpos[k]]++) return false;
   }
   qof.assign(w.ntk, -1);
-  qvec.assign(3 * (size_t)w.ntk, 0.0);
   for (int q = 0; q < w.ntq; ++q) {
-    int mq[3];
-    double v[3];
+    int m[3];
     for (int k = 0; k < w.ntk; ++k) {
       const size_t i = (size_t)q * w.ntk + k;
       for (int d = 0; d < 3; ++d) {
-        const int dm = (m[3 * ikq[i] + d] - m[3 * k + d] + n[d]) % n[d];
-        const double dv = w.sk0[3 * ikq[i] + d] + shift[3 * i + d] - w.sk0[3 * k + d];
-        if (k == 0) {
-          mq[d] = dm;
-          v[d] = dv;
-        } else if (dm != mq[d] || !(std::fabs(dv - v[d]) < 1e-12)) {
-          return false;
-        }
+        const int x = mk[3 * ikq[i] + d] + n[d] * shift[3 * i + d] - mk[3 * k + d];
+        if (k == 0) m[d] = x;
+        else if (x != m[d]) return false;
       }
     }
-    const int p = mq[0] + n[0] * (mq[1] + n[1] * mq[2]);
+    const int p = wrap(m[0], 0) + n[0] * (wrap(m[1], 1) + n[1] * wrap(m[2], 2));
     if (qof[p] >= 0) return false;
     qof[p] = q;
-    for (int d = 0; d < 3; ++d) qvec[3 * p + d] = v[d];
+    for (int d = 0; d < 3; ++d) mq[3 * p + d] = m[d];
   }
-  return true;
+  return kfft_plan(n, w.ntk, w.nw, mk, mq, phase, den);
 }
 
 // Every q's pair-density inputs in HBM, so that the loops over q only launch.
@@ -304,12 +301,11 @@ void ensure_geometry(W3d& w, hipStream_t s) {
   if (packed) w.d_geo_kqs.upload(kqs, s);
   else w.d_geo_kqs.release();
   std::vector<int> kpos, qof;
-  std::vector<double> qvec;
-  if (mesh_plan(w, ikq, shift, w.geo_mesh, kpos, qof, qvec)) {
+  std::vector<double> phase;
+  if (mesh_plan(w, ikq, shift, w.geo_mesh, kpos, qof, phase, &w.geo_phase_den)) {
     w.d_geo_kpos.upload(kpos, s);
     w.d_geo_qof.upload(qof, s);
-    w.d_geo_sk0.upload(w.sk0, s);
-    w.d_geo_qvec.upload(qvec, s);
+    w.d_geo_phase.upload(phase, s);
   } else {
     w.geo_mesh[0] = 0;
   }
@@ -341,7 +337,7 @@ void rho_all_q(W3d& w, bool full, const double2* wk, const long long* d_rho_off,
     const int nq = std::min(qchunk, w.ntq - q0);
     if (w.geo_mesh[0] > 0)  // faster at every size it takes
       launch_pair_kfft(w.d_ur.p, w.ntk, w.nwf, full, w.nw[0], w.nw[1], w.nw[2], w.geo_mesh,
-                       w.d_geo_kpos.p, w.d_geo_qof.p, q0, nq, w.d_geo_sk0.p, w.d_geo_qvec.p, wk,
+                       w.d_geo_kpos.p, w.d_geo_qof.p, q0, nq, w.d_geo_phase.p, w.geo_phase_den, wk,
                        w.d_P.p, s);
     else
       launch_pair_rsum(w.d_ur.p, w.ntk, w.nwf, full, w.nw[0], w.nw[1], w.nw[2],
