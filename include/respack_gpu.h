@@ -139,7 +139,8 @@ int rp_dyson_noalloc(rp_handle h, const double* chi_dev, double* epsinv_dev);
 /* All four stages for one q.  timings (optional, 8 doubles): seconds of pair
  * densities, weights, contraction, Dyson, total device time, host prepare,
  * the main contraction kernel alone (summed over its launches), and the
- * number of those launches (1, or 3 at q = 0). */
+ * number of those launches (1, or 3 at q = 0).  chi_out is filled also when the
+ * Dyson step fails. */
 int rp_chiqw_q(rp_handle h, const double* q, int32_t precision, double* epsinv_out,
                double* chi_out, double* timings);
 /* Device-resident number of pairs (after the Max_excitation_energy filter). */

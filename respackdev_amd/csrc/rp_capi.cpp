@@ -900,6 +900,13 @@ int rp_chiqw_q(rp_handle h, const double* q, int32_t precision, double* epsinv_o
   if (rp_chiqw_prepare_q(h, q, &ng, nullptr, 0)) return 1;
   return guarded([&] {
     hipStream_t s = h->stream;
+    // chi is delivered also when the Dyson step fails on it
+    auto dyson = [&] {
+      if (!rp_dyson(h, nullptr)) return;
+      const Error e(g_err);
+      if (chi_out) copy_to_host(h, chi_out, h->d_chi.p, chi_bytes(h));
+      throw e;
+    };
     RP_HIP(hipEventRecord(h->ev[0], s));
     if (rp_pairdens_batch(h, nullptr)) throw Error(g_err);
     RP_HIP(hipEventRecord(h->ev[1], s));
@@ -907,7 +914,7 @@ int rp_chiqw_q(rp_handle h, const double* q, int32_t precision, double* epsinv_o
     RP_HIP(hipEventRecord(h->ev[2], s));
     if (rp_chi_accumulate(h, precision, nullptr)) throw Error(g_err);
     RP_HIP(hipEventRecord(h->ev[3], s));
-    if (rp_dyson(h, nullptr)) throw Error(g_err);
+    dyson();
     RP_HIP(hipEventRecord(h->ev[4], s));
     // an ill-conditioned eps amplifies the FP32 accumulation error of the
     // split-BF16 contraction: run it again with the span its eps^-1 calls for
@@ -922,7 +929,7 @@ int rp_chiqw_q(rp_handle h, const double* q, int32_t precision, double* epsinv_o
       RP_HIP(hipEventRecord(h->ev[1], s));
       if (rp_chi_accumulate(h, precision, nullptr)) throw Error(g_err);
       RP_HIP(hipEventRecord(h->ev[2], s));
-      if (rp_dyson(h, nullptr)) throw Error(g_err);
+      dyson();
       RP_HIP(hipEventRecord(h->ev[3], s));
       RP_HIP(hipEventSynchronize(h->ev[3]));
       const double ta = event_seconds(h->ev[1], h->ev[2]), td = event_seconds(h->ev[2], h->ev[3]);

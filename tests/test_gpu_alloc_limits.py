@@ -1,0 +1,55 @@
+"""Calls that meet an allocation that fails: hipMalloc or hipHostMalloc refused from a
+size on by alloc_limits.c, in a process of its own (the refusal comes from the host;
+every kernel runs as usual).  What the caller asked for still arrives, or an error and
+what was computed before it."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes as C, sys
+sys.path.insert(0, sys.argv[2])
+lim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+lim.alloc_limits.argtypes = [C.c_size_t, C.c_size_t]
+ALL = 2 ** 64 - 1
+import numpy as np
+from respackdev_amd import _lib, gen
+from respackdev_amd.chiqw import Chiqw, from_system
+def opened(ecut, nen=14, **kw):
+    c = Chiqw(0)
+    c.open(from_system(gen.make_system(a=7.0, seed=47, **kw)), ecut_for_eps=ecut, num_freq_grid=nen)
+    return c
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+"""
+
+
+def run(tmp_path, body):
+    so = str(tmp_path / "alloc_limits.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", os.path.join(HERE, "alloc_limits.c"), "-o", so, "-ldl"],
+                   check=True)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body, so, os.path.dirname(HERE)],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.split()[-1:] == ["done"], r.stdout + r.stderr
+
+
+def test_chi_arrives_when_the_dyson_step_fails(tmp_path):
+    run(tmp_path, """
+c = opened(4.0, nk=2, nocc=2, nvir=3, ecut_psi=9.0)
+q = (0.0, 0.0, 0.5)
+lg = c.prepare_q(q); c.pair_densities(False); c.weights(False)
+ref = c.accumulate("fp64")
+lim.alloc_limits(0, ALL)  # eps^-1 has no buffer yet
+chi = np.zeros_like(ref); eps = np.zeros_like(ref); qq = np.array(q)
+rc = _lib.lib().rp_chiqw_q(c._h, _lib.ptr(qq), 0, _lib.ptr(eps), _lib.ptr(chi), None)
+assert rc != 0 and lim.alloc_refused() > 0, (rc, lim.alloc_refused())
+assert rel(chi, ref) <= 1e-13, rel(chi, ref)  # the weights' sums meet in any order
+lim.alloc_limits(ALL, ALL)
+assert rel(c.run_q(q, "fp64", want_chi=True)["chi"], ref) <= 1e-13
+c.close(); print("done")
+""")
