@@ -619,13 +619,18 @@ void issue_operands(rp_ctx* h, int prec) {
   if (h->q0) launch_presplit_column(h->d_heads.p, h->lda, h->kpad, h->g0, h->d_Ao.p, s);
 }
 
+// Elements of the partial-sum buffer of a launch (the head of a further direction at
+// q = 0 needs at least 2 nen ng of it).
+static size_t partial_room(const rp_ctx* h, const ChiLaunch& c) {
+  return std::max((size_t)c.nsplit * h->ng * h->ng * h->nen, 2 * (size_t)h->nen * h->ng);
+}
+
 void issue_accumulate(rp_ctx* h, int prec, const ChiLaunch& c, bool events, bool operands_ready) {
   hipStream_t s = h->stream;
   const int ng = h->ng, nen = h->nen, nc = h->q0 ? 3 : 1;
   const size_t per = (size_t)ng * ng * nen;
   grow(h, h->d_chi, (size_t)nc * per, "chi buffer");
-  // (the head of a further direction at q = 0 needs at least 2 nen ng of it)
-  const size_t room = std::max((size_t)c.nsplit * per, 2 * (size_t)nen * ng);
+  const size_t room = partial_room(h, c);
   grow(h, h->d_part, room, "partial-sum buffer");
   if (prec == RP_PREC_BF16X3) {
     grow(h, h->d_sync, bf16x3_sync_words(), "rendezvous counters");
@@ -696,9 +701,11 @@ void issue_dyson(rp_ctx* h) {
 // Candidates around the heuristic: for the split-BF16 kernel the K splits
 // whose work rounds per XCD slot (the heuristic's model) are within 15% of the
 // best, plus half and double the heuristic's; for the FP64/FP32 kernels half
-// and double the heuristic's split.  Each is timed on the
+// and double the heuristic's split, within its bounds.  Each is timed on the
 // current q's data (one warm-up, then the best of two), and the fastest is
-// kept for every later q of the same shape.
+// kept for every later q of the same shape; one whose partial sums do not fit is
+// passed over, and the partials' buffer goes back to what was there before or
+// the winner needs.
 static std::vector<ChiLaunch> chi_candidates(const rp_ctx* h, int prec) {
   std::vector<ChiLaunch> out;
   const ChiLaunch base = chi_launch_heuristic(h, prec);
@@ -722,8 +729,8 @@ static std::vector<ChiLaunch> chi_candidates(const rp_ctx* h, int prec) {
     if (base.nsplit > 1) add({base.nsplit / 2, base.nwg});
     if ((size_t)base.nsplit * 2 <= nchunks && base.nsplit * 2 <= 64) add({base.nsplit * 2, base.nwg});
   } else {
-    const int kchunks = (int)(h->kpad / chi_kchunk());
-    for (int sp : {base.nsplit / 2, base.nsplit * 2}) add({std::min(kchunks, std::max(1, sp)), 0});
+    const int most = chi_gemm_max_nsplit(h->ng, h->nen, h->kpad);
+    for (int sp : {base.nsplit / 2, base.nsplit * 2}) add({std::min(most, std::max(1, sp)), 0});
   }
   return out;
 }
@@ -755,8 +762,24 @@ static double time_launch(rp_ctx* h, int prec, const ChiLaunch& c) {
   return best;
 }
 
+// The partial-sum buffer of a launch, or false if the memory is not to be had.
+static bool reserve_partials(rp_ctx* h, const ChiLaunch& c) {
+  try {
+    h->d_part.reserve(partial_room(h, c));
+    return true;
+  } catch (const Error&) {
+    (void)hipGetLastError();
+    return false;
+  }
+}
+
 ChiLaunch chi_launch(rp_ctx* h, int prec) {
   ChiLaunch c = chi_launch_tuned(h, prec);
+  // FP64 splits K further than it must where that is faster: less so when memory is short
+  if (prec == RP_PREC_FP64 && !h->capturing)
+    for (const int fewest = chi_gemm_min_nsplit(h->ng, h->nen, h->kpad);
+         c.nsplit > fewest && !reserve_partials(h, c);)
+      c.nsplit = std::max(fewest, c.nsplit / 2);
   if (prec == RP_PREC_BF16X3) c.span = h->span > 0 ? h->span : h->q_span;
   return c;
 }
@@ -796,13 +819,22 @@ ChiLaunch chi_launch_tuned(rp_ctx* h, int prec) {
   const auto cand = chi_candidates(h, prec);
   t.ncand = (int)cand.size();
   t.best_ms = 1e300;
+  t.best = base;
+  const size_t part = h->d_part.n;
   for (const auto& c : cand) {
+    if (!reserve_partials(h, c)) continue;
     const double ms = time_launch(h, prec, c);
     if (c.nsplit == base.nsplit && c.nwg == base.nwg) t.heuristic_ms = ms;
     if (ms < t.best_ms) {
       t.best_ms = ms;
       t.best = c;
     }
+  }
+  if (t.best_ms == 1e300) return base;  // none fits
+  const size_t need = std::max(part, partial_room(h, t.best));
+  if (h->d_part.n > need) {
+    h->d_part.release();
+    h->d_part.reserve(need);
   }
   h->tune.push_back(t);
   return t.best;

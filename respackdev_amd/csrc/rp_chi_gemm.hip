@@ -366,24 +366,38 @@ __global__ void k_chi_reduce_cross(const double2* __restrict__ part, int ng, int
 int chi_tile() { return kTile; }
 int chi_kchunk() { return kKC; }
 
-// K splits.  FP32: enough for 2048 workgroups.  FP64: at least as many, for the
+// K splits for 2048 workgroups: the fewest of either precision.
+int chi_gemm_min_nsplit(int ng, int nen, size_t kpad) {
+  const int ntile = (ng + kTile - 1) / kTile;
+  const long wgs = (long)ntile * ntile * nen;
+  return (int)std::min<long>((long)(kpad / kKC), (2048 + wgs - 1) / wgs);
+}
+
+// The most: 64, or twice the fewest where that is more, with partials of at most
+// 2 GiB (one split whatever its size).
+int chi_gemm_max_nsplit(int ng, int nen, size_t kpad) {
+  const long room = (long)(2147483648.0 / (16.0 * ng * ng * nen));
+  const long most = std::min(room, std::max(64L, 2L * chi_gemm_min_nsplit(ng, nen, kpad)));
+  return (int)std::max(1L, std::min((long)(kpad / kKC), most));
+}
+
+// K splits.  FP32: the fewest.  FP64: at least as many, for the
 // rounding of a sum falls with its splits (K 1296, NG 81: 9 splits left the real
 // part off by 2.6e-16, 37 by 1.9e-16), and more where they are faster: with W workgroups per
 // split, S = 4 resident per CU and C chunks of 32 K, a launch takes about
 //   (W sp / S + 1/2 round of tail) (C / sp + 2 chunks of start and end)
 // chunk times of a full CU (5.2 us: four workgroups' MFMAs), plus the traffic
 // of the partial tiles, written and read once per split (32 bytes per element
-// at about 4.5 TB/s); sp is where that is least, with at most 2 GiB of partials.
+// at about 4.5 TB/s); sp is where that is least.
 int chi_gemm_nsplit(int prec, int ng, int nen, size_t kpad, int ncu) {
+  const int fewest = chi_gemm_min_nsplit(ng, nen, kpad);
+  if (prec != RP_PREC_FP64) return fewest;
   const int ntile = (ng + kTile - 1) / kTile;
-  const long kchunks = (long)(kpad / kKC), wgs = (long)ntile * ntile * nen;
-  if (prec != RP_PREC_FP64)
-    return (int)std::min<long>(kchunks, std::max<long>(1, (2048 + wgs - 1) / wgs));
+  const double wgs = (double)ntile * ntile * nen;
   const double per = 16.0 * ng * ng * nen;  // bytes of one partial set
-  const double cost = 2.0 * (double)wgs / (4.0 * ncu) + 2.0 * per / 4.5e6 / 5.2;
-  const double sp = std::min(std::sqrt(0.5 * (double)kchunks / cost), 2147483648.0 / per);
-  const long fast = (long)std::max(1.0, std::min(64.0, std::round(sp)));
-  return (int)std::min(kchunks, std::max(fast, (2048 + wgs - 1) / wgs));
+  const double cost = 2.0 * wgs / (4.0 * ncu) + 2.0 * per / 4.5e6 / 5.2;
+  const double sp = std::min(64.0, std::round(std::sqrt(0.5 * (double)(kpad / kKC) / cost)));
+  return std::min(std::max((int)sp, fewest), chi_gemm_max_nsplit(ng, nen, kpad));
 }
 
 void launch_chi_gemm(int prec, const float2* A, size_t lda, const double2* dw, size_t ldd,

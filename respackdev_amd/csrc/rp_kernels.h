@@ -105,6 +105,8 @@ void launch_drude(const double2* coef, const int* kg, const int* ng0, int ntk, i
 // rp_chi_gemm.hip
 int chi_tile();
 int chi_kchunk();
+int chi_gemm_min_nsplit(int ng, int nen, size_t kpad);
+int chi_gemm_max_nsplit(int ng, int nen, size_t kpad);
 int chi_gemm_nsplit(int prec, int ng, int nen, size_t kpad, int ncu);
 void launch_chi_gemm(int prec, const float2* A, size_t lda, const double2* dw, size_t ldd,
                      size_t kpad, int ng, int nen, int nsplit, int cross, double2* partial,

@@ -53,3 +53,52 @@ lim.alloc_limits(ALL, ALL)
 assert rel(c.run_q(q, "fp64", want_chi=True)["chi"], ref) <= 1e-13
 c.close(); print("done")
 """)
+
+
+# NG ~ 300, 200 frequencies, K 38400: partial sums of 0.3 GB per split of K, four splits
+# (twice that is above the 2 GiB bound), one where it must be
+LARGE = """
+c = opened(14.0, nen=200, nk=4, nocc=10, nvir=60, ecut_psi=14.5)
+ng = len(c.prepare_q((0.0, 0.0, 0.25))); c.pair_densities(False); c.weights(False)
+per = 16 * ng * ng * 200
+"""
+
+
+def test_tuner_stays_within_the_bound_of_the_partial_sums(tmp_path):
+    run(tmp_path, LARGE + """
+lim.alloc_limits(2 ** 31, ALL)
+c.autotune(True); c.accumulate("fp64", copy=False)
+t = c.tune_table()[0]
+assert t["heuristic_nsplit"] == 4 and 8 * per > 2 ** 31 and lim.alloc_refused() == 0, t
+c.close(); print("done")
+""")
+
+
+def test_tuner_passes_over_what_does_not_fit(tmp_path):
+    run(tmp_path, """
+c = opened(6.9, nk=4, nocc=4, nvir=8, ecut_psi=9.0)
+ng = len(c.prepare_q((0.0, 0.0, 0.25))); c.pair_densities(False); c.weights(False)
+ref = c.accumulate("fp64"); c.close()
+c = opened(6.9, nk=4, nocc=4, nvir=8, ecut_psi=9.0)
+c.autotune(True)
+c.prepare_q((0.0, 0.0, 0.25)); c.pair_densities(False); c.weights(False)
+sp = min(4 * 8 * 64 // 32, -(-2048 // ((-(-ng // 64)) ** 2 * 14)))
+lim.alloc_limits(sp * 16 * ng * ng * 14, ALL)  # the heuristic's partials, not twice them
+chi = c.accumulate("fp64")
+t = c.tune_table()[0]
+assert t["heuristic_nsplit"] == sp and t["nsplit"] <= sp and lim.alloc_refused() > 0, t
+assert rel(chi, ref) <= 1e-13
+c.close(); print("done")
+""")
+
+
+def test_fewer_splits_when_memory_is_short(tmp_path):
+    run(tmp_path, LARGE + """
+ref = c.accumulate("fp64"); c.close()
+c = opened(14.0, nen=200, nk=4, nocc=10, nvir=60, ecut_psi=14.5)
+c.prepare_q((0.0, 0.0, 0.25)); c.pair_densities(False); c.weights(False)
+lim.alloc_limits(3 * per, ALL)
+chi = c.accumulate("fp64")
+assert lim.alloc_refused() > 0 and rel(chi, ref) <= 1e-13, rel(chi, ref)
+c.close(); print("done")
+""")
