@@ -21,6 +21,11 @@
 
 namespace rp {
 
+// Work buffers of the exchange that stay with the handle (seven R of 25 pairs on 64 k
+// take 0.25 GB and 2.7 ms); larger ones go back at the end of the call, which is then long
+// beside their allocation.
+constexpr size_t kJKeepBytes = size_t(512) << 20;
+
 struct W3d {
   bool open = false, have_wan = false, have_q = false, have_funcs = false;
   double a[3][3], b[3][3], volume = 0, ecut_psi = 0, ecut_eps = 0;
@@ -75,8 +80,15 @@ struct W3d {
   double geo_phase_den = 0;
   // summed pair-density grids P[q][p][r] of a chunk of q (launch_pair_rsum)
   DevBuf<double2> d_P;
-  // exchange (rp_j3d_run): work buffers kept between calls, sized to a batch of R
+  // exchange (rp_j3d_run): work buffers sized to a batch of R, kept between calls up to
+  // kJKeepBytes in all
   DevBuf<double2> d_pfk, d_jrho, d_jfunc, d_jfuncw, d_jx, d_jj, d_jz, d_jxs;
+  void trim_exchange() {
+    size_t n = 0;
+    for (auto* b : {&d_jrho, &d_jfunc, &d_jfuncw, &d_jx, &d_jj, &d_jz, &d_jxs}) n += b->n;
+    if (n * sizeof(double2) > kJKeepBytes)
+      for (auto* b : {&d_jrho, &d_jfunc, &d_jfuncw, &d_jx, &d_jj, &d_jz, &d_jxs}) b->release();
+  }
   DevBuf<long long> d_joff;
   DevBuf<char> d_jgrp;
   DevBuf<int> d_jmem, d_jr0;
@@ -875,6 +887,7 @@ int rp_j3d_run(rp_handle h, int32_t nr, const int32_t* rvec, double* xmat, doubl
     w.stage_s[6] = tj;
     w.stage_s[7] = event_s(w.ev[2], w.ev[1]);
     w.stage_s[5] = w.stage_s[7] - tr - tj;
+    w.trim_exchange();
     if (heads) {
       heads[0] = w.chead;
       heads[1] = 0.0;

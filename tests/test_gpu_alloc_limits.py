@@ -1,7 +1,7 @@
 """Calls that meet an allocation that fails: hipMalloc or hipHostMalloc refused from a
 size on by alloc_limits.c, in a process of its own (the refusal comes from the host;
 every kernel runs as usual).  What the caller asked for still arrives, or an error and
-what was computed before it."""
+what was computed before it.  And what a call leaves allocated."""
 import os
 import subprocess
 import sys
@@ -16,6 +16,7 @@ import ctypes as C, sys
 sys.path.insert(0, sys.argv[2])
 lim = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
 lim.alloc_limits.argtypes = [C.c_size_t, C.c_size_t]
+lim.alloc_live.restype = C.c_size_t
 ALL = 2 ** 64 - 1
 import numpy as np
 from respackdev_amd import _lib, gen
@@ -101,4 +102,32 @@ lim.alloc_limits(3 * per, ALL)
 chi = c.accumulate("fp64")
 assert lim.alloc_refused() > 0 and rel(chi, ref) <= 1e-13, rel(chi, ref)
 c.close(); print("done")
+""")
+
+
+def test_exchange_gives_large_buffers_back(tmp_path):
+    """Nine functions on 6^3 k, four R: 1.1 GB of vectors at a time."""
+    run(tmp_path, """
+from respackdev_amd.w3d import W3d
+s = gen.make_system(a=7.0, nk=6, nocc=1, nvir=1, ecut_psi=30.0, seed=64)
+wan, _ = gen.make_wannier(s, 9, 65)
+w = from_system(s)
+W = np.zeros((len(wan), 9, max(c.shape[1] for c in wan)), np.complex128)
+for k, c in enumerate(wan):
+    W[k, :, :c.shape[1]] = c
+rs = [(0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1)]
+g = W3d(0)
+g.open(w, 1.5, np.zeros(1, np.complex128))
+g.set_wannier(W)
+for iq, n in enumerate(g.set_q(w.ski)):
+    g.set_epsinv(iq, 0.7 * np.eye(n, dtype=np.complex128)[None])
+x1 = g.j3d(rs[:1])[0]
+one = lim.alloc_live()
+x4 = g.j3d(rs)[0]
+assert one > 2 ** 20 and lim.alloc_live() <= one, (one, lim.alloc_live())
+assert np.array_equal(x4, g.j3d(rs)[0])
+assert np.abs(x4[0] - x1[0]).max() <= 5e-14 * np.abs(x1).max()
+g.close()
+assert lim.alloc_live() == 0, lim.alloc_live()
+print("done")
 """)
