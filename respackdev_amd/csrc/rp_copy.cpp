@@ -72,16 +72,39 @@ void copy_chunks(rp_ctx* h, char* host, char* dev, size_t bytes, bool to_host, i
   }
 }
 
+// Whether the runtime knows the caller's memory (pinned, managed): it then copies
+// straight to or from it, at the rate of the link.
+bool known_memory(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
+// Threads for a copy, with the handle's pinned chunks for them; 0: none of this, the
+// copy is left to the runtime.
+int copy_threads(rp_ctx* h, const void* host, size_t bytes) {
+  if (bytes < kPlainBytes || known_memory(host)) return 0;
+  const int nt = std::min(kMaxThreads, std::max(1, (int)std::thread::hardware_concurrency() / 2));
+  try {
+    h->h_copy.reserve(2 * (size_t)nt * kChunkBytes);
+  } catch (const Error&) {  // no pinned memory to be had
+    (void)hipGetLastError();
+    return 0;
+  }
+  return nt;
+}
+
 void copy(rp_ctx* h, void* host, void* dev, size_t bytes, bool to_host) {
-  if (bytes < kPlainBytes) {
+  const int nt = copy_threads(h, host, bytes);
+  if (nt == 0) {
     if (to_host) RP_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, h->stream));
     else RP_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, h->stream));
     RP_HIP(hipStreamSynchronize(h->stream));
     return;
   }
-  const int cores = std::max(1, (int)std::thread::hardware_concurrency() / 2);
-  const int nt = std::min(kMaxThreads, cores);
-  h->h_copy.reserve(2 * (size_t)nt * kChunkBytes);
   std::vector<std::exception_ptr> err(nt);
   auto work = [&](int t) {
     try {

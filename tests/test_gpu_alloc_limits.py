@@ -131,3 +131,47 @@ g.close()
 assert lim.alloc_live() == 0, lim.alloc_live()
 print("done")
 """)
+
+
+# chi in and eps^-1 out are 4.8 MiB each: by chunks over several threads
+COPIES = """
+c = opened(8.3, nk=2, nocc=2, nvir=3, ecut_psi=16.0)
+n = len(c.prepare_q((0.0, 0.0, 0.5)))
+rng = np.random.default_rng(48)
+chi = 1e-3 * (rng.standard_normal((1, 14, n, n)) + 1j * rng.standard_normal((1, 14, n, n)))
+assert chi.nbytes > 4 << 20
+"""
+
+
+def test_large_copies_without_pinned_memory(tmp_path):
+    run(tmp_path, COPIES + """
+lim.alloc_limits(ALL, 0)
+plain = c.dyson_from(chi)
+assert lim.alloc_refused() > 0
+lim.alloc_limits(ALL, ALL)
+assert np.array_equal(c.dyson_from(chi), plain)
+c.close(); print("done")
+""")
+
+
+def test_pinned_arrays_take_no_chunks(tmp_path):
+    run(tmp_path, COPIES + """
+hip = C.CDLL("libamdhip64.so.7")
+hip.hipHostMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_uint]
+hip.hipHostFree.argtypes = [C.c_void_p]
+ps = [C.c_void_p(), C.c_void_p()]
+for p in ps:
+    assert hip.hipHostMalloc(C.byref(p), chi.nbytes, 0) == 0
+a, b = [np.frombuffer((C.c_char * chi.nbytes).from_address(p.value), np.complex128).reshape(chi.shape)
+        for p in ps]
+a[:] = chi
+lim.alloc_limits(ALL, 0)  # the handle has no chunks yet
+_lib.check(_lib.lib().rp_chi_set(c._h, ps[0])); _lib.check(_lib.lib().rp_dyson(c._h, ps[1]))
+assert lim.alloc_refused() == 0
+lim.alloc_limits(ALL, ALL)
+assert np.array_equal(c.dyson_from(chi), b)
+c.close()
+for p in ps:
+    hip.hipHostFree(p)
+print("done")
+""")
