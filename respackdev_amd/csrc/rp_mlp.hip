@@ -565,6 +565,9 @@ void launch_bwd_layer(const float* dZ, const float* A, int n, int nin, int nout,
                                (int)kBwdWLds));
     hipLaunchKernelGGL(kernel, dim3(nd + nw), dim3(256), kBwdWLds, s, dZ, A, W, Zprev, n, nin, nw, dA, part);
   };
+  // a kernel of its own for the widths of hidden layers and the closure's two outputs;
+  // any other width (an output layer of a network that is not the closure's) runs the
+  // two general kernels
 #define RP_BWD(KK) \
   case KK: both(big ? k_bwd<KK, kRowsS> : k_bwd<KK, kRowsS / 2>); break;
   if (!dA) {
