@@ -149,3 +149,28 @@ def test_q_in_two_passes():
     (x9, j9), (x3, j3) = out
     assert np.abs(x9[:, :3, :3] - x3).max() <= 5e-14 * np.abs(x3).max()
     assert np.abs(j9[:, :, :3, :3] - j3).max() <= 5e-14 * np.abs(j3).max()
+
+
+def test_most_k_and_most_functions():
+    """256 k (8 x 8 x 4) and sixteen functions, the largest that the LDS of the mesh
+    transforms holds, against the first two functions alone (eight grid points at a time
+    instead of one): rho of a pair takes the same operations whatever its company, the
+    sums over G and the contraction at most a few hundred 2^-53 of the largest element."""
+    n, out = (8, 8, 4), []
+    w, _, _, _, W1 = system(n, 1, 4.0)
+    rng = np.random.default_rng(82)
+    W = (rng.standard_normal((W1.shape[0], 16, W1.shape[2])) +
+         1j * rng.standard_normal((W1.shape[0], 16, W1.shape[2])))
+    W *= (np.abs(W1) > 0)  # the plane waves of each k
+    for nwf in (16, 2):
+        g = W3d(0)
+        try:
+            g.open(w, 2.0, np.zeros(1, np.complex128))
+            g.set_wannier(W[:, :nwf])
+            for iq, m in enumerate(g.set_q(w.ski)):
+                g.set_epsinv(iq, 0.7 * np.eye(m, dtype=np.complex128)[None])
+            out.append(g.funcs() + g.j3d([(1, 0, -1)])[:2])
+        finally:
+            g.close()
+    for a, b in zip(*out):
+        assert np.abs(a[..., :2, :2] - b).max() <= 5e-14 * np.abs(b).max()
