@@ -959,8 +959,8 @@ constexpr int kKfftTw = 2 * (kKfftAxis / 2 + 1);  // factors of an axis: m = 0 .
 // k and N - k are v_0 + sum_j cos(2pi jk/N) p_j -+ i sum_j sin(2pi jk/N) d_j (with
 // (-1)^k v_{N/2} if N is even).  tw[2 m] = (cos, sin)(2pi m/N), tw[2 m + 1] what their
 // rounding left: a rounded factor is the same for every value that goes through it, and
-// the eight passes of an axis would add its error up (three points: rho off by 4.5e-16
-// instead of 1.6e-16).
+// the passes along the axes, there and back, would add its error up (three points: func off
+// by 4.5e-16 instead of 2.0e-16).
 template <int N>
 __device__ __forceinline__ void kfft_line(const double2 (&v)[N], double2 (&o)[N], const double2* tw) {
   constexpr int H = (N - 1) / 2;

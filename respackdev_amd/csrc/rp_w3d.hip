@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(512) k_w_contract(
 // Z_c(a) Y(a, c).  A wave takes one column block of 16 and every row block of the
 // tile (with fewer column blocks the rows are dealt out).  Bound by the FP64 MFMAs
 // (shared with the FP64 vector unit, hence E and X widened once per workgroup): 64 q,
-// 16 frequencies, 25 pairs, NG_eps ~310, seven R: 2.28 ms (60 TFLOP/s; 4.16 ms with
+// 16 frequencies, 25 pairs, NG_eps ~310, seven R: 2.30 ms (59 TFLOP/s; 4.16 ms with
 // every (q, R) on its own).  Four workgroups per CU; three take 2.41 ms; 12 columns of E
 // at a time 2.55.  Three real products per complex one take 1.98 ms, but leave Im J
 // further off (as Im W of k_w_contract).
@@ -341,11 +341,12 @@ __global__ void __launch_bounds__(256) k_j_vecs(const double2* __restrict__ rho,
   }
 }
 
-// NR row blocks from block rb on by the column block cb of a staged chunk.
+// NR row blocks from block rb on by the column block cb of a staged chunk.  (Unrolled, the
+// loop's operands do not fit beside the sums in the 128 registers of four workgroups.)
 template <int NR>
 __device__ __forceinline__ void j_chunk(const double* pe, const double* px, int rb, int cb, int li,
                                         int lk, jd4 (&re)[NR], jd4 (&im)[NR]) {
-#pragma unroll
+#pragma unroll 1
   for (int k0 = 0; k0 < kJKC; k0 += 4) {
     const int o = (k0 + lk) * kJRow + li;
     const double xr = px[o + 16 * cb], xi = px[kJPlane + o + 16 * cb], nxi = -xi;
@@ -378,6 +379,8 @@ __global__ void __launch_bounds__(256, 4) k_j_contract(
     double2* __restrict__ out) {
   __shared__ double se[2 * kJPlane], sx[2 * kJPlane];
   __shared__ double2 red[4][16];
+  __shared__ double2 sum[256];  // each thread's rows of its column so far (not in registers
+                                // through the loops over b)
   const int w = blockIdx.x, rs = (int)blockIdx.z % nrs, tc = (int)blockIdx.z / nrs;
   const JGroup g = grp[blockIdx.y];
   const int ncb = (g.ncol + 15) / 16, nct = (ncb + 3) / 4, cpad = 16 * ncb;
@@ -407,7 +410,7 @@ __global__ void __launch_bounds__(256, 4) k_j_contract(
       xv[e] = (X + (size_t)b * cpad)[xc];
     }
   };
-  double sre = 0.0, sim = 0.0;  // this lane's rows of column 16 (hb + cb) + li
+  sum[threadIdx.x] = make_double2(0.0, 0.0);
   if (rs < nat) load(16 * (rs * nab / nat), 0);
   // one row tile for a wave with NR of its row blocks, from rb on (0: it only
   // stages); next: first row of the workgroup's next tile, < 0 for none
@@ -431,12 +434,17 @@ __global__ void __launch_bounds__(256, 4) k_j_contract(
       if constexpr (NR > 0) j_chunk<NR>(se, sx, rb, cb, li, lk, re, im);
       __syncthreads();
     }
-    const int c = 16 * (hb + cb) + li;
+    // (the compiler would form every row's and the column's index before the loop over
+    // b and keep them in registers through it)
+    int row = lk, col = li;
+    asm volatile("" : "+v"(row), "+v"(col));
+    const int c = 16 * (hb + cb) + col;
+    double sre = sum[threadIdx.x].x, sim = sum[threadIdx.x].y;
 #pragma unroll
     for (int a = 0; a < NR; ++a) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const int ar = 16 * (ab + rb + a) + lk + 4 * v;
+        const int ar = 16 * (ab + rb + a) + row + 4 * v;
         if (ar >= g.nge) continue;
         const double yr = re[a][v], yi = im[a][v];
         const double2 z = Z[(size_t)ar * cpad + c];
@@ -445,6 +453,7 @@ __global__ void __launch_bounds__(256, 4) k_j_contract(
         if (v & 1) __builtin_amdgcn_sched_barrier(0);  // few Z in registers at a time: no spills
       }
     }
+    sum[threadIdx.x] = make_double2(sre, sim);
   };
   using std::integral_constant;
   for (int t = rs; t < nat; t += nrs) {
@@ -457,6 +466,7 @@ __global__ void __launch_bounds__(256, 4) k_j_contract(
     else if (nrb == 1) tile(integral_constant<int, 1>{}, ab, rb, next);
     else tile(integral_constant<int, 0>{}, ab, rb, next);
   }
+  double sre = sum[threadIdx.x].x, sim = sum[threadIdx.x].y;
   for (int off = 16; off < 64; off <<= 1) {
     sre += __shfl_xor(sre, off);
     sim += __shfl_xor(sim, off);
